@@ -1291,9 +1291,14 @@ __device__ __forceinline__ void makeF32(const Params& P, const PairView& v, Pair
   f.m[3] = float(c0.y); f.m[4] = float(c1.y); f.m[5] = float(c2.y);
   f.m[6] = float(c0.z); f.m[7] = float(c1.z); f.m[8] = float(c2.z);
   f.t[0] = float(t.x); f.t[1] = float(t.y); f.t[2] = float(t.z);
-  // |g| of any node that can pass is below reach; FP32 error of g is ~1e-7 reach
+  // Every term of g = M n + t lies below reach: |M n| <= rA / spacing for a node (and sqrt(3) times
+  // that for a cluster's box centre).  The FP32 rounding of M, n, t, the products and the sums is below
+  // 12 x 2^-24 reach = 7e-7 reach, so the margins below are 14 times what they have to cover.  (A bound
+  // of 8 scale / spacing in rA's place is right for shapes of unit size only: shapes given in metres at
+  // scale 1 had margins of 0.16 grid cells, and 4.06M candidate nodes for 0.21M contacts in an ordered
+  // bed of 27,000 of them; with rA 0.21M, and its candidate kernel takes 184 us instead of 497.)
   const double cg = len(v.goB) * is;
-  const double reach = len(t) + 8.0 * v.sA * is + cg + double(SB.nx + SB.ny + SB.nz);
+  const double reach = len(t) + v.rA * is + cg + double(SB.nx + SB.ny + SB.nz);
   const double abs = 1e-5 * reach + 1e-6;
   f.c[0] = float(-v.goB.x * is); f.c[1] = float(-v.goB.y * is); f.c[2] = float(-v.goB.z * is);
   if (v.type == PT_PP) {

@@ -27,9 +27,9 @@ __global__ void k_broad_phase(Params P);
 __global__ void k_bucket_count(const int* bucket, int n, int* count, int* rank, const int* gate);
 __global__ void k_bucket_scatter(const int* bucket, int n, const int* start, const int* rank, int* out,
                                  int* bigCount, const int* gate);
-__global__ void k_bucket_sort(const int* start, int nb, const int* tmp, int* items, int* bigList, int* bigCount,
-                              const int* gate, int nItems);
-__global__ void k_bucket_sort_big(const int* start, int nb, const int* tmp, int* items, const int* bigList,
+__global__ void k_bucket_sort(const int* start, int nb, const int* tmp, int* items, int* inv, int* bigList,
+                              int* bigCount, const int* gate, int nItems);
+__global__ void k_bucket_sort_big(const int* start, int nb, const int* tmp, int* items, int* inv, const int* bigList,
                                   const int* bigCount, const int* gate, int nItems);
 __global__ void k_mark_build(Params P);
 __global__ void k_pairs_find(Params P);
@@ -47,6 +47,7 @@ size_t candidatesLdsBytes(int maxClusters);
 __global__ void k_bonds(Params P);
 __global__ void k_reduce_kick(Params P, int kick);
 __global__ void k_kick(Params P);
+__global__ void k_dissipation(BodyProp* prop, int n);
 __global__ void k_prime_end(Params P);
 __global__ void k_snap_save(Params P, SnapDev S);
 __global__ void k_snap_restore(Params P, SnapDev S);
@@ -247,7 +248,10 @@ struct lsdem_ctx {
   DBuf<BodyStep> dStep;
   DBuf<float4> dQrel, dWMotion, dWSph, dWQrel, dCert, dCertE, dCertQA, dCertQB;
   DBuf<float> dSurSlack;
-  DBuf<unsigned char> dBodyHit, dForceSet;
+  DBuf<unsigned char> dForceSet;
+  DBuf<uint2> dHitMask;
+  DBuf<int2> dPairSpan, dRcSpan;
+  DBuf<double> dCTerm;
   DBuf<q4> dWBuildQ;
   bool forceRebuild = true;
   bool primePending = false;  // the pre-loop build runs before the next step
@@ -296,39 +300,33 @@ struct lsdem_ctx {
     }
   } sur;
   DBuf<float> dSdf;
-  DBuf<d3> dPos, dPosDet, dVel, dAng, dForce, dTorque, dGorig;
-  DBuf<q4> dQuat;
+  DBuf<d3> dState;     // state vectors of the bodies (Params::pos), walls after the particles
+  DBuf<q4> dQuats;     // their orientations (Params::quat)
+  DBuf<d3> dForce, dTorque;
   DBuf<s6> dInvI;
-  DBuf<double> dInvM, dRadius, dKn, dKs, dMu, dRes, dScale, dInvSp;
-  DBuf<int> dShape, dNodeStart, dScell;
-  DBuf<d3> dWPos, dWVel, dWAng;
-  DBuf<q4> dWQuat;
-  DBuf<double> dWMu, dWRes;
+  DBuf<double> dInvM, dRadius, dScale;
+  DBuf<BodyProp> dProp;
+  DBuf<int> dShape, dScell;
   DBuf<int> dWShape, dWKey;
-  DBuf<d3> dGPos[3];
-  DBuf<q4> dGQuat[3];  // sector images: orientations and velocities
-  DBuf<d3> dGVel[3];
-  DBuf<q4> dQuatDet;   // sector periodicity: detection orientation of the particles
   DBuf<int> dCellCount, dCellStart, dSorted, dRank;
   DBuf<float4> dSPR, dSPRw;
   DBuf<float> dSBoxR;
   DBuf<uint32_t> dPairSlab;
-  DBuf<int> dPairCount, dPairStart, dPairA, dPairCoff, dPairCcnt, dRcCount, dRcStart, dRcPair, dRcRank, dRcTmp;
+  DBuf<int> dPairCount, dPairStart, dPairA, dPairCcnt, dRcCount, dRcStart, dRcPair, dRcSlot, dRcRank, dRcTmp;
   DBuf<int> dSortTmp, dSortBig;
   DBuf<uint32_t> dPairInfo, dOldInfo;
   DBuf<int> dOldStart;
   DBuf<float4> dOldCert;
   DBuf<int> dCNode[2], dCPair;
-  DBuf<d3> dCF, dCTA, dCTB;
   DBuf<uint32_t> dCInfo[2];
   DBuf<d3> dCSpring[2], dCPoint[2], dCNormal[2];
   DBuf<double> dCOverlap[2], dCEn[2], dCEs[2];
   DBuf<unsigned long long> dHashKey[2];
   DBuf<int> dHashVal[2], dHashSlot[2];
   DBuf<unsigned long long> dStatSlots;
-  DBuf<int> dBI, dBJ, dBActive, dBcStart, dBcItem;
-  DBuf<double> dBConst, dBOut;
-  DBuf<d3> dBLocal, dBPoint, dBF, dBMi, dBMj;
+  DBuf<int> dBI, dBJ, dBActive, dBcStart, dBEndAt;
+  DBuf<double> dBConst, dBOut, dBEnd;
+  DBuf<d3> dBLocal, dBPoint;
   DBuf<int> dDevInt, dScanBlocks, dBarrier;
   DBuf<unsigned long long> dDevStat;
   long long hashSize = 0;
@@ -366,23 +364,16 @@ struct lsdem_ctx {
 
 void lsdem_ctx::releaseAll() {
   dShapes.release(); dClusters.release(); dNodes.release(); dNodes32.release(); dPairMap.release(); dSurMask.release(); dClusters32.release(); dSubs32.release(); dSdf.release();
-  dCPair.release(); dCF.release(); dCTA.release(); dCTB.release();
-  dPos.release(); dPosDet.release(); dVel.release(); dAng.release(); dForce.release(); dTorque.release();
-  dGorig.release(); dQuat.release(); dInvI.release();
-  dInvM.release(); dRadius.release(); dKn.release(); dKs.release(); dMu.release(); dRes.release();
-  dScale.release(); dInvSp.release(); dShape.release(); dNodeStart.release(); dScell.release();
-  dWPos.release(); dWVel.release(); dWAng.release(); dWQuat.release(); dWMu.release(); dWRes.release();
+  dCPair.release(); dCTerm.release();
+  dState.release(); dQuats.release(); dForce.release(); dTorque.release(); dInvI.release();
+  dInvM.release(); dRadius.release(); dScale.release(); dProp.release(); dShape.release(); dScell.release();
   dWShape.release(); dWKey.release();
-  for (int s = 0; s < 3; ++s) {
-    dGPos[s].release();
-    dGQuat[s].release();
-    dGVel[s].release();
-  }
   dCellCount.release(); dCellStart.release(); dSorted.release(); dRank.release();
   dSPR.release(); dSPRw.release(); dPairSlab.release(); dStatSlots.release();
   dSBoxR.release();
-  dPairCount.release(); dPairStart.release(); dPairA.release(); dPairCoff.release(); dPairCcnt.release();
-  dRcCount.release(); dRcStart.release(); dRcPair.release(); dRcRank.release(); dRcTmp.release();
+  dPairCount.release(); dPairStart.release(); dPairA.release(); dPairCcnt.release(); dPairSpan.release();
+  dRcCount.release(); dRcStart.release(); dRcPair.release(); dRcSlot.release(); dRcSpan.release();
+  dRcRank.release(); dRcTmp.release();
   dSortTmp.release(); dSortBig.release();
   dPairInfo.release(); dOldInfo.release(); dOldStart.release(); dOldCert.release();
   for (int b = 0; b < 2; ++b) {
@@ -392,15 +383,14 @@ void lsdem_ctx::releaseAll() {
   for (int b = 0; b < 2; ++b) {
     dHashKey[b].release(); dHashVal[b].release(); dHashSlot[b].release();
   }
-  dBI.release(); dBJ.release(); dBActive.release(); dBcStart.release(); dBcItem.release();
-  dBConst.release(); dBOut.release(); dBLocal.release(); dBPoint.release(); dBF.release(); dBMi.release();
-  dBMj.release();
+  dBI.release(); dBJ.release(); dBActive.release(); dBcStart.release(); dBEndAt.release();
+  dBConst.release(); dBOut.release(); dBLocal.release(); dBPoint.release(); dBEnd.release();
   dBarrier.release(); dDevInt.release(); dScanBlocks.release(); dDevStat.release();
   dNodeCluster.release();
   dXBuild.release(); dXBuildW.release(); dWBuildPos.release(); dWBuildQ.release();
   dQBuild.release(); dImgBuild.release(); dStep.release(); dPairRec.release();
   dQrel.release(); dWQrel.release(); dCertE.release(); dCertQA.release(); dCertQB.release();
-  dWMotion.release(); dWSph.release(); dCert.release(); dSurSlack.release(); dBodyHit.release(); dForceSet.release();
+  dWMotion.release(); dWSph.release(); dCert.release(); dSurSlack.release(); dHitMask.release(); dForceSet.release();
   sur.release();
   snap.release();
 }
@@ -459,9 +449,10 @@ int bucketSort(lsdem_ctx* c, const int* bucket, int n, int nb, int* count, int* 
     hipLaunchKernelGGL(k_bucket_scatter, dim3(blocksFor(n, bs)), dim3(bs), 0, c->stream, bucket, n,
                        (const int*)start, (const int*)rank, c->dSortTmp.p, bigCount, gate);
     hipLaunchKernelGGL(k_bucket_sort, dim3(blocksFor(nb, bs)), dim3(bs), 0, c->stream, (const int*)start, nb,
-                       (const int*)c->dSortTmp.p, out, c->dSortBig.p, bigCount, gate, n);
+                       (const int*)c->dSortTmp.p, out, (int*)nullptr, c->dSortBig.p, bigCount, gate, n);
     hipLaunchKernelGGL(k_bucket_sort_big, dim3(unsigned(c->numCU)), dim3(256), 0, c->stream, (const int*)start, nb,
-                       (const int*)c->dSortTmp.p, out, (const int*)c->dSortBig.p, (const int*)bigCount, gate, n);
+                       (const int*)c->dSortTmp.p, out, (int*)nullptr, (const int*)c->dSortBig.p,
+                       (const int*)bigCount, gate, n);
   }
   return LSDEM_OK;
 }
@@ -528,10 +519,10 @@ int pairLaunches(lsdem_ctx* c, const int* gate, Phase& phase) {
   hipLaunchKernelGGL(k_rc_scatter, dim3(gsPairs), dim3(256), 0, s, P);
   const int rcItems = int(std::min<long long>(P.pairCap, (1ll << 31) - 1));
   hipLaunchKernelGGL(k_bucket_sort, dim3(blocksFor(P.nP, 256)), dim3(256), 0, s, (const int*)P.rcStart, P.nP,
-                     (const int*)P.rcTmp, P.rcPair, c->dSortBig.p, P.devInt + 2, gate, rcItems);
+                     (const int*)P.rcTmp, P.rcPair, P.rcSlot, c->dSortBig.p, P.devInt + 2, gate, rcItems);
   hipLaunchKernelGGL(k_bucket_sort_big, dim3(unsigned(c->numCU)), dim3(256), 0, s, (const int*)P.rcStart, P.nP,
-                     (const int*)P.rcTmp, P.rcPair, (const int*)c->dSortBig.p, (const int*)(P.devInt + 2), gate,
-                     rcItems);
+                     (const int*)P.rcTmp, P.rcPair, P.rcSlot, (const int*)c->dSortBig.p, (const int*)(P.devInt + 2),
+                     gate, rcItems);
   return LSDEM_OK;
 }
 
@@ -763,8 +754,8 @@ s6 inverse6(s6 A) {
 int allocPairs(lsdem_ctx* c, long long pairCap) {
   HIPCHK(c->dPairA.alloc(pairCap));
   HIPCHK(c->dPairInfo.alloc(pairCap));
-  HIPCHK(c->dPairCoff.alloc(pairCap));
   HIPCHK(c->dPairCcnt.alloc(pairCap));
+  HIPCHK(c->dPairSpan.alloc(pairCap));
   HIPCHK(c->dSurMask.alloc(pairCap));
   HIPCHK(c->dSurSlack.alloc(pairCap));
   HIPCHK(c->dCert.alloc(pairCap));
@@ -776,6 +767,8 @@ int allocPairs(lsdem_ctx* c, long long pairCap) {
   HIPCHK(c->dPairRec.alloc(pairCap));
   HIPCHK(c->dPairMap.alloc(pairCap * 10));
   HIPCHK(c->dRcPair.alloc(pairCap));
+  HIPCHK(c->dRcSlot.alloc(pairCap));
+  HIPCHK(c->dRcSpan.alloc(pairCap));
   HIPCHK(c->dRcTmp.alloc(pairCap));
   HIPCHK(c->dRcRank.alloc(pairCap));
   c->P.pairCap = pairCap;
@@ -787,9 +780,7 @@ int allocPairs(lsdem_ctx* c, long long pairCap) {
 int allocContacts(lsdem_ctx* c, long long contactCap) {
   hipStream_t s = c->stream;
   HIPCHK(c->dCPair.alloc(contactCap));
-  HIPCHK(c->dCF.alloc(contactCap));
-  HIPCHK(c->dCTA.alloc(contactCap));
-  HIPCHK(c->dCTB.alloc(contactCap));
+  HIPCHK(c->dCTerm.alloc(9 * contactCap));
   for (int b = 0; b < 2; ++b) {
     HIPCHK(c->dCNode[b].alloc(contactCap));
     HIPCHK(c->dCInfo[b].alloc(contactCap));
@@ -898,38 +889,42 @@ void bindPointers(lsdem_ctx* c) {
   Params& P = c->P;
   P.shapes = c->dShapes.p; P.clusters = c->dClusters.p; P.nodes = c->dNodes.p; P.sdf = c->dSdf.p;
   P.nodes32 = c->dNodes32.p; P.clusters32 = c->dClusters32.p; P.subs32 = c->dSubs32.p; P.nodeCluster = c->dNodeCluster.p;
-  P.cPair = c->dCPair.p; P.cF = c->dCF.p; P.cTA = c->dCTA.p; P.cTB = c->dCTB.p;
-  P.pos = c->dPos.p; P.posDet = c->dPosDet.p; P.quat = c->dQuat.p; P.vel = c->dVel.p; P.angvel = c->dAng.p;
+  P.cPair = c->dCPair.p; P.cTerm = c->dCTerm.p;
+  const long long nB = P.nBodies;
+  d3* sv = c->dState.p;
+  q4* sq = c->dQuats.p;
+  P.pos = sv + kSvPos * nB; P.posDet = sv + kSvDet * nB; P.vel = sv + kSvVel * nB; P.angvel = sv + kSvAng * nB;
+  P.quat = sq;
+  P.wpos = P.pos + P.nP; P.wvel = P.vel + P.nP; P.wangvel = P.angvel + P.nP; P.wquat = P.quat + P.nP;
+  const bool images = P.periodicX || P.periodicY || P.periodicSector;
+  for (int g = 0; g < 3; ++g) {  // (used only with the periodicity that allocates them)
+    P.gpos[g] = images ? sv + (kSvImg + g) * nB : nullptr;
+    P.gvel[g] = P.periodicSector ? sv + (kSvImgVel + g) * nB : nullptr;
+    P.gquat[g] = P.periodicSector ? sq + (2 + g) * nB : nullptr;
+  }
+  P.quatDet = P.periodicSector ? sq + nB : nullptr;
   P.force = c->dForce.p; P.torque = c->dTorque.p; P.invI = c->dInvI.p; P.invM = c->dInvM.p;
-  P.radius = c->dRadius.p; P.kn = c->dKn.p; P.ks = c->dKs.p; P.mu = c->dMu.p; P.res = c->dRes.p;
-  P.scale = c->dScale.p; P.invSp = c->dInvSp.p; P.gorig = c->dGorig.p; P.shape = c->dShape.p;
-  P.nodeStart = c->dNodeStart.p; P.scell = c->dScell.p;
+  P.radius = c->dRadius.p; P.scale = c->dScale.p; P.shape = c->dShape.p; P.prop = c->dProp.p; P.scell = c->dScell.p;
   P.xBuild = c->dXBuild.p; P.xBuildW = c->dXBuildW.p; P.wBuildPos = c->dWBuildPos.p; P.wBuildQ = c->dWBuildQ.p;
   P.qBuild = c->dQBuild.p; P.imgBuild = c->dImgBuild.p; P.step = c->dStep.p;
   P.wMotion = c->dWMotion.p; P.wSph = c->dWSph.p; P.cert = c->dCert.p; P.oldInfo = c->dOldInfo.p; P.oldCert = c->dOldCert.p; P.oldStart = c->dOldStart.p; P.pairRec = c->dPairRec.p;
   P.qrel = c->dQrel.p; P.wQrel = c->dWQrel.p; P.certE = c->dCertE.p; P.certQA = c->dCertQA.p; P.certQB = c->dCertQB.p;
   P.surSlack = c->dSurSlack.p;
-  P.bodyHit = c->dBodyHit.p;
+  P.hitMask = c->dHitMask.p;
+  P.pairSpan = c->dPairSpan.p; P.rcSpan = c->dRcSpan.p; P.rcSlot = c->dRcSlot.p;
   P.forceSet = c->dForceSet.p;
-  P.wpos = c->dWPos.p; P.wquat = c->dWQuat.p; P.wvel = c->dWVel.p; P.wangvel = c->dWAng.p;
-  P.wmu = c->dWMu.p; P.wres = c->dWRes.p; P.wshape = c->dWShape.p; P.wkey = c->dWKey.p;
-  for (int g = 0; g < 3; ++g) {
-    P.gpos[g] = c->dGPos[g].p;
-    P.gquat[g] = c->dGQuat[g].p;
-    P.gvel[g] = c->dGVel[g].p;
-  }
-  P.quatDet = c->dQuatDet.p;
+  P.wshape = c->dWShape.p; P.wkey = c->dWKey.p;
   P.cellCount = c->dCellCount.p; P.cellStart = c->dCellStart.p; P.sorted = c->dSorted.p; P.rank = c->dRank.p;
   P.sPR = c->dSPR.p; P.sPRw = c->dSPRw.p; P.pairSlab = c->dPairSlab.p;
   P.sBoxR = c->dSBoxR.p;
   P.statSlots = c->dStatSlots.p;
   P.pairCount = c->dPairCount.p; P.pairStart = c->dPairStart.p; P.pairA = c->dPairA.p;
-  P.pairInfo = c->dPairInfo.p; P.pairCoff = c->dPairCoff.p; P.pairCcnt = c->dPairCcnt.p; P.pairMap = c->dPairMap.p; P.surMask = c->dSurMask.p;
+  P.pairInfo = c->dPairInfo.p; P.pairCcnt = c->dPairCcnt.p; P.pairMap = c->dPairMap.p; P.surMask = c->dSurMask.p;
   P.rcCount = c->dRcCount.p; P.rcStart = c->dRcStart.p; P.rcPair = c->dRcPair.p; P.rcRank = c->dRcRank.p;
   P.rcTmp = c->dRcTmp.p; P.sortTmp = c->dSortTmp.p; P.sortBig = c->dSortBig.p; P.scanTiles = c->dScanBlocks.p;
   P.bI = c->dBI.p; P.bJ = c->dBJ.p; P.bActive = c->dBActive.p; P.bConst = c->dBConst.p; P.bLocal = c->dBLocal.p;
-  P.bPoint = c->dBPoint.p; P.bOut = c->dBOut.p; P.bF = c->dBF.p; P.bMi = c->dBMi.p; P.bMj = c->dBMj.p;
-  P.bcStart = c->dBcStart.p; P.bcItem = c->dBcItem.p;
+  P.bPoint = c->dBPoint.p; P.bOut = c->dBOut.p; P.bEnd = c->dBEnd.p;
+  P.bcStart = c->dBcStart.p; P.bEndAt = c->dBEndAt.p;
   P.barrier = c->dBarrier.p; P.evalCount = c->dBarrier.p + 10 * kBarrierLine;
   P.devInt = c->dDevInt.p; P.devStat = c->dDevStat.p;
   setCurrentBuffers(c);
@@ -1208,38 +1203,57 @@ int lsdem_initialize(lsdem_ctx* c) {
   if ((rc = upload(c->dSdf, sdf, s))) return rc;
 
   // ---- particles ----
-  std::vector<double> invSp(nP);
-  std::vector<d3> gorig(nP), zero3(nP, mk3(0, 0, 0));
-  std::vector<int> nodeStart(nP + 1, 0);
+  std::vector<d3> zero3(nP, mk3(0, 0, 0));
+  std::vector<BodyProp> prop(std::max(nP + nW, 1));
+  int nodeCount = 0;
   double rMax = 0, boxRMax = 0;
   for (int i = 0; i < nP; ++i) {
     const HostShape& S = c->shapes[c->pShape[i]];
-    invSp[i] = 1. / (S.h * c->pScale[i]);
-    gorig[i] = S.origin * c->pScale[i];
-    nodeStart[i + 1] = nodeStart[i] + int(S.nodes.size());
+    const d3 o = S.origin * c->pScale[i];
+    BodyProp& b = prop[i];
+    b = BodyProp{{o.x, o.y, o.z}, c->pScale[i], c->pRadius[i], 1. / (S.h * c->pScale[i]), c->pKn[i], c->pKs[i], c->pMu[i],
+                 c->pRes[i], 0., c->pInvM[i], c->pScale[i] * sd[c->pShape[i]].nodeR, nodeCount, c->pShape[i],
+                 int(S.nodes.size()), {}};
+    if ((long long)nodeCount + (long long)S.nodes.size() >= (1ll << 31) - 1) return fail(LSDEM_ERR_ARG, "too many boundary nodes");
+    nodeCount += int(S.nodes.size());
     rMax = std::max(rMax, c->pRadius[i]);
     boxRMax = std::max(boxRMax, c->pScale[i] * S.boxR);
   }
-  if ((long long)nodeStart[nP] >= (1ll << 31) - 1) return fail(LSDEM_ERR_ARG, "too many boundary nodes");
-  if ((rc = upload(c->dPos, c->pPos, s))) return rc;
-  if ((rc = upload(c->dPosDet, c->pPos, s))) return rc;
-  if ((rc = upload(c->dVel, c->pVel, s))) return rc;
-  if ((rc = upload(c->dAng, c->pAng, s))) return rc;
+  for (int w = 0; w < nW; ++w) {
+    const HostShape& S = c->shapes[c->wShape[w]];
+    prop[nP + w] = BodyProp{{S.origin.x, S.origin.y, S.origin.z}, 1., 0., 1. / S.h, 0., 0., c->wMu[w], c->wRes[w], 0., 0., 0.,
+                            0, c->wShape[w], 0, {}};
+  }
+  {
+    const bool images = P.periodicX || P.periodicY || P.periodicSector;
+    const size_t nB = size_t(std::max(nP + nW, 1));
+    P.nBodies = int(nB);
+    HIPCHK(c->dState.alloc(nB * (P.periodicSector ? kSvImgVel + 3 : images ? kSvImg + 3 : kSvAng + 1)));
+    HIPCHK(c->dQuats.alloc(nB * (P.periodicSector ? 5 : 1)));
+    auto put = [&](auto* to, const auto& v) {
+      return v.empty() ? hipSuccess : hipMemcpyAsync(to, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice, s);
+    };
+    d3* sv = c->dState.p;
+    HIPCHK(put(sv + kSvPos * nB, c->pPos));
+    HIPCHK(put(sv + kSvDet * nB, c->pPos));
+    HIPCHK(put(sv + kSvVel * nB, c->pVel));
+    HIPCHK(put(sv + kSvAng * nB, c->pAng));
+    HIPCHK(put(c->dQuats.p, c->pQuat));
+    HIPCHK(put(sv + kSvPos * nB + nP, c->wPos));
+    HIPCHK(put(sv + kSvDet * nB + nP, c->wPos));
+    HIPCHK(put(sv + kSvVel * nB + nP, c->wVel));
+    HIPCHK(put(sv + kSvAng * nB + nP, c->wAng));
+    HIPCHK(put(c->dQuats.p + nP, c->wQuat));
+  }
+  if ((rc = upload(c->dProp, prop, s))) return rc;
+  hipLaunchKernelGGL(k_dissipation, dim3(blocksFor(nP + nW, 256)), dim3(256), 0, s, c->dProp.p, nP + nW);
   if ((rc = upload(c->dForce, zero3, s))) return rc;
   if ((rc = upload(c->dTorque, zero3, s))) return rc;
-  if ((rc = upload(c->dQuat, c->pQuat, s))) return rc;
   if ((rc = upload(c->dInvI, c->pInvI, s))) return rc;
   if ((rc = upload(c->dInvM, c->pInvM, s))) return rc;
   if ((rc = upload(c->dRadius, c->pRadius, s))) return rc;
-  if ((rc = upload(c->dKn, c->pKn, s))) return rc;
-  if ((rc = upload(c->dKs, c->pKs, s))) return rc;
-  if ((rc = upload(c->dMu, c->pMu, s))) return rc;
-  if ((rc = upload(c->dRes, c->pRes, s))) return rc;
   if ((rc = upload(c->dScale, c->pScale, s))) return rc;
-  if ((rc = upload(c->dInvSp, invSp, s))) return rc;
-  if ((rc = upload(c->dGorig, gorig, s))) return rc;
   if ((rc = upload(c->dShape, c->pShape, s))) return rc;
-  if ((rc = upload(c->dNodeStart, nodeStart, s))) return rc;
   HIPCHK(c->dXBuild.alloc(std::max(nP, 1)));
   HIPCHK(c->dXBuildW.alloc(std::max(nP, 1)));
   HIPCHK(c->dQBuild.alloc(std::max(nP, 1)));
@@ -1249,12 +1263,6 @@ int lsdem_initialize(lsdem_ctx* c) {
   HIPCHK(c->dScell.alloc(std::max(nP, 1)));
 
   // ---- walls ----
-  if ((rc = upload(c->dWPos, c->wPos, s))) return rc;
-  if ((rc = upload(c->dWVel, c->wVel, s))) return rc;
-  if ((rc = upload(c->dWAng, c->wAng, s))) return rc;
-  if ((rc = upload(c->dWQuat, c->wQuat, s))) return rc;
-  if ((rc = upload(c->dWMu, c->wMu, s))) return rc;
-  if ((rc = upload(c->dWRes, c->wRes, s))) return rc;
   if ((rc = upload(c->dWShape, c->wShape, s))) return rc;
   HIPCHK(c->dWKey.alloc(std::max(nW, 1)));
   HIPCHK(c->dWBuildPos.alloc(std::max(nW, 1)));
@@ -1302,15 +1310,6 @@ int lsdem_initialize(lsdem_ctx* c) {
   HIPCHK(c->dSBoxR.alloc(std::max(nP, 1)));
   HIPCHK(c->dPairSlab.alloc(size_t(std::max(nP, 1)) * kPairSlabHost));
   const bool periodic = P.periodicX || P.periodicY || P.periodicSector;
-  for (int g = 0; g < 3; ++g) {
-    const bool on = (g == 0 && P.periodicX) || (g == 1 && P.periodicY) || (g == 2 && P.periodicX && P.periodicY) ||
-                    P.periodicSector;
-    const size_t n = on ? size_t(std::max(nP, 1)) : 1;
-    HIPCHK(c->dGPos[g].alloc(n));
-    HIPCHK(c->dGQuat[g].alloc(P.periodicSector ? n : 1));
-    HIPCHK(c->dGVel[g].alloc(P.periodicSector ? n : 1));
-  }
-  HIPCHK(c->dQuatDet.alloc(P.periodicSector ? size_t(std::max(nP, 1)) : 1));
 
   // ---- pairs and contacts ----
   long long pairCap = c->cfg.pair_capacity > 0 ? c->cfg.pair_capacity : 64ll * nP + 4096 + (periodic ? 32ll * nP : 0);
@@ -1359,7 +1358,7 @@ int lsdem_initialize(lsdem_ctx* c) {
   contactCap = std::min<long long>(contactCap, (1ll << 30));
   HIPCHK(c->dPairCount.alloc(std::max(nP, 1)));
   HIPCHK(c->dPairStart.alloc(nP + 1));
-  HIPCHK(c->dBodyHit.alloc(std::max(nP, 1)));
+  HIPCHK(c->dHitMask.alloc(std::max(nP, 1)));
   HIPCHK(c->dForceSet.alloc(std::max(nP, 1)));
   HIPCHK(c->dOldStart.alloc(nP + 1));
   HIPCHK(c->dRcCount.alloc(std::max(nP, 1)));
@@ -1370,13 +1369,13 @@ int lsdem_initialize(lsdem_ctx* c) {
 
   // ---- bonds (+ per-particle CSR of bond ends, in bond order) ----
   {
-    std::vector<int> cnt(nP + 1, 0), item(2 * nB);
+    std::vector<int> cnt(nP + 1, 0), endAt(2 * nB);
     for (int k = 0; k < nB; ++k) { cnt[c->bI[k] + 1]++; cnt[c->bJ[k] + 1]++; }
     for (int i = 0; i < nP; ++i) cnt[i + 1] += cnt[i];
     std::vector<int> fillp(cnt.begin(), cnt.end() - 1);
     for (int k = 0; k < nB; ++k) {
-      item[fillp[c->bI[k]]++] = (k << 1);
-      item[fillp[c->bJ[k]]++] = (k << 1) | 1;
+      endAt[2 * k] = fillp[c->bI[k]]++;
+      endAt[2 * k + 1] = fillp[c->bJ[k]]++;
     }
     if ((rc = upload(c->dBI, c->bI, s))) return rc;
     if ((rc = upload(c->dBJ, c->bJ, s))) return rc;
@@ -1385,11 +1384,9 @@ int lsdem_initialize(lsdem_ctx* c) {
     if ((rc = upload(c->dBLocal, c->bLocal, s))) return rc;
     if ((rc = upload(c->dBPoint, c->bPoint, s))) return rc;
     if ((rc = upload(c->dBcStart, cnt, s))) return rc;
-    if ((rc = upload(c->dBcItem, item, s))) return rc;
+    if ((rc = upload(c->dBEndAt, endAt, s))) return rc;
     HIPCHK(c->dBOut.alloc(std::max(6 * nB, 1)));
-    HIPCHK(c->dBF.alloc(std::max(nB, 1)));
-    HIPCHK(c->dBMi.alloc(std::max(nB, 1)));
-    HIPCHK(c->dBMj.alloc(std::max(nB, 1)));
+    HIPCHK(c->dBEnd.alloc(std::max(12 * nB, 1)));
     HIPCHK(hipMemsetAsync(c->dBOut.p, 0, sizeof(double) * std::max(6 * nB, 1), s));
   }
 
@@ -1405,7 +1402,7 @@ int lsdem_initialize(lsdem_ctx* c) {
   HIPCHK(hipMemsetAsync(c->dDevInt.p, 0, kDevInts * sizeof(int), s));
   HIPCHK(hipMemsetAsync(c->dDevStat.p, 0, kDevStats * sizeof(unsigned long long), s));
   HIPCHK(hipMemsetAsync(c->dPairStart.p, 0, (nP + 1) * sizeof(int), s));
-  HIPCHK(hipMemsetAsync(c->dBodyHit.p, 0, std::max(nP, 1), s));
+  HIPCHK(hipMemsetAsync(c->dHitMask.p, 0, std::max(nP, 1) * sizeof(uint2), s));
   HIPCHK(hipMemsetAsync(c->dForceSet.p, 1, std::max(nP, 1), s));
 
   P.surSlot = nullptr; P.surBand = 0.f; P.sur = SurNet{}; P.maxClusters = maxClusters;
@@ -1770,10 +1767,10 @@ int lsdem_get_particles(lsdem_ctx* c, double* pos, double* quat, double* vel, do
   HIPCHK(hipStreamSynchronize(c->stream));
   const size_t n = size_t(c->P.nP);
   if (n == 0) return LSDEM_OK;
-  if (pos) HIPCHK(hipMemcpy(pos, c->dPos.p, n * sizeof(d3), hipMemcpyDeviceToHost));
-  if (quat) HIPCHK(hipMemcpy(quat, c->dQuat.p, n * sizeof(q4), hipMemcpyDeviceToHost));
-  if (vel) HIPCHK(hipMemcpy(vel, c->dVel.p, n * sizeof(d3), hipMemcpyDeviceToHost));
-  if (angvel) HIPCHK(hipMemcpy(angvel, c->dAng.p, n * sizeof(d3), hipMemcpyDeviceToHost));
+  if (pos) HIPCHK(hipMemcpy(pos, c->P.pos, n * sizeof(d3), hipMemcpyDeviceToHost));
+  if (quat) HIPCHK(hipMemcpy(quat, c->P.quat, n * sizeof(q4), hipMemcpyDeviceToHost));
+  if (vel) HIPCHK(hipMemcpy(vel, c->P.vel, n * sizeof(d3), hipMemcpyDeviceToHost));
+  if (angvel) HIPCHK(hipMemcpy(angvel, c->P.angvel, n * sizeof(d3), hipMemcpyDeviceToHost));
   if (force) HIPCHK(hipMemcpy(force, c->dForce.p, n * sizeof(d3), hipMemcpyDeviceToHost));
   if (torque) HIPCHK(hipMemcpy(torque, c->dTorque.p, n * sizeof(d3), hipMemcpyDeviceToHost));
   return LSDEM_OK;
@@ -1788,12 +1785,12 @@ int lsdem_set_particles(lsdem_ctx* c, const double* pos, const double* quat, con
   if (n == 0) return LSDEM_OK;
   c->forceRebuild = true;  // poses changed outside the step: rebuild the candidate pairs
   if (pos) {
-    HIPCHK(hipMemcpy(c->dPos.p, pos, n * sizeof(d3), hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(c->dPosDet.p, pos, n * sizeof(d3), hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpy(c->P.pos, pos, n * sizeof(d3), hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpy(c->P.posDet, pos, n * sizeof(d3), hipMemcpyHostToDevice));
   }
-  if (quat) HIPCHK(hipMemcpy(c->dQuat.p, quat, n * sizeof(q4), hipMemcpyHostToDevice));
-  if (vel) HIPCHK(hipMemcpy(c->dVel.p, vel, n * sizeof(d3), hipMemcpyHostToDevice));
-  if (angvel) HIPCHK(hipMemcpy(c->dAng.p, angvel, n * sizeof(d3), hipMemcpyHostToDevice));
+  if (quat) HIPCHK(hipMemcpy(c->P.quat, quat, n * sizeof(q4), hipMemcpyHostToDevice));
+  if (vel) HIPCHK(hipMemcpy(c->P.vel, vel, n * sizeof(d3), hipMemcpyHostToDevice));
+  if (angvel) HIPCHK(hipMemcpy(c->P.angvel, angvel, n * sizeof(d3), hipMemcpyHostToDevice));
   if (force) HIPCHK(hipMemcpy(c->dForce.p, force, n * sizeof(d3), hipMemcpyHostToDevice));
   if (torque) HIPCHK(hipMemcpy(c->dTorque.p, torque, n * sizeof(d3), hipMemcpyHostToDevice));
   if (force || torque) HIPCHK(hipMemset(c->dForceSet.p, 1, n));  // stored sums no longer known to be zero
@@ -1806,10 +1803,10 @@ int lsdem_get_walls(lsdem_ctx* c, double* pos, double* quat, double* vel, double
   HIPCHK(hipStreamSynchronize(c->stream));
   const size_t n = size_t(c->P.nW);
   if (n == 0) return LSDEM_OK;
-  if (pos) HIPCHK(hipMemcpy(pos, c->dWPos.p, n * sizeof(d3), hipMemcpyDeviceToHost));
-  if (quat) HIPCHK(hipMemcpy(quat, c->dWQuat.p, n * sizeof(q4), hipMemcpyDeviceToHost));
-  if (vel) HIPCHK(hipMemcpy(vel, c->dWVel.p, n * sizeof(d3), hipMemcpyDeviceToHost));
-  if (angvel) HIPCHK(hipMemcpy(angvel, c->dWAng.p, n * sizeof(d3), hipMemcpyDeviceToHost));
+  if (pos) HIPCHK(hipMemcpy(pos, c->P.wpos, n * sizeof(d3), hipMemcpyDeviceToHost));
+  if (quat) HIPCHK(hipMemcpy(quat, c->P.wquat, n * sizeof(q4), hipMemcpyDeviceToHost));
+  if (vel) HIPCHK(hipMemcpy(vel, c->P.wvel, n * sizeof(d3), hipMemcpyDeviceToHost));
+  if (angvel) HIPCHK(hipMemcpy(angvel, c->P.wangvel, n * sizeof(d3), hipMemcpyDeviceToHost));
   return LSDEM_OK;
 }
 
@@ -1820,10 +1817,10 @@ int lsdem_set_walls(lsdem_ctx* c, const double* pos, const double* quat, const d
   const size_t n = size_t(c->P.nW);
   if (n == 0) return LSDEM_OK;
   c->forceRebuild = true;  // poses changed outside the step: rebuild the candidate pairs
-  if (pos) HIPCHK(hipMemcpy(c->dWPos.p, pos, n * sizeof(d3), hipMemcpyHostToDevice));
-  if (quat) HIPCHK(hipMemcpy(c->dWQuat.p, quat, n * sizeof(q4), hipMemcpyHostToDevice));
-  if (vel) HIPCHK(hipMemcpy(c->dWVel.p, vel, n * sizeof(d3), hipMemcpyHostToDevice));
-  if (angvel) HIPCHK(hipMemcpy(c->dWAng.p, angvel, n * sizeof(d3), hipMemcpyHostToDevice));
+  if (pos) HIPCHK(hipMemcpy(c->P.wpos, pos, n * sizeof(d3), hipMemcpyHostToDevice));
+  if (quat) HIPCHK(hipMemcpy(c->P.wquat, quat, n * sizeof(q4), hipMemcpyHostToDevice));
+  if (vel) HIPCHK(hipMemcpy(c->P.wvel, vel, n * sizeof(d3), hipMemcpyHostToDevice));
+  if (angvel) HIPCHK(hipMemcpy(c->P.wangvel, angvel, n * sizeof(d3), hipMemcpyHostToDevice));
   return LSDEM_OK;
 }
 

@@ -1,6 +1,8 @@
 // Device data layout of one LS-DEM context.  All arrays live in HBM; the struct is passed by
 // value to every kernel.
 #pragma once
+#include <cstddef>
+
 #include "dmath.h"
 #include "surrogate.h"
 
@@ -62,6 +64,29 @@ struct alignas(16) BodyStep {
   int4 key;
 };
 constexpr int kFlipBit = 30;
+
+// The state vectors' places in their block (Params::pos).
+enum { kSvPos = 0, kSvDet = 1, kSvVel = 2, kSvAng = 3, kSvImg = 4, kSvImgVel = 7 };
+
+// What does not change of a particle or wall, in one 128-byte line: the narrow phase reads it for pairs
+// picked from anywhere in the list, where an array per property cost a line each.
+struct alignas(128) BodyProp {
+  double origin[3];           // scale * grid origin
+  double scale, radius;       // a wall: 1, 0
+  double invSp;               // 1 / (scale * spacing)
+  double kn, ks;              // a wall: 0
+  double mu, res, diss;       // diss = dissipation(res), computed on the device at initialisation
+  double invM;                // a wall: 0
+  double rNode;               // scale * largest node distance from the body's origin
+  int nodeStart, shape;       // first of its boundary nodes in the numbering over all particles
+  int nNodes, pad[3];
+};
+static_assert(sizeof(BodyProp) == 128, "a line each");
+// its values by number, as doubles (kPropInts: nodeStart and shape)
+enum { kPropOrigin = 0, kPropScale = 3, kPropRadius = 4, kPropInvSp = 5, kPropKn = 6, kPropKs = 7, kPropMu = 8, kPropRes = 9,
+       kPropDiss = 10, kPropInvM = 11, kPropInts = 13 };
+static_assert(offsetof(BodyProp, nodeStart) == 8 * kPropInts && offsetof(BodyProp, invM) == 8 * kPropInvM &&
+                  offsetof(BodyProp, radius) == 8 * kPropRadius, "kProp* name BodyProp's doubles");
 static_assert(sizeof(BodyStep) == 32 && alignof(BodyStep) == 16, "step record: motion then key, 16 B each");
 
 struct Params {
@@ -96,6 +121,11 @@ struct Params {
   int maxClusters;        // largest cluster count of any shape
 
   // ---- particles ----
+  // State vectors lie in one block of nBodies = nP + nW entries each, walls after the particles, in the
+  // order of kSv* (pos, posDet, vel, angvel, then the image positions and, with sector periodicity, their
+  // velocities); orientations likewise (quat, then quatDet and the three image sets with sector
+  // periodicity).  Vector s of body i is pos[s * nBodies + i].
+  int nBodies;
   d3* pos;      // state position (after any periodic wrap)
   d3* posDet;   // position used by the particle-particle and wall detection of this step
   q4* quat;
@@ -106,15 +136,9 @@ struct Params {
   const s6* invI;
   const double* invM;
   const double* radius;
-  const double* kn;
-  const double* ks;
-  const double* mu;
-  const double* res;
   const double* scale;
-  const double* invSp;   // 1 / (scale * spacing)
-  const d3* gorig;       // scale * grid origin
   const int* shape;
-  const int* nodeStart;  // N+1 prefix of boundary-node counts
+  const BodyProp* prop;  // per particle, then per wall
   int* scell;            // search-grid cell of pos (post-wrap), rebuild steps only
   d3* xBuild;            // posDet when the candidate pairs were built
   d3* xBuildW;           // pos when the candidate pairs were built
@@ -123,13 +147,11 @@ struct Params {
   BodyStep* step;        // per particle, written every step: motion since the build and keys
   float4* qrel;          // per particle: conj(q_build) q in FP32 (rotation since the build)
 
-  // ---- walls ----
+  // ---- walls (state vectors: nP entries into the particles') ----
   d3* wpos;
   q4* wquat;
   d3* wvel;
   d3* wangvel;
-  const double* wmu;
-  const double* wres;
   const int* wshape;
   int* wkey;
   d3* wBuildPos;         // wall pose when the candidate pairs were built
@@ -171,8 +193,8 @@ struct Params {
   int* pairStart;   // nP + 1
   int* pairA;       // pairCap
   uint32_t* pairInfo;  // (type << 28) | partner
-  int* pairCoff;    // first contact slot of the pair (its contacts are contiguous)
   int* pairCcnt;    // contacts of the pair
+  int2* pairSpan;   // of a pair with contacts: the first of its terms in cTerm and their number
   // separation certificates: a pair whose nodes were all culled with slack s (world units, less
   // the motion bound at that step) is skipped while the motion bound since the build stays below s
   int* oldStart;           // the previous pair list kept through a rebuild: per-master starts (nP + 1),
@@ -189,15 +211,16 @@ struct Params {
   int* rcCount;     // nP
   int* rcStart;     // nP + 1
   int* rcPair;      // pairCap
+  int* rcSlot;      // pairCap: place of a reaction pair in rcPair
+  int2* rcSpan;     // pairSpan of the pairs in rcPair's order
   int* rcRank;      // pairCap (scratch)
 
   // ---- contacts (current step) ----
   int* cNode;
   uint32_t* cInfo;      // (type << 28) | partner, kInvalidInfo for an unused slot
   int* cPair;           // candidate pair of the contact
-  d3* cF;               // force on the master particle
-  d3* cTA;              // torque on the master particle
-  d3* cTB;              // torque on the partner
+  double* cTerm;        // 9 per contact (force, torque on the master, torque on the partner), a pair's
+                        // contacts side by side from its first candidate slot on
   d3* cSpring;
   d3* cPoint;
   d3* cNormal;
@@ -222,11 +245,9 @@ struct Params {
   const d3* bLocal;      // 8 per bond: n1i n2i n3i pi n1j n2j n3j pj
   d3* bPoint;
   double* bOut;          // 6 per bond: Un Us Ub Ut sigmaMax tauMax
-  d3* bF;                // force on i
-  d3* bMi;               // torque on i (moment + arm x F)
-  d3* bMj;               // torque on j
-  const int* bcStart;    // nP + 1 CSR of bond ends per particle
-  const int* bcItem;     // 2*nBonds: (bond << 1) | (0 = i end, 1 = j end)
+  double* bEnd;          // 6 per bond end, in the CSR's order: force and torque (moment + arm x F) there
+  const int* bEndAt;     // 2*nBonds: place of bond k's i end (2k) and j end (2k + 1) in bEnd
+  const int* bcStart;    // nP + 1 CSR of bond ends per particle, in bond order
 
   // ---- device counters ----
   // devInt: [1] contact slots allocated this step, [3] error flags (kErr*: any flag halts every later
@@ -259,8 +280,9 @@ struct Params {
   unsigned long long* surMask;  // per evaluated pair (list position): bit c = 0 when the network
                                 // culls cluster c
   float* surSlack;              // per evaluated pair: smallest slack of the clusters it culled
-  unsigned char* bodyHit;       // per particle: 1 when a pair of it holds candidate nodes this step
-                                // (set by the narrow phase, cleared by the sums that read it)
+  uint2* hitMask;               // per particle: which of its pairs as master (x) and of its reactions (y)
+                                // hold contacts this step (hitBit), set by the narrow phase, cleared by
+                                // the sums that read it
   unsigned char* forceSet;      // per particle: 0 when its stored force and torque are exactly zero
 };
 

@@ -152,17 +152,20 @@ LSD_HD d3 slidingSpring(d3 s0, d3 sv, d3 n, d3 Fn, double mu, double k, double c
   }
   return spring;
 }
+// Dissipation of a contact with restitution `res`: damping ratio of the normal and tangential dashpots.
+LSD_HD double dissipation(double res) {
+  const double logRes = log(res);
+  return -logRes / double(sqrtf(float(logRes * logRes + kPi * kPi)));
+}
 // Force and updated tangential spring of a contact (returned by value: reference outputs kept the
 // pair in scratch memory on the GPU).
 struct ContactLaw {
   d3 F, spring;
 };
 LSD_HD ContactLaw linearContact(d3 spring, d3 vc, d3 n, double delta, double dt, double kn, double ks, double mu,
-                                double res, double effM) {
+                                double diss, double effM) {
   d3 F = mk3(0., 0., 0.);
   if (delta > 0.) {
-    const double logRes = log(res);
-    const double diss = -logRes / double(sqrtf(float(logRes * logRes + kPi * kPi)));
     const double cn = 2. * diss * double(sqrtf(float(effM * kn)));
     const d3 vn = dot(vc, n) * n;
     const d3 Fn = kn * delta * n - cn * vn;

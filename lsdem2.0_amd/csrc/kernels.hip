@@ -537,6 +537,7 @@ __device__ void wallDrift(const Params& P, int w, int buf) {
     q = qintegrate(q, P.wangvel[w], P.dt);
     P.wquat[w] = q;
   }
+  P.posDet[P.nP + w] = p;
   P.wkey[w] = refKey(P.gridW, p);
   // displacement bound of any point of the wall's grid box since the last build: translation plus
   // 2 R sin(angle / 2) for the rotation
@@ -560,6 +561,9 @@ __device__ void markBuildOne(const Params& P, int i) {
     P.xBuild[i] = P.posDet[i];
     P.xBuildW[i] = P.pos[i];
     P.qBuild[i] = P.periodicSector ? P.quatDet[i] : P.quat[i];
+    // (zero already, unless the last call halted on an error between the narrow phase and the sums: the bits
+    // would then name pairs of another list)
+    P.hitMask[i] = make_uint2(0u, 0u);
     BodyStep st = P.step[i];
     st.motion = make_float4(0.f, 0.f, 0.f, 0.f);
     P.qrel[i] = make_float4(1.f, 0.f, 0.f, 0.f);
@@ -597,14 +601,17 @@ __device__ void bucketScatter(const int* bucket, int n, const int* start, const 
 }
 // Buckets of up to 16 items are sorted in registers (odd-even transposition network) from
 // `tmp` into `items`; larger ones are listed for bucketSortBig (*bigCount starts at 0).
-__device__ void bucketSortSmall(const int* start, int nb, const int* tmp, int* items, int* bigList, int* bigCount,
-                                Span g, int nItems) {
+// inv (may be null): also records each item's place, inv[item] = position in items.
+__device__ void bucketSortSmall(const int* start, int nb, const int* tmp, int* items, int* inv, int* bigList,
+                                int* bigCount, Span g, int nItems) {
   for (int b = g.tid; b < nb; b += g.nth) {
     const int s = start[b], e = start[b + 1];
     const int n = e - s;
     if (n <= 0 || s < 0 || e > nItems) continue;  // (never with a complete scan of the counts)
     if (n == 1) {
-      items[s] = tmp[s];
+      const int v0 = tmp[s];
+      items[s] = v0;
+      if (inv) inv[v0] = s;
       continue;
     }
     if (n > 16) {
@@ -626,13 +633,16 @@ __device__ void bucketSortSmall(const int* start, int nb, const int* tmp, int* i
     }
 #pragma unroll
     for (int k = 0; k < 16; ++k)
-      if (k < n) items[s + k] = v[k];
+      if (k < n) {
+        items[s + k] = v[k];
+        if (inv) inv[v[k]] = s + k;
+      }
   }
 }
 // One wavefront per listed bucket: each item's place is the number of smaller items (items are
 // distinct indices).  `wave` / `nWaves`: this wavefront's index and the number of wavefronts.
-__device__ void bucketSortBig(const int* start, const int* tmp, int* items, const int* bigList, const int* bigCount,
-                              int wave, int nWaves, int nb, int nItems) {
+__device__ void bucketSortBig(const int* start, const int* tmp, int* items, int* inv, const int* bigList,
+                              const int* bigCount, int wave, int nWaves, int nb, int nItems) {
   const int lane = threadIdx.x & 63;
   const int nBig = min(*bigCount, nb);
   for (int q = wave; q < nBig; q += nWaves) {
@@ -646,7 +656,10 @@ __device__ void bucketSortBig(const int* start, const int* tmp, int* items, cons
         const int u = c1 + lane < e ? tmp[c1 + lane] : 0x7fffffff;
         for (int k = 0; k < 64; ++k) rank += __shfl(u, k, 64) < v ? 1 : 0;
       }
-      if (c0 + lane < e) items[s + rank] = v;
+      if (c0 + lane < e) {
+        items[s + rank] = v;
+        if (inv) inv[v] = s + rank;
+      }
     }
   }
 }
@@ -660,16 +673,16 @@ __global__ void k_bucket_scatter(const int* bucket, int n, const int* start, con
   if (blockIdx.x == 0 && threadIdx.x == 0) *bigCount = 0;  // list of large buckets of k_bucket_sort
   bucketScatter(bucket, n, start, rank, out, gridSpan());
 }
-__global__ void k_bucket_sort(const int* start, int nb, const int* tmp, int* items, int* bigList, int* bigCount,
-                              const int* gate, int nItems) {
+__global__ void k_bucket_sort(const int* start, int nb, const int* tmp, int* items, int* inv, int* bigList,
+                              int* bigCount, const int* gate, int nItems) {
   LSD_GATE(gate);
-  bucketSortSmall(start, nb, tmp, items, bigList, bigCount, gridSpan(), nItems);
+  bucketSortSmall(start, nb, tmp, items, inv, bigList, bigCount, gridSpan(), nItems);
 }
-__global__ void k_bucket_sort_big(const int* start, int nb, const int* tmp, int* items, const int* bigList,
+__global__ void k_bucket_sort_big(const int* start, int nb, const int* tmp, int* items, int* inv, const int* bigList,
                                   const int* bigCount, const int* gate, int nItems) {
   LSD_GATE(gate);
   const Span g = gridSpan();
-  bucketSortBig(start, tmp, items, bigList, bigCount, g.tid >> 6, g.nth >> 6, nb, nItems);
+  bucketSortBig(start, tmp, items, inv, bigList, bigCount, g.tid >> 6, g.nth >> 6, nb, nItems);
 }
 
 // Search-grid cell of a particle's post-wrap centre: ghost images are searched through their
@@ -1130,6 +1143,13 @@ __device__ __forceinline__ d3 histLookup(const Params& P, unsigned long long key
 // ------------------------------------------------------------------------------------------
 constexpr int kNarrowBlock = 256;
 
+// Contact terms and masks.  Bit of the k-th pair of a body's list in its contact mask: the first kHitBits pairs have a bit each, the
+// rest share the last one (and are then told apart by their contact counts).
+constexpr int kTermDoubles = 9;  // of a contact in cTerm: force, torque on the master, torque on the partner
+constexpr int kHitBits = 31;
+constexpr unsigned int kHitRest = 1u << kHitBits;
+__device__ __forceinline__ unsigned int hitBit(int k) { return k < kHitBits ? 1u << k : kHitRest; }
+
 // Stat slot `slot` of accumulator family f (one 128-byte line per slot).
 __device__ __forceinline__ unsigned long long* statSlot(const Params& P, int f, int slot) {
   return P.statSlots + (f * kStatSlots + slot) * kStatStride;
@@ -1143,7 +1163,7 @@ __device__ __forceinline__ double wsum(double v) {
 
 // Detection-side view of a pair (everything the node tests need).
 struct PairView {
-  int pair, A, partner, nodeBase, valid;
+  int pair, A, partner, nodeBase, nNodes, valid;
   uint32_t type, info;
   d3 xA;        // master position used for detection
   q4 qA;
@@ -1153,9 +1173,8 @@ struct PairView {
   d3 xB;        // partner pose used for detection
   q4 qB;
   double rB;    // particle-particle radius cull (0 for fixed partners)
-  double scB, invSpB;
+  double invSpB;
   d3 goB;
-  int keyB;
 };
 
 // (info and A as in pairInfo[p], pairA[p], when the caller already holds them)
@@ -1170,38 +1189,31 @@ __device__ __forceinline__ PairView loadPair(const Params& P, int p, uint32_t in
   const bool ghost = v.type >= PT_GX;
   v.xA = ghost ? P.pos[v.A] : P.posDet[v.A];
   v.qA = (SEC && !ghost) ? P.quatDet[v.A] : P.quat[v.A];
-  v.sA = P.scale[v.A];
-  const ShapeDev SA = P.shapes[P.shape[v.A]];
+  const BodyProp& pA = P.prop[v.A];
+  v.sA = pA.scale;
+  v.rA = pA.rNode;
+  v.nodeBase = pA.nodeStart;
+  v.nNodes = pA.nNodes;
+  const ShapeDev& SA = P.shapes[pA.shape];
   v.clusterOff = SA.clusterOff;
   v.nClusters = SA.nClusters;
   v.nodeOff = SA.nodeOff;
-  v.rA = v.sA * SA.nodeR;
-  v.nodeBase = P.nodeStart[v.A];
-  const int j = v.partner;
-  if (v.type == PT_PW) {
-    v.xB = P.wpos[j]; v.qB = P.wquat[j]; v.rB = 0.; v.shapeB = P.wshape[j]; v.scB = 1.0;
-    const ShapeDev SB = P.shapes[v.shapeB];
-    v.invSpB = 1. / SB.h; v.goB = mk3(SB.ox, SB.oy, SB.oz); v.keyB = P.wkey[j];
+  const int j = v.type == PT_PW ? P.nP + v.partner : v.partner;  // (walls follow the particles)
+  if (ghost) {
+    v.xB = imgPos<SEC>(P, int(v.type - PT_GX))[j];
+    v.qB = SEC ? imgQuat(P, int(v.type - PT_GX))[j] : P.quat[j];
   } else {
-    // keys from the partner's step record (an image key carries its shift-flip bit there)
-    const int* keys = reinterpret_cast<const int*>(P.step + j) + 4;  // BodyStep::key as 4 ints
-    const int k = keys[v.type == PT_PP ? 0 : 1 + int(v.type - PT_GX)];
-    if (v.type == PT_PP) {
-      v.xB = P.posDet[j]; v.keyB = k;
-      v.qB = SEC ? P.quatDet[j] : P.quat[j];
-    } else {
-      v.xB = imgPos<SEC>(P, int(v.type - PT_GX))[j];
-      v.keyB = k >= 0 ? (k & ~(1 << kFlipBit)) : -1;
-      v.qB = SEC ? imgQuat(P, int(v.type - PT_GX))[j] : P.quat[j];
-    }
-    v.rB = P.radius[j]; v.shapeB = P.shape[j]; v.scB = P.scale[j];
-    v.invSpB = P.invSp[j]; v.goB = P.gorig[j];
+    v.xB = P.posDet[j];
+    v.qB = SEC && v.type == PT_PP ? P.quatDet[j] : P.quat[j];
   }
+  const BodyProp& pB = P.prop[j];
+  v.rB = pB.radius;
+  v.shapeB = pB.shape;
+  v.invSpB = pB.invSp;
+  v.goB = mk3(pB.origin[0], pB.origin[1], pB.origin[2]);
   v.valid = 1;
   return v;
 }
-
-constexpr int kContactChunk = 1024;  // candidate slots reserved per atomic
 
 // The step record's key of a pair's partner of type t (the body's own key, or its image's): a
 // select, since a runtime index into the record's fields would go through scratch memory.
@@ -1212,50 +1224,64 @@ __device__ __forceinline__ int partnerKey(int4 key, uint32_t t) {
 struct NodeHit {
   d3 point, normal;
   double ov;
-  int gnode;
 };
 
-// Exact node-vs-SDF test of global node `ni` (cluster-ordered node array) in the reference's
-// arithmetic: node transform, radius cull or cell window, grid bounds, trilinear overlap >= 0.
+// What the exact test and the contact law of a pair need, in LDS (k_candidates fills it for the pairs of
+// its batch that hold candidate nodes): the state vectors, orientation and properties of both bodies
+// ([0] the master), the law's constants and the partner's cell key.
+struct BodySide {
+  double v[4][3];    // kSvPos, kSvDet, kSvVel, kSvAng (an image's own in place of its body's)
+  double q[4];       // orientation used by the detection
+  double prop[16];   // BodyProp
+};
+struct alignas(16) PairExact {
+  BodySide side[2];
+  double law[5];     // kn, ks, mu, dissipation, effective mass
+  int keyB, pad;
+};
+static_assert(sizeof(PairExact) % 16 == 0, "PairExact records follow one another in LDS");
+__device__ __forceinline__ d3 lds3(const double* v) { return mk3(v[0], v[1], v[2]); }
+__device__ __forceinline__ q4 lds4(const double* v) { return q4{v[0], v[1], v[2], v[3]}; }
+
+// Exact node-vs-SDF test of a node of the pair's master in the reference's arithmetic: node transform,
+// radius cull or cell window, grid bounds, trilinear overlap >= 0.
 // (nB and sdfOff: the partner's grid size and its offset in the SDF pool)
-__device__ __forceinline__ bool exactTest(const Params& P, const PairView& v, const NodeDev& nd, i3 nB,
-                                          long long sdfOff, bool full, NodeHit& h, unsigned long long& tests,
-                                          unsigned long long& queries) {
-  h.gnode = v.nodeBase + nd.orig;
-  const d3 xw = rot(v.qA, mk3(nd.x * v.sA, nd.y * v.sA, nd.z * v.sA)) + v.xA;
-  tests++;
-  if (v.type == PT_PP) {
-    if (len2(xw - v.xB) > v.rB * v.rB) return false;
+__device__ __forceinline__ bool exactTest(const Params& P, const PairExact& X, uint32_t type, d3 nd, i3 nB, int sdfOff,
+                                          NodeHit& h, unsigned int& queries) {
+  const BodySide &A = X.side[0], &B = X.side[1];
+  const double sA = A.prop[kPropScale];
+  // (the images are built after the periodic wrap, from the position the master then has)
+  const d3 xA = lds3(type >= PT_GX ? A.v[kSvPos] : A.v[kSvDet]);
+  const d3 xw = rot(lds4(A.q), mk3(nd.x * sA, nd.y * sA, nd.z * sA)) + xA;
+  const d3 dB = xw - lds3(B.v[kSvDet]);
+  if (type == PT_PP) {
+    const double rB = B.prop[kPropRadius];
+    if (len2(dB) > rB * rB) return false;
   } else {
-    if (!keyInWindow(v.type == PT_PW ? P.gridW : P.gridP, v.keyB, xw)) return false;
+    if (!keyInWindow(type == PT_PW ? P.gridW : P.gridP, X.keyB, xw)) return false;
   }
-  const d3 loc = rotInv(xw - v.xB, v.qB);
-  const double gx = (loc.x - v.goB.x) * v.invSpB, gy = (loc.y - v.goB.y) * v.invSpB,
-               gz = (loc.z - v.goB.z) * v.invSpB;
+  const q4 qB = lds4(B.q);
+  const d3 loc = rotInv(dB, qB), goB = lds3(B.prop + kPropOrigin);
+  const double invSp = B.prop[kPropInvSp];
+  const double gx = (loc.x - goB.x) * invSp, gy = (loc.y - goB.y) * invSp, gz = (loc.z - goB.z) * invSp;
   const int i0 = (int)floor(gx), j0 = (int)floor(gy), k0 = (int)floor(gz);
   if (i0 < 0 || j0 < 0 || k0 < 0 || i0 >= nB.x - 1 || j0 >= nB.y - 1 || k0 >= nB.z - 1) return false;
-  const int i1 = i0 + 1, j1 = j0 + 1, k1 = k0 + 1;
   const double x = gx - double(i0), y = gy - double(j0), z = gz - double(k0);
-  const float* g = P.sdf + sdfOff;
-  double cc[8];
-  cc[0] = double(g[lin3(i3{i0, j0, k0}, nB)]) * v.scB;
-  cc[1] = double(g[lin3(i3{i1, j0, k0}, nB)]) * v.scB;
-  cc[2] = double(g[lin3(i3{i0, j1, k0}, nB)]) * v.scB;
-  cc[3] = double(g[lin3(i3{i1, j1, k0}, nB)]) * v.scB;
-  cc[4] = double(g[lin3(i3{i0, j0, k1}, nB)]) * v.scB;
-  cc[5] = double(g[lin3(i3{i1, j0, k1}, nB)]) * v.scB;
-  cc[6] = double(g[lin3(i3{i0, j1, k1}, nB)]) * v.scB;
-  cc[7] = double(g[lin3(i3{i1, j1, k1}, nB)]) * v.scB;
+  const float* g = P.sdf + sdfOff + lin3(i3{i0, j0, k0}, nB);
+  const int sy = nB.x, sz = nB.x * nB.y;
+  const float f000 = g[0], f100 = g[1], f010 = g[sy], f110 = g[sy + 1];
+  const float f001 = g[sz], f101 = g[sz + 1], f011 = g[sz + sy], f111 = g[sz + sy + 1];
+  const double sc = B.prop[kPropScale];
+  const double cc[8] = {double(f000) * sc, double(f100) * sc, double(f010) * sc, double(f110) * sc,
+                        double(f001) * sc, double(f101) * sc, double(f011) * sc, double(f111) * sc};
   queries++;
   h.ov = -triValue(x, y, z, cc);
   if (!(h.ov >= 0.)) return false;
-  if (full) {
-    d3 n = triGradient((P.quirks & 1) ? double(int(x)) : x, y, z, cc);
-    n = rot(v.qB, n);
-    n = normalize(n);
-    h.normal = n;
-    h.point = xw + 0.5 * h.ov * n;
-  }
+  d3 n = triGradient((P.quirks & 1) ? double(int(x)) : x, y, z, cc);
+  n = rot(qB, n);
+  n = normalize(n);
+  h.normal = n;
+  h.point = xw + 0.5 * h.ov * n;
   return true;
 }
 
@@ -1265,13 +1291,14 @@ __device__ __forceinline__ bool exactTest(const Params& P, const PairView& v, co
 struct alignas(16) PairF32 {
   float m[9], t[3];
   float c[3], r2;     // pp: partner centre in g and squared bounding radius (g units); r2 < 0: no sphere test
-  float hi[3], lo;    // grid box in g: [lo, hi] per axis
+  float lo;           // grid box in g: [lo, n - 1 - lo] per axis
   float phiMargin;    // SDF prefilter margin for FP32 map rounding (unscaled SDF units)
   float rhoScale;     // A's unscaled cluster radius -> g units
   float lipH;         // Lipschitz bound of the partner's SDF per g unit
   int nx, ny, nz, sdfOff;
   int nodeOff, clusterOff, nClusters;  // A's shape
-  int pair;           // candidate pair index
+  int pair, A;        // candidate pair index, its master
+  uint32_t info;      // its list entry
   float gToWorld;     // world length of one g unit (the partner's scaled spacing)
   float o[3], h;      // partner's unscaled grid origin and spacing (g -> local point)
   int slot;           // partner's surrogate family slot, -1 if none (walls)
@@ -1279,6 +1306,9 @@ struct alignas(16) PairF32 {
   float certCB, certCA;  // certificate coefficients of the partner's and the master's rotation
 };
 static_assert(sizeof(PairF32) == 160, "pair map record is 160 bytes");
+// Upper bound of the grid box on an axis of n nodes (rounded to FP32 once more: 4e-6 for 50 nodes, within
+// the 13 margins to spare in -lo).
+__device__ __forceinline__ float boxHi(const PairF32& f, int n) { return float(n - 1) - f.lo; }
 
 __device__ __forceinline__ void makeF32(const Params& P, const PairView& v, PairF32& f) {
   const ShapeDev SB = P.shapes[v.shapeB];
@@ -1308,9 +1338,6 @@ __device__ __forceinline__ void makeF32(const Params& P, const PairView& v, Pair
     f.r2 = -1.f;
   }
   f.lo = float(-abs);
-  f.hi[0] = float(SB.nx - 1 + abs);
-  f.hi[1] = float(SB.ny - 1 + abs);
-  f.hi[2] = float(SB.nz - 1 + abs);
   f.lipH = float(SB.lip * SB.h * (1.0 + 1e-5));
   f.phiMargin = float(SB.lip * SB.h * abs * 2.0 + 1e-30);
   f.rhoScale = float(v.sA * is * (1.0 + 1e-5));
@@ -1320,6 +1347,8 @@ __device__ __forceinline__ void makeF32(const Params& P, const PairView& v, Pair
   f.clusterOff = v.clusterOff;
   f.nClusters = v.nClusters;
   f.pair = v.pair;
+  f.A = v.A;
+  f.info = v.info;
   f.gToWorld = float(1.0 / is);
   f.o[0] = float(SB.ox); f.o[1] = float(SB.oy); f.o[2] = float(SB.oz);
   f.h = float(SB.h);
@@ -1561,7 +1590,7 @@ __global__ __launch_bounds__(256) void k_pair_check(Params P, int full) {
       makeF32(P, v, f);
       out[a] = f;
       P.pairRec[p] = a;
-      evNodes += unsigned(P.nodeStart[v.A + 1] - v.nodeBase);
+      evNodes += unsigned(v.nNodes);
       P.certE[p] = make_float4(sa.motion.x - mB.x, sa.motion.y - mB.y, sa.motion.z - mB.z, flip);
       P.certQA[p] = qA;
       P.certQB[p] = qB;
@@ -1642,9 +1671,9 @@ __device__ __forceinline__ bool clusterGeomF32(const PairF32& f, const ClusterF3
       return false;
     }
   }
-  const float dx = fmaxf(0.f, fmaxf(f.lo - gx, gx - f.hi[0]));
-  const float dy = fmaxf(0.f, fmaxf(f.lo - gy, gy - f.hi[1]));
-  const float dz = fmaxf(0.f, fmaxf(f.lo - gz, gz - f.hi[2]));
+  const float dx = fmaxf(0.f, fmaxf(f.lo - gx, gx - boxHi(f, f.nx)));
+  const float dy = fmaxf(0.f, fmaxf(f.lo - gy, gy - boxHi(f, f.ny)));
+  const float dz = fmaxf(0.f, fmaxf(f.lo - gz, gz - boxHi(f, f.nz)));
   const float d2 = dx * dx + dy * dy + dz * dz;
   if (d2 > rho * rho * 1.0001f) {
     slack = sqrtf(d2) * kSlackRound - rho * 1.00005f;
@@ -1710,8 +1739,8 @@ __device__ __forceinline__ bool nodeF32(const float* __restrict__ sdf, const Pai
       return false;
     }
   }
-  const float out = fmaxf(fmaxf(fmaxf(f.lo - gx, gx - f.hi[0]), fmaxf(f.lo - gy, gy - f.hi[1])),
-                          fmaxf(f.lo - gz, gz - f.hi[2]));
+  const float out = fmaxf(fmaxf(fmaxf(f.lo - gx, gx - boxHi(f, f.nx)), fmaxf(f.lo - gy, gy - boxHi(f, f.ny))),
+                          fmaxf(f.lo - gz, gz - boxHi(f, f.nz)));
   if (out > 0.f) {  // outside the grid box on some axis, by `out`
     slack = out * kSlackRound;
     return false;
@@ -1738,8 +1767,8 @@ __device__ __forceinline__ bool nodeGeomF32(const PairF32& f, float4 n, float& g
       return false;
     }
   }
-  const float out = fmaxf(fmaxf(fmaxf(f.lo - gx, gx - f.hi[0]), fmaxf(f.lo - gy, gy - f.hi[1])),
-                          fmaxf(f.lo - gz, gz - f.hi[2]));
+  const float out = fmaxf(fmaxf(fmaxf(f.lo - gx, gx - boxHi(f, f.nx)), fmaxf(f.lo - gy, gy - boxHi(f, f.ny))),
+                          fmaxf(f.lo - gz, gz - boxHi(f, f.nz)));
   if (out > 0.f) {
     slack = out * kSlackRound;
     return false;
@@ -1775,96 +1804,39 @@ __device__ __forceinline__ bool nodeSdfF32(const PairF32& f, const float (&c)[8]
 }
 
 // Exact test and contact law of one candidate slot: the reference's node-vs-SDF membership in
-// FP64, then (for contacts) tangential history and the linear spring-dashpot.
-// (p, node, pInfo, pA: the slot's pair and node, and that pair's pairInfo and pairA)
-// grid: the partner's grid size and SDF offset when the caller holds the pair's map record (which
-// spares the read of the partner's shape record), else x < 0.  (Values, not a pointer to the record:
-// a pointer that is either to LDS or to global memory makes flat loads.)
-template <bool SEC>
-__device__ void exactSlot(const Params& P, int c, int p, int node, uint32_t pInfo, int pA, int4 grid,
-                          unsigned long long& statQueries, unsigned long long& statContacts) {
-  if (p < 0) {
-    P.cInfo[c] = kInvalidInfo;
-    P.hashSlot[c] = -1;
-    return;
-  }
-  const PairView v = loadPair<SEC>(P, p, pInfo, pA);
-  // everything the contact law and the tangential history need is read here, before the exact
-  // test, so that its round trips overlap the test's: a candidate that is no contact wastes these
-  // reads, a contact saves their latency
+// FP64, then (for contacts) tangential history and the linear spring-dashpot.  f, X: the pair's records in
+// LDS; info: its list entry; node: the candidate in cluster order.  Returns whether the slot is a contact;
+// out: its force and torque on the master, torque on the partner.
+struct SlotTerms {
+  d3 F, TA, TB;
+};
+__device__ __forceinline__ bool exactSlot(const Params& P, int c, const PairF32& f, const PairExact& X, uint32_t info,
+                                          int node, SlotTerms& out, unsigned int& statQueries,
+                                          unsigned int& statContacts) {
   const NodeDev nd = P.nodes[node];
-  const uint32_t type = v.type;
-  const int j = v.partner;
-  const int A = v.A;
-  const d3 riA = P.pos[A];
-  const d3 vA = P.vel[A], wA = P.angvel[A];
-  const double invMA = P.invM[A], knA = P.kn[A], ksA = P.ks[A], muA = P.mu[A], resA = P.res[A];
-  d3 xf, vB, wB;
-  double knB, ksB, invMB, muB, resB;
-  if (type == PT_PW) {
-    xf = P.wpos[j]; vB = P.wvel[j]; wB = P.wangvel[j];
-    knB = ksB = invMB = 0.;
-    muB = P.wmu[j];
-    resB = P.wres[j];
-  } else {
-    xf = (type == PT_PP) ? P.pos[j] : imgPos<SEC>(P, int(type - PT_GX))[j];
-    // an image's velocity (a turned image's is turned), the real body's angular velocity
-    // (contactKernel.cu:236-238)
-    vB = (type != PT_PP && SEC) ? imgVel(P, int(type - PT_GX))[j] : P.vel[j];
-    wB = P.angvel[j];
-    knB = P.kn[j];
-    ksB = P.ks[j];
-    invMB = P.invM[j];
-    muB = P.mu[j];
-    resB = P.res[j];
-  }
-  // tangential history of the same (list, node, partner) from the previous step (its first slot
-  // read now); this step's contact goes into this step's table for the next one
-  const unsigned long long key = histKey(type, v.nodeBase + nd.orig, j);
+  const uint32_t type = info >> 28;
+  // tangential history of the same (list, node, partner) from the previous step (its first slot is read
+  // with the SDF's corners); this step's contact goes into this step's table for the next one
+  const int gnode = reinterpret_cast<const int*>(X.side[0].prop + kPropInts)[0] + nd.orig;
+  const unsigned long long key = histKey(type, gnode, int(info & kPartnerMask));
   const unsigned long long slot0 = mix64(key) & P.hashMask;
   const unsigned long long k0 = P.prevHashKey[slot0];
   const int v0 = P.prevHashVal[slot0];
   NodeHit h;
-  unsigned long long tests = 0;
-  i3 nB;
-  long long sdfOff;
-  if (grid.x >= 0) {
-    nB = i3{grid.x, grid.y, grid.z};
-    sdfOff = grid.w;
-  } else {
-    const ShapeDev SB = P.shapes[v.shapeB];
-    nB = i3{SB.nx, SB.ny, SB.nz};
-    sdfOff = SB.sdfOff;
-  }
-  const bool hit = exactTest(P, v, nd, nB, sdfOff, true, h, tests, statQueries);
-  if (!hit) {
+  if (!exactTest(P, X, type, mk3(nd.x, nd.y, nd.z), i3{f.nx, f.ny, f.nz}, f.sdfOff, h, statQueries)) {
     P.cInfo[c] = kInvalidInfo;
     P.hashSlot[c] = -1;
-    return;
+    return false;
   }
   statContacts++;
-  double kn = 0., ks = 0., effM = 0., mu, res;
-  if (type == PT_PW) {
-    kn = knA; ks = ksA;
-    if (invMA > 0.) effM = 1. / invMA;
-    mu = fmin(muA, muB);
-    res = fmin(resA, resB);
-  } else {
-    if (knA > 0. && knB > 0.) kn = knA * knB / (knA + knB);
-    if (ksA > 0. && ksB > 0.) ks = ksA * ksB / (ksA + ksB);
-    if (invMA > 0. || invMB > 0.) effM = 1. / (invMA + invMB);
-    res = fmin(resA, resB);
-    mu = fmin(muA, muB);
-  }
   d3 spring = histLookup(P, key, slot0, k0, v0);
   // (the slot's stores after every load above)
-  P.cInfo[c] = v.info;
-  P.cNode[c] = h.gnode;
+  P.cInfo[c] = info;
+  P.cNode[c] = gnode;
   P.cPoint[c] = h.point;
   P.cNormal[c] = h.normal;
   P.cOverlap[c] = h.ov;
   P.hashSlot[c] = histInsert(P, key, c);
-  const d3 vc = vA + cross(wA, h.point - riA) - (vB + cross(wB, h.point - xf));
   d3 F = mk3(0., 0., 0.);
   if (P.prime) {
     // the pre-loop build only lists the contact with the spring it found
@@ -1872,20 +1844,95 @@ __device__ void exactSlot(const Params& P, int c, int p, int node, uint32_t pInf
     P.cSpring[c] = spring;
     P.cEn[c] = 0.;
     P.cEs[c] = 0.;
-    P.cF[c] = F;
-    P.cTA[c] = F;
-    P.cTB[c] = F;
-    return;
+    out = SlotTerms{F, F, F};
+    return true;
   }
-  const ContactLaw law = linearContact(spring, vc, h.normal, h.ov, P.dt, kn, ks, mu, res, effM);
+  // (the real body's angular velocity for an image, contactKernel.cu:236-238)
+  const BodySide &A = X.side[0], &B = X.side[1];
+  const d3 armA = h.point - lds3(A.v[kSvPos]), armB = h.point - lds3(B.v[kSvPos]);
+  const d3 vc = lds3(A.v[kSvVel]) + cross(lds3(A.v[kSvAng]), armA) - (lds3(B.v[kSvVel]) + cross(lds3(B.v[kSvAng]), armB));
+  const double kn = X.law[0], ks = X.law[1];
+  const ContactLaw law = linearContact(spring, vc, h.normal, h.ov, P.dt, kn, ks, X.law[2], X.law[3], X.law[4]);
   F = law.F;
   spring = law.spring;
   P.cSpring[c] = spring;
   P.cEn[c] = 0.5 * h.ov * h.ov * kn;
   P.cEs[c] = 0.5 * len2(spring) * ks;
-  P.cF[c] = F;
-  P.cTA[c] = cross(h.point - riA, F);
-  P.cTB[c] = cross(h.point - xf, -F);
+  out = SlotTerms{F, cross(armA, F), cross(armB, -F)};
+  return true;
+}
+
+// v, as a value of turn `turn` of a loop: what is computed from it stays inside the loop.  (No volatile
+// asm: the compiler takes that for a write to memory, and reads uniform values with vector loads from there
+// on.)
+__device__ __forceinline__ int inLoop(int v, int turn) {
+  asm("" : "+v"(v) : "s"(turn));
+  return v;
+}
+
+// One lane's share of a pair's PairExact record: 8 lanes fill a record, 4 per body.  Lane t of a body reads
+// its t-th state vector, the t-th component of its orientation and the t-th quarter of its properties; the
+// state vectors of particles, walls and images lie in one block, so a lane's address needs no choice
+// between arrays.  All reads of a record are in flight together (one round trip).
+struct PairShare {
+  double v[3], q, prop[4];
+  int key;
+};
+template <bool SEC>
+__device__ __forceinline__ PairShare readShare(const Params& P, uint32_t info, int A, int k) {
+  const uint32_t type = info >> 28;
+  const int j = int(info & kPartnerMask), t = k & 3;
+  const bool B = k >= 4, wall = type == PT_PW, ghost = type >= PT_GX;
+  const int g = int(type) - int(PT_GX);
+  const int idx = !B ? A : wall ? P.nP + j : j;
+  int vSlot = t, qSlot = 0;
+  if (B && ghost && t < 2) vSlot = kSvImg + g;
+  if (SEC) {
+    if (B && ghost && t == kSvVel) vSlot = kSvImgVel + g;
+    qSlot = ghost ? (B ? 2 + g : 0) : (B && wall ? 0 : 1);
+  }
+  const double* v = reinterpret_cast<const double*>(P.pos + ((long long)vSlot * P.nBodies + idx));
+  const double* q = reinterpret_cast<const double*>(P.quat + ((long long)qSlot * P.nBodies + idx));
+  const double* prop = reinterpret_cast<const double*>(P.prop + idx) + 4 * t;
+  PairShare r;
+  r.v[0] = v[0]; r.v[1] = v[1]; r.v[2] = v[2];
+  r.q = q[t];
+  r.prop[0] = prop[0]; r.prop[1] = prop[1]; r.prop[2] = prop[2]; r.prop[3] = prop[3];
+  r.key = 0;
+  if (k == 4 && type != PT_PP)
+    r.key = *(wall ? P.wkey + j : reinterpret_cast<const int*>(P.step + j) + 5 + g);  // (BodyStep::key from its y on)
+  return r;
+}
+__device__ __forceinline__ void writeShare(const PairShare& r, uint32_t info, int k, PairExact& X) {
+  const int t = k & 3;
+  BodySide& S = X.side[k >> 2];
+  S.v[t][0] = r.v[0]; S.v[t][1] = r.v[1]; S.v[t][2] = r.v[2];
+  S.q[t] = r.q;
+  S.prop[4 * t] = r.prop[0]; S.prop[4 * t + 1] = r.prop[1]; S.prop[4 * t + 2] = r.prop[2]; S.prop[4 * t + 3] = r.prop[3];
+  // (an image's key carries its shift-flip bit)
+  if (k == 4) X.keyB = ((info >> 28) == PT_PW || r.key < 0) ? r.key : (r.key & ~(1 << kFlipBit));
+}
+// The contact law's constants, once per pair (the master's own stiffnesses and mass against a wall, whose
+// properties hold zeros there): lane k of the pair's 8 takes constant k.
+__device__ __forceinline__ void pairLaw(uint32_t info, int k, PairExact& X) {
+  if (k >= 5) return;
+  const bool wall = (info >> 28) == PT_PW;
+  const int at = k == 0 ? kPropKn : k == 1 ? kPropKs : k == 2 ? kPropMu : k == 3 ? kPropDiss : kPropInvM;
+  const double a = X.side[0].prop[at], b = X.side[1].prop[at];
+  const double resA = X.side[0].prop[kPropRes], resB = X.side[1].prop[kPropRes];
+  const double quot = (k < 2 ? a * b : 1.) / (a + b);
+  double c;
+  if (k < 2) c = wall ? a : (a > 0. && b > 0. ? quot : 0.);              // stiffnesses in series
+  else if (k == 2) c = fmin(a, b);
+  else if (k == 3) c = (resA <= resB || resB != resB) ? a : b;           // of the smaller restitution
+  else c = (a > 0. || b > 0.) ? quot : 0.;                               // 1 / (1 / m_A + 1 / m_B)
+  X.law[k] = c;
+}
+
+// Dissipation of each particle's and wall's restitution for the contact law (once, at initialisation).
+__global__ void k_dissipation(BodyProp* prop, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) prop[i].diss = dissipation(prop[i].res);
 }
 
 constexpr int kBatch = 8;  // candidate pairs per wave batch
@@ -1896,8 +1943,8 @@ constexpr int kSlotStage = 128;  // candidate slots of a batch handed to the exa
 // (pair, sub-cluster) entries with their 16-bit node masks, per-pair counts, offsets and slacks.
 __host__ __device__ inline int candWaveBytes(int maxClusters) {
   const int nEnt = kBatch * maxClusters, nSub = kMaxSub * nEnt;
-  const int b = int(sizeof(PairF32)) * kBatch + 8 * nEnt + 8 * nSub + 4 * nSub + 12 * kBatch + 16 + 8 * kBatch +
-                8 * kSlotStage;
+  const int b = int(sizeof(PairF32)) * kBatch + int(sizeof(PairExact)) * kBatch + 8 * kSlotStage + 16 * kBatch +
+                8 * nEnt + 8 * nSub + 4 * nSub;
   return (b + 15) & ~15;
 }
 size_t candidatesLdsBytes(int maxClusters) { return size_t(candWaveBytes(maxClusters)) * (kNarrowBlock / 64); }
@@ -1922,49 +1969,50 @@ __device__ __forceinline__ float groupMin(float v) {
   return v;
 }
 
-// Candidate nodes: one wavefront per batch of 8 evaluated pairs, three levels of conservative
-// FP32 culls.
+// Candidate nodes: one wavefront per batch of up to 8 evaluated pairs, three levels of conservative
+// FP32 culls, then the exact test of what is left.  Bound by each wavefront's chain of round trips (about 9
+// with the exact test) and by how many wavefronts share a SIMD: 146 registers, 3 wavefronts (256 and 2 when
+// every lane of the exact test loaded its pair's state itself; 101 -> 77 us for 200,000 falling bodies that
+// evaluate some 15,000 pairs a step, 184 -> 160 us for an ordered bed that evaluates 80,000, a falling
+// column of 20,000 at its 20 us either way).  A limit of 128 registers spills 24 and LDS has no room for a
+// fourth wavefront.
 //   1. lanes = (pair, cluster of <= 64 nodes): bounding spheres, grid box, SDF Lipschitz bound at
 //      the cluster centre (or the surrogate's decision); survivors become entries;
 //   2. lanes = (entry, sub-cluster of <= 16 nodes), 16 entries per pass: the same tests with the
 //      sub-cluster's smaller sphere; survivors become sub-entries;
 //   3. lanes = (sub-entry, node), 4 sub-entries per pass: the node prefilter.
-// The batch reserves its exact candidate count with one atomic and writes each pair's candidates
-// to a contiguous range, in (cluster, sub-cluster, node) order.  Every node of a pair is ruled
+// The batch reserves its exact candidate count with one atomic and numbers each pair's candidates
+// consecutively, in (cluster, sub-cluster, node) order.  Every node of a pair is ruled
 // out by exactly one cull (cluster, sub-cluster or node) or becomes a candidate; the smallest
 // slack of those culls, less the rounding of the map, is the pair's separation certificate
 // (none when a node is a candidate).
 template <bool SUR, bool SEC>
-__global__ __launch_bounds__(kNarrowBlock) void k_candidates(Params P) {
+__global__ __launch_bounds__(kNarrowBlock, 3) void k_candidates(Params P) {
   extern __shared__ __align__(16) unsigned char candLds[];
-  const int lane = threadIdx.x & 63, wl = threadIdx.x >> 6;
+  const int lane0 = threadIdx.x & 63, wl = threadIdx.x >> 6;
   const int maxC = P.maxClusters;
   const int entCap = kBatch * maxC, subCap = kMaxSub * entCap;
   unsigned char* wb = candLds + wl * candWaveBytes(maxC);
   PairF32* sF = reinterpret_cast<PairF32*>(wb);
-  int2* sEnt = reinterpret_cast<int2*>(wb + sizeof(PairF32) * kBatch);  // (first sub-cluster, count | pair j << 4)
-  int2* sSub = sEnt + entCap;                                            // (first node, count | j << 16)
-  unsigned int* sMask = reinterpret_cast<unsigned int*>(sSub + subCap);  // 16-bit node masks
-  int* sCnt = reinterpret_cast<int*>(sMask + subCap);
-  int* sOff = sCnt + kBatch;
-  unsigned int* sSlack = reinterpret_cast<unsigned int*>(sOff + kBatch);  // bits of a float >= 0
-  int* sBase4 = reinterpret_cast<int*>(sSlack + kBatch);  // write offsets of the 4 sub-entries of a pass
-  uint32_t* sPInfo = reinterpret_cast<uint32_t*>(sBase4 + 4);  // pairInfo and pairA of the batch's pairs
-  int* sPA = reinterpret_cast<int*>(sPInfo + kBatch);
-  int2* sStage = reinterpret_cast<int2*>(sPA + kBatch);  // (batch pair, node) of the first slots
-  const int q = lane >> 4, b16 = lane & 15;
-  const unsigned int lt16 = (1u << b16) - 1u;
+  PairExact* sX = reinterpret_cast<PairExact*>(sF + kBatch);
+  int2* sStage = reinterpret_cast<int2*>(sX + kBatch);           // (batch pair, node) of the first slots
+  int* sCnt = reinterpret_cast<int*>(sStage + kSlotStage);       // candidates of each pair
+  int* sOff = sCnt + kBatch;                                     // next free slot of each pair
+  int* sHits = sOff + kBatch;                                    // contacts of each pair
+  unsigned int* sSlack = reinterpret_cast<unsigned int*>(sHits + kBatch);  // bits of a float >= 0
+  int2* sEnt = reinterpret_cast<int2*>(sSlack + kBatch);         // (first sub-cluster, count | pair j << 4)
+  int2* sSub = sEnt + entCap;                                    // (first node, count | j << 16)
+  unsigned int* sMask = reinterpret_cast<unsigned int*>(sSub + subCap);  // 16-bit node masks, then also first slot << 16
+  static_assert(kBatch * 4096 <= 65536, "a batch's slot offsets fit 16 bits (shapes have at most 4096 nodes)");
   const float kInf = __builtin_huge_valf();
   LSD_HALT(P);
-  unsigned long long statCand = 0, statEnt = 0, statQueries = 0, statContacts = 0;
+  unsigned int statCand = 0, statEnt = 0, statQueries = 0, statContacts = 0;
   const EvalRecords rec = evalRecords(P);
   const int nAct = rec.n;
   const int wave = __builtin_amdgcn_readfirstlane(int(blockIdx.x * (kNarrowBlock / 64) + wl));
   const int nWaves = int(gridDim.x * (kNarrowBlock / 64));
-  if (wave == 0 && lane == 0) P.devStat[13] += (unsigned long long)nAct;  // evaluated pairs, summed over steps
+  if (wave == 0 && lane0 == 0) P.devStat[13] += (unsigned long long)nAct;  // evaluated pairs, summed over steps
   const int iters = (maxC + 7) >> 3;
-  const int j = lane >> 3, k = lane & 7;
-  const unsigned long long ltMask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   // batch bi takes the evaluated pairs bi, bi + NB, bi + 2 NB, ...: pairs near contact come in
   // spatial runs, and spreading them over the batches keeps the slowest wavefront short
   // pairs per batch: when few pairs are evaluated, small batches spread the slowest pairs (those
@@ -1974,6 +2022,12 @@ __global__ __launch_bounds__(kNarrowBlock) void k_candidates(Params P) {
                                    : (nAct <= nWaves / 8 ? 1 : (nAct <= nWaves / 2 ? 2 : (nAct <= nWaves ? 4 : kBatch)));
   const int NB = (nAct + nb - 1) / nb;
   for (int bi = wave; bi < NB; bi += nWaves) {
+    // (what follows from the lane is worked out in each batch: kept in registers through the loop, the
+    // addresses of every stage together take half of a wavefront's registers)
+    const int lane = inLoop(lane0, bi);
+    const int j = lane >> 3, k = lane & 7, q = lane >> 4, b16 = lane & 15;
+    const unsigned int lt16 = (1u << b16) - 1u;
+    const unsigned long long ltMask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     // ---- level 1: clusters ----
     const int a = bi + j * NB;  // map record
     const bool own = j < nb && a < nAct;
@@ -1988,13 +2042,6 @@ __global__ __launch_bounds__(kNarrowBlock) void k_candidates(Params P) {
     __builtin_amdgcn_wave_barrier();
     const PairF32& f = sF[j];
     const int clusterOff = own ? f.clusterOff : 0, nCl = own ? f.nClusters : 0;
-    // the pair's list entries for the exact test, loaded now and first used at its end
-    uint32_t myInfo = 0;
-    int myA = 0;
-    if (own && k == 0) {
-      myInfo = P.pairInfo[f.pair];
-      myA = P.pairA[f.pair];
-    }
     int E = 0;
     float lmin = kInf;  // smallest slack of this lane's culled clusters
     for (int it = 0; it < iters; ++it) {
@@ -2022,7 +2069,7 @@ __global__ __launch_bounds__(kNarrowBlock) void k_candidates(Params P) {
     }
     lmin = groupMin<8>(lmin);
     if (k == 0) sSlack[j] = __float_as_uint(lmin);
-    statEnt += (lane == 0) ? (unsigned long long)E : 0ull;
+    statEnt += (lane == 0) ? unsigned(E) : 0u;
     __builtin_amdgcn_wave_barrier();
     // ---- level 2: sub-clusters, 16 entries x 4 per pass ----
     int NS = 0;
@@ -2119,17 +2166,27 @@ __global__ __launch_bounds__(kNarrowBlock) void k_candidates(Params P) {
         total += __popcll(m);
       }
     }
-    // the batch's pair entries (loaded at level 1) for the contact flags and the exact test
-    if (k == 0 && j < kBatch) {
-      sPInfo[j] = myInfo;
-      sPA[j] = myA;
-    }
     __builtin_amdgcn_wave_barrier();
-    // ---- one reservation per batch, exact size (its result is first needed after the
-    // certificates) ----
+    // ---- one reservation per batch, exact size, and the reads of what the exact tests need: in flight
+    // together, used after the certificates and the list of slots are done ----
     int first = 0;
     if (total > 0 && lane == 0) first = atomicAdd(&P.devInt[1], total);
-    if (lane < nb && bi + lane * NB < nAct) {
+    const bool mine = lane < nb && bi + lane * NB < nAct;
+    const bool share = own && sCnt[j] > 0;
+    PairShare part{};
+    if (share) part = readShare<SEC>(P, sF[j].info, sF[j].A, k);
+    // the pair's place in its master's list and in its partner's reaction list
+    int masterFirst = 0, rcSlot = -1, rcFirst = 0;
+    if (mine && sCnt[lane] > 0) {
+      const uint32_t info = sF[lane].info, type = info >> 28;
+      const int B = int(info & kPartnerMask);
+      masterFirst = P.pairStart[sF[lane].A];
+      if (type == PT_PP || (type >= PT_GX && B != sF[lane].A)) {
+        rcSlot = P.rcSlot[sF[lane].pair];
+        rcFirst = P.rcStart[B];
+      }
+    }
+    if (mine) {
       const PairF32& fl = sF[lane];
       // separation certificate in world units, net of the motion since the build
       float sg = __uint_as_float(sSlack[lane]);
@@ -2151,8 +2208,47 @@ __global__ __launch_bounds__(kNarrowBlock) void k_candidates(Params P) {
       P.cert[fl.pair] = make_float4(sw > 0.f ? sw : -1.f, fl.certCB, surDep ? -fl.certCA : fl.certCA,
                                     s0 > 0.f ? s0 : -1.f);
     }
+    int contacts = 0;  // contacts of this lane's pair
     if (total > 0) {
-      first = __builtin_amdgcn_readfirstlane(__shfl(first, 0, 64));
+      // ---- slots, relative to the batch's first: a pair's candidates are contiguous, in (cluster,
+      // sub-cluster, node) order.  Lanes = sub-entries: an entry's first slot is its pair's next free one
+      // plus the candidates of the pair's entries before it, counted bit by bit across the wavefront ----
+      if (mine) {
+        int off = 0;
+        for (int jj = 0; jj < lane; ++jj) off += sCnt[jj];
+        sOff[lane] = off;
+        sHits[lane] = 0;
+      }
+      __builtin_amdgcn_wave_barrier();
+      for (int e0 = 0; e0 < NS; e0 += 64) {
+        const int e = e0 + lane;
+        const unsigned int mq = e < NS ? sMask[e] : 0u;
+        const int jj = e < NS ? sSub[e].y >> 16 : 0, n = __popc(mq);
+        unsigned long long same = ~0ull;  // the lanes with an entry of the same pair
+#pragma unroll
+        for (int b = 0; b < 3; ++b) {
+          const unsigned long long m = __ballot((jj >> b) & 1);
+          same &= (jj >> b) & 1 ? m : ~m;
+        }
+        int before = 0, all = 0;
+#pragma unroll
+        for (int b = 0; b < 5; ++b) {
+          const unsigned long long m = __ballot((n >> b) & 1) & same;
+          before += __popcll(m & ltMask) << b;
+          all += __popcll(m) << b;
+        }
+        const int base = sOff[jj] + before;
+        if (e < NS) sMask[e] = mq | unsigned(base) << 16;
+        __builtin_amdgcn_wave_barrier();
+        if (e < NS && (same & ltMask) == 0) sOff[jj] += all;  // (the pair's first lane)
+        __builtin_amdgcn_wave_barrier();
+      }
+      if (share) {
+        writeShare(part, sF[j].info, k, sX[j]);
+        __builtin_amdgcn_wave_barrier();
+        pairLaw(sF[j].info, k, sX[j]);
+      }
+      first = __builtin_amdgcn_readfirstlane(first);
       if ((long long)first + total > P.contactCap) {
         // the call halts with a capacity error; slots reserved below the capacity stay empty
         if (lane == 0) {
@@ -2167,68 +2263,78 @@ __global__ __launch_bounds__(kNarrowBlock) void k_candidates(Params P) {
         total = 0;
       }
     }
-    if (lane < nb && bi + lane * NB < nAct) {
-      const int pr = sF[lane].pair;
-      int off = first;
-      for (int jj = 0; jj < lane; ++jj) off += sCnt[jj];
-      P.pairCoff[pr] = off;
-      P.pairCcnt[pr] = total ? sCnt[lane] : 0;
-      if (total && sCnt[lane] > 0) {
-        // both bodies have contact terms to sum this step
-        P.bodyHit[sPA[lane]] = 1;
-        const uint32_t info = sPInfo[lane];
-        if ((info >> 28) != PT_PW) P.bodyHit[info & kPartnerMask] = 1;
-      }
-      sOff[lane] = off;  // running write offset of each pair
-    }
-    __builtin_amdgcn_wave_barrier();
-    // ---- write candidate slots; a pair's candidates are contiguous ----
-    if (total) {
+    if (total > 0) {
       for (int e0 = 0; e0 < NS; e0 += 4) {
-        if (lane == 0) {
-          for (int t = 0; t < 4 && e0 + t < NS; ++t) {
-            const int jj = sSub[e0 + t].y >> 16;
-            sBase4[t] = sOff[jj];
-            sOff[jj] += __popc(sMask[e0 + t]);
-          }
-        }
-        __builtin_amdgcn_wave_barrier();
         const int e = e0 + q;
         if (e < NS) {
           const unsigned int mq = sMask[e];
           if ((mq >> b16) & 1u) {
             const int2 se = sSub[e];
-            const int dst = sBase4[q] + __popc(mq & lt16);
-            P.cPair[dst] = sF[se.y >> 16].pair;
-            P.cNode[dst] = se.x + b16;  // cluster-ordered node index until the exact test
-            if (dst - first < kSlotStage) sStage[dst - first] = make_int2(se.y >> 16, se.x + b16);
+            const int r = int(mq >> 16) + __popc(mq & lt16);
+            if (r < kSlotStage) sStage[r] = make_int2(se.y >> 16, se.x + b16);
+            else P.cNode[first + r] = se.x + b16;  // cluster-ordered node index until the exact test
           }
         }
-        __builtin_amdgcn_wave_barrier();
       }
-      // the exact test and contact law of this batch's candidates, by the whole wavefront
+      // ---- the exact test and contact law of the batch's candidates, by the whole wavefront, 64 slots at
+      // a time; a pair's contacts leave their terms side by side from the pair's first slot on ----
       __threadfence_block();
       __builtin_amdgcn_wave_barrier();
-      for (int c = first + lane; c < first + total; c += 64) {
-        if (c - first < kSlotStage) {
-          const int2 st = sStage[c - first];
-          const PairF32& fs = sF[st.x];
-          exactSlot<SEC>(P, c, fs.pair, st.y, sPInfo[st.x], sPA[st.x], make_int4(fs.nx, fs.ny, fs.nz, fs.sdfOff),
-                         statQueries, statContacts);
-        } else {
-          const int pc = P.cPair[c];
-          exactSlot<SEC>(P, c, pc, P.cNode[c], P.pairInfo[pc], P.pairA[pc], make_int4(-1, 0, 0, 0), statQueries,
-                         statContacts);
+      for (int r0 = 0; r0 < total; r0 += 64) {
+        const int r = r0 + lane;
+        int jj = 0;
+        bool hit = false;
+        SlotTerms terms{};
+        if (r < total) {
+          int node;
+          if (r < kSlotStage) {
+            const int2 st = sStage[r];
+            jj = st.x;
+            node = st.y;
+          } else {
+            while (r >= sOff[jj]) ++jj;  // (sOff now holds each pair's end)
+            node = P.cNode[first + r];
+          }
+          P.cPair[first + r] = sF[jj].pair;
+          hit = exactSlot(P, first + r, sF[jj], sX[jj], sF[jj].info, node, terms, statQueries, statContacts);
+        }
+        const unsigned long long hits = __ballot(hit);
+        // the hits among this chunk's slots of pair j
+        auto hitsOf = [&](int j) {
+          const int lo = max(sOff[j] - sCnt[j] - r0, 0), hi = min(sOff[j] - r0, 64);
+          return hi > lo ? hits & (~0ull >> (64 - (hi - lo)) << lo) : 0ull;
+        };
+        if (hit) {
+          const int at = first + sOff[jj] - sCnt[jj] + sHits[jj] + __popcll(hitsOf(jj) & ltMask);
+          double* o = P.cTerm + (long long)at * kTermDoubles;
+          o[0] = terms.F.x; o[1] = terms.F.y; o[2] = terms.F.z;
+          o[3] = terms.TA.x; o[4] = terms.TA.y; o[5] = terms.TA.z;
+          o[6] = terms.TB.x; o[7] = terms.TB.y; o[8] = terms.TB.z;
+        }
+        __builtin_amdgcn_wave_barrier();
+        if (mine) sHits[lane] += __popcll(hitsOf(lane));
+        __builtin_amdgcn_wave_barrier();
+      }
+      // each pair with a contact: the place of its terms to both bodies' lists, its bit to their masks
+      if (mine) contacts = sHits[lane];
+      if (contacts > 0) {
+        const int2 span = make_int2(first + sOff[lane] - sCnt[lane], contacts);
+        P.pairSpan[sF[lane].pair] = span;
+        atomicOr(&P.hitMask[sF[lane].A].x, hitBit(sF[lane].pair - masterFirst));
+        if (rcSlot >= 0) {
+          P.rcSpan[rcSlot] = span;
+          atomicOr(&P.hitMask[sF[lane].info & kPartnerMask].y, hitBit(rcSlot - rcFirst));
         }
       }
     }
-    statCand += (lane == 0) ? (unsigned long long)total : 0ull;
+    if (mine) P.pairCcnt[sF[lane].pair] = contacts;
+    statCand += (lane == 0) ? unsigned(total) : 0u;
   }
   const unsigned long long t = (unsigned long long)wsum(double(statCand));
   const unsigned long long te = (unsigned long long)wsum(double(statEnt));
   const unsigned long long tq = (unsigned long long)wsum(double(statQueries));
   const unsigned long long tc = (unsigned long long)wsum(double(statContacts));
-  if (lane == 0 && (t | te)) {
+  if (lane0 == 0 && (t | te)) {
     const int slot = (blockIdx.x + wl) & (kStatSlots - 1);
     atomicAdd(statSlot(P, 0, slot), t);
     atomicAdd(statSlot(P, 1, slot), tq);
@@ -2307,7 +2413,7 @@ __global__ __launch_bounds__(kNarrowBlock) void k_sur_audit(Params P) {
       f = reinterpret_cast<const PairF32*>(P.pairMap)[P.pairRec[p]];
       if (f.slot >= 0) {
         const int A = P.pairA[p];
-        const int orig = P.cNode[c] - P.nodeStart[A];
+        const int orig = P.cNode[c] - P.prop[A].nodeStart;
         const int cluster = P.nodeCluster[f.nodeOff + orig];
         const ClusterF32 cl = P.clusters32[f.clusterOff + cluster];
         bool inside;
@@ -2332,6 +2438,12 @@ __global__ __launch_bounds__(kNarrowBlock) void k_sur_audit(Params P) {
 // ------------------------------------------------------------------------------------------
 // Bonds (one thread per bond)
 // ------------------------------------------------------------------------------------------
+// Force and torque of a bond on one of its bodies, at the place where that body's sums read them.
+__device__ __forceinline__ void bondEnd(const Params& P, int at, d3 F, d3 M) {
+  double* o = P.bEnd + 6ll * at;
+  o[0] = F.x; o[1] = F.y; o[2] = F.z;
+  o[3] = M.x; o[4] = M.y; o[5] = M.z;
+}
 __global__ void k_bonds(Params P) {
   LSD_HALT(P);
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
@@ -2339,9 +2451,8 @@ __global__ void k_bonds(Params P) {
   double* out = P.bOut + 6ll * k;
   if (P.bActive[k] == 0) {
     for (int t = 0; t < 6; ++t) out[t] = 0.;
-    P.bF[k] = mk3(0, 0, 0);
-    P.bMi[k] = mk3(0, 0, 0);
-    P.bMj[k] = mk3(0, 0, 0);
+    bondEnd(P, P.bEndAt[2 * k], mk3(0, 0, 0), mk3(0, 0, 0));
+    bondEnd(P, P.bEndAt[2 * k + 1], mk3(0, 0, 0), mk3(0, 0, 0));
     return;
   }
   const double* C = P.bConst + 9ll * k;
@@ -2383,9 +2494,8 @@ __global__ void k_bonds(Params P) {
     else if (coh > 0. && out[5] > coh - bmu * out[4]) active = 0;
   }
   P.bActive[k] = active;
-  P.bF[k] = F;
-  P.bMi[k] = Mij + cross(rbi - ri, F);
-  P.bMj[k] = Mji + cross(rbj - rj, -F);
+  bondEnd(P, P.bEndAt[2 * k], F, Mij + cross(rbi - ri, F));
+  bondEnd(P, P.bEndAt[2 * k + 1], -F, Mji + cross(rbj - rj, -F));
 }
 
 // ------------------------------------------------------------------------------------------
@@ -2394,43 +2504,80 @@ __global__ void k_bonds(Params P) {
 __device__ void stepEnd(const Params& P);
 __device__ void stepEndWave(const Params& P, int l);
 
-// Contact and bond sums on body b in a fixed order: its master pairs contact by contact, then the
-// reactions of the pairs where it is the partner, then its bonds.
-// A body none of whose pairs holds candidate nodes this step has no contact terms (its pairs'
-// contact counts are all 0) and skips the walk over its pairs.  Returns whether any term was
-// summed (false: F and T are exactly zero).
+// Adds `n` terms to F and T in order: term k is 6 values at base + stride * k, a force and, `tOff` values
+// further, a torque; the force counts with `sign`.  The reads of kTermsAtOnce terms are issued together
+// (as many as the body pass has registers for beside the state it has already read).
+constexpr int kTermsAtOnce = 3;
+__device__ __forceinline__ void addTerms(const double* base, int n, int stride, int tOff, double sign, d3& F, d3& T) {
+  for (int k0 = 0; k0 < n; k0 += kTermsAtOnce) {
+    d3 f[kTermsAtOnce], t[kTermsAtOnce];
+#pragma unroll
+    for (int u = 0; u < kTermsAtOnce; ++u)
+      if (k0 + u < n) {
+        const double* r = base + (long long)stride * (k0 + u);
+        f[u] = mk3(r[0], r[1], r[2]);
+        t[u] = mk3(r[tOff], r[tOff + 1], r[tOff + 2]);
+      }
+#pragma unroll
+    for (int u = 0; u < kTermsAtOnce; ++u)
+      if (k0 + u < n) {
+        F += sign * f[u];
+        T += t[u];
+      }
+  }
+}
+// The contact terms of the pairs whose bits are set, in order; spans: the pairs' places in cTerm (those of
+// four pairs are read together).  tOff: the torque's place in a term.
+__device__ __forceinline__ void addSpans(const Params& P, const int2* spans, unsigned int bits, int tOff, double sign,
+                                         d3& F, d3& T) {
+  while (bits) {
+    int2 sp[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      sp[u] = make_int2(0, 0);
+      if (bits) {
+        sp[u] = spans[__ffs(int(bits)) - 1];
+        bits &= bits - 1;
+      }
+    }
+    for (int u = 0; u < 4; ++u) {
+      const int2 q = u == 0 ? sp[0] : u == 1 ? sp[1] : u == 2 ? sp[2] : sp[3];
+      addTerms(P.cTerm + (long long)q.x * kTermDoubles, q.y, kTermDoubles, tOff, sign, F, T);
+    }
+  }
+}
+
+// Contact and bond sums on body b in a fixed order: its master pairs contact by contact, the reactions of
+// the pairs where it is the partner, its bonds.  The narrow phase left the places of the contact terms in
+// each body's own order and set the bit of each pair with a contact in the body's mask, so a body reads
+// its mask (zero for a body without contacts, whose sums stay exactly zero), then the places, then the
+// terms: three round trips, where a walk over all its pairs took two per pair and one per candidate slot
+// (body pass: 82 -> 31 us for an ordered bed of 27,000 bodies with 7.6 contacts each as master, 53 -> 14 us
+// for 8,000 bodies with 6 bonds each, 26.7 -> 23.3 us for 200,000 falling bodies, of which few touch).
+// Returns whether any term was summed (false: F and T are exactly zero).
 __device__ __forceinline__ bool reduceBody(const Params& P, int b, d3& F, d3& T) {
   F = mk3(0., 0., 0.);
   T = mk3(0., 0., 0.);
-  const bool hit = P.bodyHit[b] != 0;
-  if (hit) P.bodyHit[b] = 0;
-  const long long cap = P.pairCap;
-  for (int p = P.pairStart[b]; hit && p < P.pairStart[b + 1] && p < cap; ++p) {
-    const int c0 = P.pairCoff[p], n = P.pairCcnt[p];
-    for (int c = c0; c < c0 + n; ++c) {
-      if (P.cInfo[c] == kInvalidInfo) continue;
-      F += P.cF[c];
-      T += P.cTA[c];
-    }
+  const uint2 hit = P.hitMask[b];
+  bool any = (hit.x | hit.y) != 0;
+  if (any) {
+    P.hitMask[b] = make_uint2(0u, 0u);
+    const int p0 = P.pairStart[b], p1 = int(min((long long)P.pairStart[b + 1], P.pairCap));
+    addSpans(P, P.pairSpan + p0, hit.x & ~kHitRest, 3, 1.0, F, T);
+    if (hit.x & kHitRest)
+      for (int p = p0 + kHitBits; p < p1; ++p)
+        if (P.pairCcnt[p] > 0) addSpans(P, P.pairSpan + p, 1u, 3, 1.0, F, T);
+    const int q0 = P.rcStart[b], q1 = P.rcStart[b + 1];
+    addSpans(P, P.rcSpan + q0, hit.y & ~kHitRest, 6, -1.0, F, T);
+    if (hit.y & kHitRest)
+      for (int q = q0 + kHitBits; q < q1; ++q)
+        if (P.pairCcnt[P.rcPair[q]] > 0) addSpans(P, P.rcSpan + q, 1u, 6, -1.0, F, T);
   }
-  for (int q = P.rcStart[b]; hit && q < P.rcStart[b + 1]; ++q) {
-    const int p = P.rcPair[q];
-    const int c0 = P.pairCoff[p], n = P.pairCcnt[p];
-    for (int c = c0; c < c0 + n; ++c) {
-      if (P.cInfo[c] == kInvalidInfo) continue;
-      F += -P.cF[c];
-      T += P.cTB[c];
-    }
-  }
-  bool any = hit;
   if (P.nBonds > 0) {
-    for (int q = P.bcStart[b]; q < P.bcStart[b + 1]; ++q) {
-      const int it = P.bcItem[q];
-      const int k = it >> 1;
-      if (it & 1) { F += -P.bF[k]; T += P.bMj[k]; }
-      else { F += P.bF[k]; T += P.bMi[k]; }
-      any = true;
-    }
+    // the bond kernel left each end's terms in this order
+    const int q0 = P.bcStart[b], q1 = P.bcStart[b + 1];
+    any = any || q1 > q0;
+    addTerms(P.bEnd + 6ll * q0, q1 - q0, 6, 3, 1.0, F, T);
   }
   return any;
 }
@@ -2515,7 +2662,7 @@ __global__ void k_prime_end(Params P) {
   LSD_HALT(P);
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
   if (b == 0) stepEnd(P);
-  if (b < P.nP) P.bodyHit[b] = 0;
+  if (b < P.nP) P.hitMask[b] = make_uint2(0u, 0u);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -2544,7 +2691,7 @@ __global__ void k_snap_restore(Params P, SnapDev S) {
   for (int i = g.tid; i < P.nP; i += g.nth) {
     P.pos[i] = S.pos[i]; P.posDet[i] = S.pos[i]; P.vel[i] = S.vel[i]; P.angvel[i] = S.ang[i];
     P.force[i] = S.force[i]; P.torque[i] = S.torque[i]; P.quat[i] = S.quat[i]; P.forceSet[i] = S.forceSet[i];
-    P.bodyHit[i] = 0;
+    P.hitMask[i] = make_uint2(0u, 0u);
   }
   for (int i = g.tid; i <= P.nP; i += g.nth) P.pairStart[i] = 0;
   for (int i = g.tid; i < P.nW; i += g.nth) { P.wpos[i] = S.wpos[i]; P.wquat[i] = S.wquat[i]; }
@@ -2767,9 +2914,9 @@ __global__ __launch_bounds__(kBroadThreads) void k_broad_phase(Params P) {
   if (grid.sync()) return;
   bucketScatter(P.scell, P.nP, P.cellStart, P.rank, P.sortTmp, g);
   if (grid.sync()) return;
-  bucketSortSmall(P.cellStart, ncell, P.sortTmp, P.sorted, P.sortBig, P.devInt + 2, g, P.nP);
+  bucketSortSmall(P.cellStart, ncell, P.sortTmp, P.sorted, nullptr, P.sortBig, P.devInt + 2, g, P.nP);
   if (grid.sync()) return;
-  bucketSortBig(P.cellStart, P.sortTmp, P.sorted, P.sortBig, P.devInt + 2, wave, nWaves, ncell, P.nP);
+  bucketSortBig(P.cellStart, P.sortTmp, P.sorted, nullptr, P.sortBig, P.devInt + 2, wave, nWaves, ncell, P.nP);
   if (grid.sync()) return;
   // particle data in sorted order; candidate pairs per master, prefix, pair list
   for (int k = g.tid; k < P.nP; k += g.nth) gatherParticle(P, k);
@@ -2800,9 +2947,9 @@ __global__ __launch_bounds__(kBroadThreads) void k_broad_phase(Params P) {
   rcScatterPairs(P, g);
   if (grid.sync()) return;
   const int nRc = min(P.rcStart[P.nP], int(P.pairCap));
-  bucketSortSmall(P.rcStart, P.nP, P.rcTmp, P.rcPair, P.sortBig, P.devInt + 2, g, nRc);
+  bucketSortSmall(P.rcStart, P.nP, P.rcTmp, P.rcPair, P.rcSlot, P.sortBig, P.devInt + 2, g, nRc);
   if (grid.sync()) return;
-  bucketSortBig(P.rcStart, P.rcTmp, P.rcPair, P.sortBig, P.devInt + 2, wave, nWaves, P.nP, nRc);
+  bucketSortBig(P.rcStart, P.rcTmp, P.rcPair, P.rcSlot, P.sortBig, P.devInt + 2, wave, nWaves, P.nP, nRc);
 }
 
 template __global__ void k_candidates<false, false>(Params P);

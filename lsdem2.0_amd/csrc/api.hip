@@ -36,7 +36,6 @@ __global__ void k_pairs_find(Params P);
 __global__ void k_pairs_emit(Params P);
 __global__ void k_backup_pairs(Params P);
 __global__ void k_inherit_certs(Params P);
-__global__ void k_rc_count(Params P);
 __global__ void k_rc_scatter(Params P);
 __global__ void k_gather_particles(Params P);
 template <bool SEC> __global__ void k_pair_check(Params P, int full);
@@ -237,7 +236,6 @@ struct lsdem_ctx {
 
   // device
   DBuf<ShapeDev> dShapes;
-  DBuf<ClusterDev> dClusters;
   DBuf<NodeDev> dNodes;
   DBuf<float4> dNodes32, dPairMap;
   DBuf<unsigned long long> dSurMask;
@@ -312,6 +310,7 @@ struct lsdem_ctx {
   DBuf<float4> dSPR, dSPRw;
   DBuf<float> dSBoxR;
   DBuf<uint32_t> dPairSlab;
+  DBuf<unsigned long long> dWallMask;
   DBuf<int> dPairCount, dPairStart, dPairA, dPairCcnt, dRcCount, dRcStart, dRcPair, dRcSlot, dRcRank, dRcTmp;
   DBuf<int> dSortTmp, dSortBig;
   DBuf<uint32_t> dPairInfo, dOldInfo;
@@ -363,13 +362,13 @@ struct lsdem_ctx {
 };
 
 void lsdem_ctx::releaseAll() {
-  dShapes.release(); dClusters.release(); dNodes.release(); dNodes32.release(); dPairMap.release(); dSurMask.release(); dClusters32.release(); dSubs32.release(); dSdf.release();
+  dShapes.release(); dNodes.release(); dNodes32.release(); dPairMap.release(); dSurMask.release(); dClusters32.release(); dSubs32.release(); dSdf.release();
   dCPair.release(); dCTerm.release();
   dState.release(); dQuats.release(); dForce.release(); dTorque.release(); dInvI.release();
   dInvM.release(); dRadius.release(); dScale.release(); dProp.release(); dShape.release(); dScell.release();
   dWShape.release(); dWKey.release();
   dCellCount.release(); dCellStart.release(); dSorted.release(); dRank.release();
-  dSPR.release(); dSPRw.release(); dPairSlab.release(); dStatSlots.release();
+  dSPR.release(); dSPRw.release(); dPairSlab.release(); dWallMask.release(); dStatSlots.release();
   dSBoxR.release();
   dPairCount.release(); dPairStart.release(); dPairA.release(); dPairCcnt.release(); dPairSpan.release();
   dRcCount.release(); dRcStart.release(); dRcPair.release(); dRcSlot.release(); dRcSpan.release();
@@ -502,18 +501,18 @@ int pairLaunches(lsdem_ctx* c, const int* gate, Phase& phase) {
   Params& P = c->P;
   hipStream_t s = c->stream;
   int rc;
-  hipLaunchKernelGGL(k_pairs_find, dim3(blocksFor(P.nP, 128)), dim3(128), 0, s, P);
+  const unsigned gsFind = blocksFor(P.nP, 256 / 32);  // 32 lanes per master
+  hipLaunchKernelGGL(k_pairs_find, dim3(gsFind), dim3(256), 0, s, P);
   hipLaunchKernelGGL(k_backup_pairs, dim3(unsigned(c->numCU * 4)), dim3(256), 0, s, P);
   rc = scan(c, P.pairCount, P.nP, P.pairStart, gate);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_pairs_emit, dim3(blocksFor(P.nP, 128)), dim3(128), 0, s, P);
+  hipLaunchKernelGGL(k_fill_int, dim3(blocksFor(P.nP, 256)), dim3(256), 0, s, P.rcCount, (long long)P.nP, 0, gate);
+  hipLaunchKernelGGL(k_pairs_emit, dim3(blocksFor(P.nP, 32)), dim3(256), 0, s, P);
   hipLaunchKernelGGL(k_inherit_certs, dim3(unsigned(c->numCU * 4)), dim3(256), 0, s, P);
   hipLaunchKernelGGL(k_mark_build, dim3(blocksFor(std::max(P.nP, P.nW), 256)), dim3(256), 0, s, P);
   phase();
-  // reaction CSR
-  hipLaunchKernelGGL(k_fill_int, dim3(blocksFor(P.nP, 256)), dim3(256), 0, s, P.rcCount, (long long)P.nP, 0, gate);
+  // reaction CSR (the pairs were counted as they were written)
   const unsigned gsPairs = unsigned(c->numCU * 8);
-  hipLaunchKernelGGL(k_rc_count, dim3(gsPairs), dim3(256), 0, s, P);
   rc = scan(c, P.rcCount, P.nP, P.rcStart, gate);
   if (rc) return rc;
   hipLaunchKernelGGL(k_rc_scatter, dim3(gsPairs), dim3(256), 0, s, P);
@@ -887,7 +886,7 @@ void sectorRotation(double angle, d3& w, double& A, double& B, q4& r) {
 // Device pointers of every context array into the Params table.
 void bindPointers(lsdem_ctx* c) {
   Params& P = c->P;
-  P.shapes = c->dShapes.p; P.clusters = c->dClusters.p; P.nodes = c->dNodes.p; P.sdf = c->dSdf.p;
+  P.shapes = c->dShapes.p; P.nodes = c->dNodes.p; P.sdf = c->dSdf.p;
   P.nodes32 = c->dNodes32.p; P.clusters32 = c->dClusters32.p; P.subs32 = c->dSubs32.p; P.nodeCluster = c->dNodeCluster.p;
   P.cPair = c->dCPair.p; P.cTerm = c->dCTerm.p;
   const long long nB = P.nBodies;
@@ -915,7 +914,7 @@ void bindPointers(lsdem_ctx* c) {
   P.forceSet = c->dForceSet.p;
   P.wshape = c->dWShape.p; P.wkey = c->dWKey.p;
   P.cellCount = c->dCellCount.p; P.cellStart = c->dCellStart.p; P.sorted = c->dSorted.p; P.rank = c->dRank.p;
-  P.sPR = c->dSPR.p; P.sPRw = c->dSPRw.p; P.pairSlab = c->dPairSlab.p;
+  P.sPR = c->dSPR.p; P.sPRw = c->dSPRw.p; P.pairSlab = c->dPairSlab.p; P.wallMask = c->dWallMask.p;
   P.sBoxR = c->dSBoxR.p;
   P.statSlots = c->dStatSlots.p;
   P.pairCount = c->dPairCount.p; P.pairStart = c->dPairStart.p; P.pairA = c->dPairA.p;
@@ -925,7 +924,7 @@ void bindPointers(lsdem_ctx* c) {
   P.bI = c->dBI.p; P.bJ = c->dBJ.p; P.bActive = c->dBActive.p; P.bConst = c->dBConst.p; P.bLocal = c->dBLocal.p;
   P.bPoint = c->dBPoint.p; P.bOut = c->dBOut.p; P.bEnd = c->dBEnd.p;
   P.bcStart = c->dBcStart.p; P.bEndAt = c->dBEndAt.p;
-  P.barrier = c->dBarrier.p; P.evalCount = c->dBarrier.p + 10 * kBarrierLine;
+  P.barrier = c->dBarrier.p;
   P.devInt = c->dDevInt.p; P.devStat = c->dDevStat.p;
   setCurrentBuffers(c);
 }
@@ -1119,7 +1118,7 @@ int lsdem_initialize(lsdem_ctx* c) {
   const int nB = int(c->bI.size());
   Params& P = c->P;
   P = Params{};
-  P.nP = nP; P.nW = nW; P.nShapes = nS; P.nBonds = nB;
+  P.nP = nP; P.nW = nW; P.nBonds = nB;
   P.g = mk3(c->cfg.gravity[0], c->cfg.gravity[1], c->cfg.gravity[2]);
   P.dt = c->cfg.dt;
   P.quirks = c->cfg.quirks;
@@ -1161,7 +1160,6 @@ int lsdem_initialize(lsdem_ctx* c) {
   }
   int rc;
   if ((rc = upload(c->dShapes, sd, s))) return rc;
-  if ((rc = upload(c->dClusters, cls, s))) return rc;
   if ((rc = upload(c->dNodes, nds, s))) return rc;
   {
     std::vector<float4> n32(nds.size());
@@ -1309,6 +1307,7 @@ int lsdem_initialize(lsdem_ctx* c) {
   HIPCHK(c->dSPRw.alloc(std::max(nP, 1)));
   HIPCHK(c->dSBoxR.alloc(std::max(nP, 1)));
   HIPCHK(c->dPairSlab.alloc(size_t(std::max(nP, 1)) * kPairSlabHost));
+  HIPCHK(c->dWallMask.alloc(std::max(nP, 1)));
   const bool periodic = P.periodicX || P.periodicY || P.periodicSector;
 
   // ---- pairs and contacts ----
@@ -1323,12 +1322,14 @@ int lsdem_initialize(lsdem_ctx* c) {
     HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, reinterpret_cast<const void*>(k_broad_phase),
                                                         kBroadThreadsHost, 0));
     if (perCU < 1) return fail(LSDEM_ERR_HIP, "the single-launch broad phase does not fit a CU");
-    // one block of 1024 threads per 512 particles or per 16,384 search cells (the cell loops of a
-    // sparse domain, such as an ensemble of drums far apart), at least 8 and at most one per CU: a
-    // small simulation leaves the rest of the GPU to others stepped concurrently, and its rebuilds
-    // meet at barriers of few blocks
+    // blocks of 1024 threads: one per 512 particles or per 16,384 search cells (the cell loops of a sparse
+    // domain, such as an ensemble of drums far apart), at most one per CU; for fewer than 32,768 particles
+    // one per 64, up to a quarter of the GPU, so that four simulations of that size (the hardware queues a
+    // process has) stepped concurrently still have all their blocks resident together (a rebuild of 4,000
+    // bodies takes 304 us with 8 blocks and 152 with 63, one of 20,000 339 with 40 and 276 with 64)
     const long long byCells = ((long long)P.sg.ncell + 16383) / 16384;
-    c->coopBlocks = int(std::min<long long>(c->numCU, std::max<long long>({8, (nP + 511) / 512, byCells})));
+    const long long forSearch = std::min<long long>(c->numCU / 4, (nP + 63) / 64);
+    c->coopBlocks = int(std::min<long long>(c->numCU, std::max<long long>({8, (nP + 511) / 512, byCells, forSearch})));
     if (c->cfg.broad_phase_blocks > 0) c->coopBlocks = std::min(c->numCU, int(c->cfg.broad_phase_blocks));
     c->coopBlocks = std::min(c->coopBlocks, perCU * c->numCU);  // all resident together on an idle GPU
   }

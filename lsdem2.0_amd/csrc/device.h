@@ -89,9 +89,11 @@ static_assert(offsetof(BodyProp, nodeStart) == 8 * kPropInts && offsetof(BodyPro
                   offsetof(BodyProp, radius) == 8 * kPropRadius, "kProp* name BodyProp's doubles");
 static_assert(sizeof(BodyStep) == 32 && alignof(BodyStep) == 16, "step record: motion then key, 16 B each");
 
+constexpr int kBarrierLine = 32;                  // ints per barrier word (one 128-byte line each)
+
 struct Params {
   // ---- sizes and scalars ----
-  int nP, nW, nShapes, nBonds;
+  int nP, nW, nBonds;
   d3 g;
   double dt;
   int quirks, periodicX, periodicY, sdfCull;
@@ -111,7 +113,6 @@ struct Params {
 
   // ---- shapes ----
   const ShapeDev* shapes;
-  const ClusterDev* clusters;
   const NodeDev* nodes;
   const ClusterF32* clusters32;
   const ClusterF32* subs32;  // sub-clusters of <= 16 nodes
@@ -186,7 +187,8 @@ struct Params {
   int* sortTmp;     // counting-sort scratch (items before the per-bucket sort)
   int* sortBig;     // counting-sort scratch (list of buckets of more than 16 items)
   int* scanTiles;   // scan scratch (tile sums)
-  uint32_t* pairSlab;  // kPairSlab x nP: first candidate pairs of each master (column per master)
+  uint32_t* pairSlab;  // nP x kPairSlab: first candidate pairs of each master (32 of each master in a row)
+  unsigned long long* wallMask;  // per sorted position, with up to 64 walls: those the particle can reach
 
   // ---- candidate pairs (current step) ----
   int* pairCount;   // nP (+1) counts then exclusive prefix pairStart
@@ -256,13 +258,12 @@ struct Params {
   //         [7] images at their source's own position, [8] rebuild flag of the step,
   //         [9] (unused), [10 + b] contact slots of the
   //         last step that filled history table b, [12] grid-barrier arrivals of the broad phase,
-  //         [20] callStep of the step that raised the first error flag (-1: none)
+  //         [20] callStep of the step that raised the first error flag (-1: none), [21], [22] a rebuild's
+  //         large buckets (kBigCellsIdx, kBigRcIdx)
   int* devInt;
   int* barrier;          // grid barrier of the single-launch broad phase: kBarrierLine-int lines, one per
                          // block group (blockIdx mod 8), then the groups' counter, then the release word;
-                         // then 8 lines of evalCount
-  int* evalCount;        // word g * kBarrierLine: map records the pair check's block group g (blockIdx
-                         // mod 8) wrote this step, in its own region of pairMap
+                         // then 8 lines of evalCount(P)
   // devStat: [0] node tests, [1] sdf queries, [2] contacts (this step);
   //          [3] pairs, [4] node tests, [5] sdf queries, [6] contacts, [8] cluster entries
   //          (summed while profiling); [9] audits, [10] audited contacts, [11] missed contacts
@@ -285,6 +286,10 @@ struct Params {
                                 // the sums that read it
   unsigned char* forceSet;      // per particle: 0 when its stored force and torque are exactly zero
 };
+
+// Word g * kBarrierLine: map records the pair check's block group g (blockIdx mod 8) wrote this step, in its own
+// region of pairMap.
+__device__ inline int* evalCount(const Params& P) { return P.barrier + 10 * kBarrierLine; }
 
 // What opens a step besides the bodies: the table of tangential history this step fills, its slot
 // list from two steps ago, the step's buffer (flag set, clear count) and the host's rebuild request.
@@ -334,7 +339,6 @@ constexpr int kWaveEndBodies = 65536;
 constexpr int kStatStride = 16;
 constexpr int kStatWords = 5 * kStatSlots * kStatStride;
 constexpr int kDevInts = 32;   // devInt entries
-constexpr int kBarrierLine = 32;                  // ints per barrier word (one 128-byte line each)
 constexpr int kBarrierInts = 18 * kBarrierLine;   // 8 groups, the groups' counter, the release word, evalCount
 // The step's rebuild flag and its count of ghost images left at their source's position, two sets
 // used in alternate steps (buffer = Params::curBuf): the kernel that closes one step may already
@@ -342,8 +346,9 @@ constexpr int kBarrierInts = 18 * kBarrierLine;   // 8 groups, the groups' count
 __host__ __device__ inline int rebuildFlagIdx(int buf) { return 16 + buf; }
 __host__ __device__ inline int ghostCountIdx(int buf) { return 18 + buf; }
 constexpr int kDevStats = 16;  // devStat entries
-constexpr int kPairSlabHost = 16;
-constexpr int kBroadThreadsHost = 1024;  // block of the single-launch broad phase (kBroadThreads)  // slab depth of the broad phase (kPairSlab in the kernels)
+constexpr int kPairSlabHost = 32;        // candidate pairs of a master kept by the search (kPairSlab in the kernels)
+constexpr int kBroadThreadsHost = 1024;  // block of the single-launch broad phase (kBroadThreads)
+constexpr int kBigCellsIdx = 21, kBigRcIdx = 22;  // devInt: a rebuild has cells (reaction lists) of many items
 constexpr uint32_t kInvalidInfo = 0xFFFFFFFFu;  // unused contact slot
 
 }  // namespace lsd

@@ -213,7 +213,10 @@ __device__ void scanReduceTiles(const int* in, long long n, int* tileSum, int* l
 }
 // Phase 2: each tile adds the sums of the tiles before it and writes its exclusive prefix; the
 // last tile writes the total to out[n].  n == 0 writes out[0] = 0.
-__device__ void scanApplyTiles(const int* in, long long n, const int* tileSum, int* out, int* lds) {
+// bigFlag (may be null): set to 1 when an input is above kSmallBucket.
+constexpr int kSmallBucket = 16;  // items of a bucket that bucketSortSmall sorts
+__device__ void scanApplyTiles(const int* in, long long n, const int* tileSum, int* out, int* lds,
+                               int* bigFlag = nullptr) {
   const long long tile = (long long)blockDim.x * kScanItems;
   const long long nTiles = (n + tile - 1) / tile;
   if (n == 0 && blockIdx.x == 0 && threadIdx.x == 0) out[0] = 0;
@@ -229,6 +232,7 @@ __device__ void scanApplyTiles(const int* in, long long n, const int* tileSum, i
     for (int k = 0; k < kScanItems; ++k) {
       v[k] = (base + k < n) ? in[base + k] : 0;
       s += v[k];
+      if (bigFlag && v[k] > kSmallBucket) *bigFlag = 1;
     }
     int total;
     int ex = blockExclusiveScan(s, lds, total) + preTotal;
@@ -363,7 +367,7 @@ __device__ __forceinline__ void stepHead(const Params& P, const StepHead& H, int
     if (H.forceRebuild) atomicOr(&P.devInt[rebuildFlagIdx(H.buf)], 1);
     P.devInt[1] = 0;   // contact slots allocated
   }
-  if (i < 8) P.evalCount[i * kBarrierLine] = 0;  // map records of the pair check's block groups
+  if (i < 8) evalCount(P)[i * kBarrierLine] = 0;  // map records of the pair check's block groups
   const int nClear = P.devInt[10 + H.buf];
   for (int c = i; c < nClear; c += nth) {
     const int slot = H.hashSlot[c];
@@ -636,7 +640,7 @@ __device__ void bucketSortSmall(const int* start, int nb, const int* tmp, int* i
       if (inv) inv[v0] = s;
       continue;
     }
-    if (n > 16) {
+    if (n > kSmallBucket) {
       const int q = atomicAdd(bigCount, 1);
       if (q < nb) bigList[q] = b;
       continue;
@@ -707,100 +711,6 @@ __global__ void k_bucket_sort_big(const int* start, int nb, const int* tmp, int*
   bucketSortBig(start, tmp, items, inv, bigList, bigCount, g.tid >> 6, g.nth >> 6, nb, nItems);
 }
 
-// Search-grid cell of a particle's post-wrap centre: ghost images are searched through their
-// sources, and a particle that wrapped this step is outside the domain before the wrap (never a pp
-// partner).
-__device__ __forceinline__ int searchCellOf(const Params& P, int i) {
-  return lin3(searchCell(P.sg, P.pos[i]), P.sg.size);
-}
-
-// Gather particle (or ghost-image) data into the sorted order of the search-grid table so
-// that the candidate loops stream contiguous memory.
-__device__ void gatherParticle(const Params& P, int k) {
-  const int i = P.sorted[k];
-  const d3 x = P.posDet[i], w = P.pos[i];
-  const float r = float(P.radius[i]);
-  // a pp partner must be inside the domain when the pair is used; one that can get there before
-  // the next rebuild (within half the skin) stays a candidate
-  const bool eligible = P.step[i].key.x >= 0 || domainDist2(P.gridP, x) <= P.halfSkin * P.halfSkin;
-  P.sPR[k] = make_float4(float(x.x), float(x.y), float(x.z), eligible ? r : -1.f);
-  P.sPRw[k] = make_float4(float(w.x), float(w.y), float(w.z), r);
-  P.sBoxR[k] = float(P.scale[i] * P.shapes[P.shape[i]].boxR);
-}
-__global__ void k_search_cells(Params P) {
-  LSD_GATE(P.devInt + rebuildFlagIdx(P.curBuf));
-  const Span g = gridSpan();
-  for (int i = g.tid; i < P.nP; i += g.nth) P.scell[i] = searchCellOf(P, i);
-}
-__global__ void k_gather_particles(Params P) {
-  LSD_GATE(P.devInt + rebuildFlagIdx(P.curBuf));
-  const Span g = gridSpan();
-  for (int k = g.tid; k < P.nP; k += g.nth) gatherParticle(P, k);
-}
-
-// ------------------------------------------------------------------------------------------
-// Candidate pairs
-// ------------------------------------------------------------------------------------------
-// Squared distance from x to the search grid's box (0 inside).
-__device__ __forceinline__ double searchBoxDist2(const SearchGrid& S, d3 x) {
-  const double ex = S.size.x * S.cell, ey = S.size.y * S.cell, ez = S.size.z * S.cell;
-  const double dx = fmax(0.0, fmax(S.mn.x - x.x, x.x - (S.mn.x + ex)));
-  const double dy = fmax(0.0, fmax(S.mn.y - x.y, x.y - (S.mn.y + ey)));
-  const double dz = fmax(0.0, fmax(S.mn.z - x.z, x.z - (S.mn.z + ez)));
-  return dx * dx + dy * dy + dz * dz;
-}
-
-// Visit every item of a search-grid table lying in cells that can hold a point within `reach`
-// of x.  Rows (y, z) are pruned by their distance to x; the x-run of cells of a row is
-// contiguous in the sorted order, so each row costs one range lookup.  The lookups of four rows
-// are issued before their items are visited, so four rows cost one round trip to memory (the
-// order of the visits is the same as row by row).
-// The x-run of search-grid row (cy, cz) within reach of x, given the row's remaining squared
-// reach rem >= 0: its first and one-past-last sorted positions.
-__device__ __forceinline__ int2 rowRun(const SearchGrid& S, const int* cellStart, d3 x, int cy, int cz, double rem) {
-  const double hw = sqrt(rem);
-  const int x0 = clampCell(floor((x.x - hw - S.mn.x) * S.invCell), S.size.x);
-  const int x1 = clampCell(floor((x.x + hw - S.mn.x) * S.invCell), S.size.x);
-  const int row = (cz * S.size.y + cy) * S.size.x;
-  return make_int2(cellStart[row + x0], cellStart[row + x1 + 1]);
-}
-// r2 minus the squared distance from x to row cy of a plane at squared distance dz2.
-__device__ __forceinline__ double rowRem(const SearchGrid& S, d3 x, int cy, double r2, double dz2) {
-  const double y0 = cy == 0 ? -1e300 : S.mn.y + cy * S.cell;
-  const double y1 = cy == S.size.y - 1 ? 1e300 : S.mn.y + (cy + 1) * S.cell;
-  const double dy = fmax(0.0, fmax(y0 - x.y, x.y - y1));
-  return r2 - dy * dy - dz2;
-}
-
-template <class F>
-__device__ __forceinline__ void visitNear(const SearchGrid& S, const int* cellStart, d3 x, double reach, F&& f) {
-  const i3 c = searchCell(S, x);
-  const int R = max(1, int(ceil(reach * S.invCell)));
-  const double r2 = reach * reach;
-  for (int cz = max(0, c.z - R); cz <= min(S.size.z - 1, c.z + R); ++cz) {
-    const double z0 = cz == 0 ? -1e300 : S.mn.z + cz * S.cell;
-    const double z1 = cz == S.size.z - 1 ? 1e300 : S.mn.z + (cz + 1) * S.cell;
-    const double dz = fmax(0.0, fmax(z0 - x.z, x.z - z1));
-    const double dz2 = dz * dz;
-    if (dz2 > r2) continue;
-    const int cyLo = max(0, c.y - R), cyHi = min(S.size.y - 1, c.y + R);
-    // rows in groups of four: a group's range lookups are issued together, then its items are
-    // visited (four named runs picked by selects: an indexed array would go to scratch memory, and
-    // unrolling the visits would copy f four times)
-    for (int g0 = cyLo; g0 <= cyHi; g0 += 4) {
-      auto load = [&](int cy) {
-        const double rem = cy <= cyHi ? rowRem(S, x, cy, r2, dz2) : -1.0;
-        return rem >= 0.0 ? rowRun(S, cellStart, x, cy, cz, rem) : make_int2(0, 0);
-      };
-      const int2 q0 = load(g0), q1 = load(g0 + 1), q2 = load(g0 + 2), q3 = load(g0 + 3);
-      for (int u = 0; u < 4; ++u) {
-        const int2 r = u == 0 ? q0 : u == 1 ? q1 : u == 2 ? q2 : q3;
-        for (int k = r.x; k < r.y; ++k) f(k);
-      }
-    }
-  }
-}
-
 __device__ __forceinline__ double triAt(const Params& P, const ShapeDev& S, double sc, d3 loc, d3 go, double invSp,
                                         bool& inside, double& cmax) {
   // trilinear SDF value at a local point (for pair-level culls), inside = within the grid box,
@@ -834,6 +744,177 @@ __device__ __forceinline__ double boxDist2(d3 loc, d3 o, double h, const ShapeDe
   return dx * dx + dy * dy + dz * dz;
 }
 
+// Which walls particle A can reach before the next rebuild: sphere vs grid box, then a Lipschitz bound on
+// the wall SDF at the centre.  Every point of a wall's grid box lies within boxR of the wall's origin: walls
+// far away (the other drums of an ensemble) are dropped on an FP32 sphere test (its margin covers the FP32
+// roundings of the centres, of boxR and of the test) before the shape record is read and the centre turned
+// into the wall's frame.
+// Up to kMaskWalls walls, one thread per particle tests them all (64 particles in a wavefront: six walls of a
+// box have few lanes' work); beyond that the lanes of a particle's search take a wall each.
+constexpr int kMaskWalls = 64;
+struct WallReach {
+  d3 xA;
+  double rs, rr;
+  float fx, fy, fz, fr, mA;
+  __device__ __forceinline__ WallReach(const Params& P, int A) {
+    xA = P.posDet[A];
+    rs = P.radius[A] + 2.0 * P.halfSkin;  // the wall and the particle each move < half the skin
+    rr = rs * (1.0 + 1e-9) + 1e-12;
+    fx = float(xA.x); fy = float(xA.y); fz = float(xA.z);
+    fr = float(rr);
+    mA = fmaxf(fmaxf(fabsf(fx), fabsf(fy)), fabsf(fz));
+  }
+  __device__ __forceinline__ bool reaches(const Params& P, int w) const {
+    const float4 sw = P.wSph[w];
+    const float dx = fx - sw.x, dy = fy - sw.y, dz = fz - sw.z;
+    const float ms = fmaxf(fmaxf(fabsf(sw.x), fabsf(sw.y)), fabsf(sw.z));
+    const float reach = (sw.w + fr) * (1.f + 1e-5f) + 1e-6f * (mA + ms) + 1e-30f;
+    if (dx * dx + dy * dy + dz * dz > reach * reach * (1.f + 1e-5f)) return false;
+    const d3 dw = xA - P.wpos[w];
+    const ShapeDev S = P.shapes[P.wshape[w]];
+    const d3 loc = rotInv(dw, P.wquat[w]);
+    const d3 o = mk3(S.ox, S.oy, S.oz);
+    if (boxDist2(loc, o, S.h, S) > rr * rr) return false;
+    bool inside;
+    double cmax;
+    const double phi = triAt(P, S, 1.0, loc, o, 1. / S.h, inside, cmax);
+    return !(inside && phi > S.lip * rs * (1.0 + 1e-6) + 1e-9 * S.h + 1e-12 * cmax);
+  }
+};
+
+// Search-grid cell of a particle's post-wrap centre: ghost images are searched through their
+// sources, and a particle that wrapped this step is outside the domain before the wrap (never a pp
+// partner).
+__device__ __forceinline__ int searchCellOf(const Params& P, int i) {
+  return lin3(searchCell(P.sg, P.pos[i]), P.sg.size);
+}
+
+// Gather particle (or ghost-image) data into the sorted order of the search-grid table so
+// that the candidate loops stream contiguous memory, and, where there are few walls, the walls each
+// particle can reach.
+__device__ void gatherParticle(const Params& P, int k) {
+  const int i = P.sorted[k];
+  const d3 x = P.posDet[i], w = P.pos[i];
+  const float r = float(P.radius[i]);
+  // a pp partner must be inside the domain when the pair is used; one that can get there before
+  // the next rebuild (within half the skin) stays a candidate
+  const bool eligible = P.step[i].key.x >= 0 || domainDist2(P.gridP, x) <= P.halfSkin * P.halfSkin;
+  P.sPR[k] = make_float4(float(x.x), float(x.y), float(x.z), eligible ? r : -1.f);
+  P.sPRw[k] = make_float4(float(w.x), float(w.y), float(w.z), r);
+  P.sBoxR[k] = float(P.scale[i] * P.shapes[P.shape[i]].boxR);
+  if (P.nW > 0 && P.nW <= kMaskWalls) {
+    const WallReach R(P, i);
+    unsigned long long m = 0;
+    for (int wl = 0; wl < P.nW; ++wl) m |= (unsigned long long)(R.reaches(P, wl) ? 1 : 0) << wl;
+    P.wallMask[k] = m;
+  }
+}
+__global__ void k_search_cells(Params P) {
+  LSD_GATE(P.devInt + rebuildFlagIdx(P.curBuf));
+  const Span g = gridSpan();
+  for (int i = g.tid; i < P.nP; i += g.nth) P.scell[i] = searchCellOf(P, i);
+}
+__global__ void k_gather_particles(Params P) {
+  LSD_GATE(P.devInt + rebuildFlagIdx(P.curBuf));
+  const Span g = gridSpan();
+  for (int k = g.tid; k < P.nP; k += g.nth) gatherParticle(P, k);
+}
+
+// ------------------------------------------------------------------------------------------
+// Candidate pairs
+// ------------------------------------------------------------------------------------------
+// Squared distance from x to the search grid's box (0 inside).
+__device__ __forceinline__ double searchBoxDist2(const SearchGrid& S, d3 x) {
+  const double ex = S.size.x * S.cell, ey = S.size.y * S.cell, ez = S.size.z * S.cell;
+  const double dx = fmax(0.0, fmax(S.mn.x - x.x, x.x - (S.mn.x + ex)));
+  const double dy = fmax(0.0, fmax(S.mn.y - x.y, x.y - (S.mn.y + ey)));
+  const double dz = fmax(0.0, fmax(S.mn.z - x.z, x.z - (S.mn.z + ez)));
+  return dx * dx + dy * dy + dz * dz;
+}
+
+__device__ __forceinline__ int clampCellF(float v, int n) { return int(fminf(fmaxf(v, 0.f), float(n - 1))); }
+
+// 32 lanes that search one master's neighbourhood together: its lane l of the group, the group's first lane
+// in the wavefront, and kFindQueue ints of LDS of its own.
+constexpr int kFindLanes = 32, kFindQueue = 256;
+struct FindGroup {
+  int l, first;
+  int* q;
+  __device__ __forceinline__ unsigned int ballot(bool v) const { return (unsigned int)(__ballot(v) >> first); }
+  __device__ __forceinline__ unsigned int below() const { return (1u << l) - 1u; }  // the group's lanes before this one
+};
+__device__ __forceinline__ FindGroup findGroup(int* queues) {  // queues: kFindQueue ints per group of the block
+  const int lane = threadIdx.x & 63;
+  return FindGroup{lane & (kFindLanes - 1), lane & ~(kFindLanes - 1), queues + (threadIdx.x / kFindLanes) * kFindQueue};
+}
+
+// Visit every item of a search-grid table lying in cells that can hold a point within `reach` of x, 32 at a
+// time, by the whole group (`in` tells which lanes hold an item, sorted position k).  Rows
+// (y, z) are pruned by their distance to x; the x-run of cells of a row is contiguous in the sorted order,
+// so each row costs one range lookup.  Lanes = rows for the lookups (one round trip for 32 rows), then lanes =
+// items, listed in LDS; items come row by row, each row in sorted order.
+// K rounds of items are read together (load(k)), then taken in order (use(item, k, in)).
+template <int K, class Load, class Use>
+__device__ __forceinline__ void visitNear(const SearchGrid& S, const int* cellStart, d3 x, double reach,
+                                          const FindGroup& G, Load&& load, Use&& use) {
+  // (FP32 relative to the grid's corner: the reach is widened by far more than its rounding, and an item
+  // visited in vain fails its own test)
+  const float cell = float(S.cell), inv = float(S.invCell);
+  const float rx = float(x.x - S.mn.x), ry = float(x.y - S.mn.y), rz = float(x.z - S.mn.z);
+  const float far = fmaxf(fmaxf(fabsf(rx), fabsf(ry)), fabsf(rz));
+  const float rr = float(reach) * (1.f + 1e-6f) + 1e-5f * cell + 1e-6f * far, r2 = rr * rr;
+  const int cyLo = clampCellF(floorf((ry - rr) * inv), S.size.y), cyHi = clampCellF(floorf((ry + rr) * inv), S.size.y);
+  const int czLo = clampCellF(floorf((rz - rr) * inv), S.size.z), czHi = clampCellF(floorf((rz + rr) * inv), S.size.z);
+  const int ny = cyHi - cyLo + 1, nRows = ny * (czHi - czLo + 1);
+  for (int r0 = 0; r0 < nRows; r0 += kFindLanes) {
+    const int r = r0 + G.l;
+    int2 run = make_int2(0, 0);
+    if (r < nRows) {
+      const int zi = r / ny, cz = czLo + zi, cy = cyLo + (r - zi * ny);
+      // (a body beyond the grid lies in a cell of its boundary, which has no end there)
+      const float y0 = cy == 0 ? -3e38f : float(cy) * cell, y1 = cy == S.size.y - 1 ? 3e38f : float(cy + 1) * cell;
+      const float z0 = cz == 0 ? -3e38f : float(cz) * cell, z1 = cz == S.size.z - 1 ? 3e38f : float(cz + 1) * cell;
+      const float dy = fmaxf(0.f, fmaxf(y0 - ry, ry - y1)), dz = fmaxf(0.f, fmaxf(z0 - rz, rz - z1));
+      const float rem = r2 - dy * dy - dz * dz;
+      if (rem >= 0.f) {
+        const float hw = sqrtf(rem);
+        const int row = (cz * S.size.y + cy) * S.size.x;
+        run = make_int2(cellStart[row + clampCellF(floorf((rx - hw) * inv), S.size.x)],
+                        cellStart[row + clampCellF(floorf((rx + hw) * inv), S.size.x) + 1]);
+      }
+    }
+    const int len = max(0, run.y - run.x);
+    int incl = len;
+#pragma unroll
+    for (int o = 1; o < kFindLanes; o <<= 1) {
+      const int t = __shfl_up(incl, o, kFindLanes);
+      if (G.l >= o) incl += t;
+    }
+    const int total = __shfl(incl, kFindLanes - 1, kFindLanes), before = incl - len;
+    for (int w0 = 0; w0 < total; w0 += kFindQueue) {
+      for (int u = max(0, w0 - before); u < min(len, w0 + kFindQueue - before); ++u) G.q[before + u - w0] = run.x + u;
+      __builtin_amdgcn_wave_barrier();
+      const int n = min(kFindQueue, total - w0);
+      for (int i0 = G.l; i0 - G.l < n; i0 += K * kFindLanes) {
+        int k[K];
+        decltype(load(0)) item[K];
+#pragma unroll
+        for (int u = 0; u < K; ++u) {
+          k[u] = 0;
+          if (i0 + u * kFindLanes < n) {
+            k[u] = G.q[i0 + u * kFindLanes];
+            item[u] = load(k[u]);
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < K; ++u)
+          if (i0 - G.l + u * kFindLanes < n) use(item[u], k[u], i0 + u * kFindLanes < n);
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+  }
+}
+
 // FP32 sphere-overlap test with a margin covering the FP32 rounding of both centres and radii:
 // accepts every pair whose FP64 bounding spheres overlap (a superset is harmless, every pair is
 // settled by the exact node tests).
@@ -845,168 +926,256 @@ __device__ __forceinline__ bool spheresMayOverlap(float4 a, float4 b, float rb) 
   return dx * dx + dy * dy + dz * dz <= rr * rr * (1.f + 1e-6f);
 }
 
-// Candidate pairs of the master in sorted position t (A = sorted[t]), in a fixed order:
-// particle partners, walls, then ghost images set by set.  DIRECT writes them to the pair list
-// at `out`; otherwise the first kPairSlab go to the master's slab column and all are counted.
-constexpr int kPairSlab = kPairSlabHost;
-template <bool DIRECT>
-__device__ __forceinline__ int pairsOf(const Params& P, int t, int A, long long out) {
-  int cnt = 0;
-  auto emit = [&](uint32_t type, int partner) {
-    const uint32_t info = (type << 28) | uint32_t(partner);
-    if (DIRECT) {
-      if (out < P.pairCap) {
-        P.pairA[out] = A;
-        P.pairInfo[out] = info;
-      }
-      ++out;
-    } else if (cnt < kPairSlab) {
-      P.pairSlab[(long long)cnt * P.nP + t] = info;
-    }
-    ++cnt;
-  };
-  const float4 a = P.sPR[t];
-  const float skin = float(2.0 * P.halfSkin);
-  // particle-particle: B > A, B inside the domain, bounding spheres within the skin
-  {
-    const float ma = fmaxf(fmaxf(fabsf(a.x), fabsf(a.y)), fabsf(a.z));
-    const double reach = (double(a.w) + P.rMax + 2.0 * P.halfSkin) * (1.0 + 2e-6) + 1e-6 * double(ma) + 1e-12;
-    visitNear(P.sg, P.cellStart, mk3(a.x, a.y, a.z), reach, [&](int k) {
-      const float4 b = P.sPR[k];
-      if (b.w < 0.f || !spheresMayOverlap(a, b, b.w + skin)) return;
-      const int B = P.sorted[k];
-      if (B <= A) return;
-      emit(PT_PP, B);
-    });
-  }
-  // walls: sphere vs grid box, then a Lipschitz bound on the wall SDF at the centre
-  if (P.nW > 0) {
-    const double rA = P.radius[A];
-    const d3 xA = P.posDet[A];
-    const double rs = rA + 2.0 * P.halfSkin;  // the wall and the particle each move < half the skin
-    const double rr = rs * (1.0 + 1e-9) + 1e-12;
-    // every point of a wall's grid box lies within boxR of the wall's origin: walls far away (the
-    // other drums of an ensemble) are dropped on an FP32 sphere test (its margin covers the FP32
-    // roundings of the centres, of boxR and of the test) before the shape record is read and the
-    // centre turned into the wall's frame.  The searching lanes of the wavefront load the spheres of
-    // as many walls at once, one each, and pass them round: one memory round trip per that many
-    // walls instead of one per wall.
-    const float fx = float(xA.x), fy = float(xA.y), fz = float(xA.z);
-    const float fr = float(rr);
-    const float mA = fmaxf(fmaxf(fabsf(fx), fabsf(fy)), fabsf(fz));
-    const unsigned long long act = __ballot(1);
-    const int nAct = __popcll(act);
-    const int myRank = __popcll(act & laneLtMask());
-    for (int w0 = 0; w0 < P.nW; w0 += nAct) {
-      const int wl = w0 + myRank;
-      const float4 mine = wl < P.nW ? P.wSph[wl] : make_float4(0.f, 0.f, 0.f, 0.f);
-      const int cnt = min(nAct, P.nW - w0);
-      unsigned long long rest = act;
-      for (int u = 0; u < cnt; ++u) {  // a wall's key is checked each step when the pair is used
-        const int src = __ffsll((long long)rest) - 1;  // the lane holding wall w0 + u
-        rest &= rest - 1;
-        const float4 sw = make_float4(__shfl(mine.x, src, 64), __shfl(mine.y, src, 64), __shfl(mine.z, src, 64),
-                                      __shfl(mine.w, src, 64));
-        const int w = w0 + u;
-        const float dx = fx - sw.x, dy = fy - sw.y, dz = fz - sw.z;
-        const float ms = fmaxf(fmaxf(fabsf(sw.x), fabsf(sw.y)), fabsf(sw.z));
-        const float reach = (sw.w + fr) * (1.f + 1e-5f) + 1e-6f * (mA + ms) + 1e-30f;
-        if (dx * dx + dy * dy + dz * dz > reach * reach * (1.f + 1e-5f)) continue;
-        const d3 dw = xA - P.wpos[w];
-        const ShapeDev S = P.shapes[P.wshape[w]];
-        const d3 loc = rotInv(dw, P.wquat[w]);
-        const d3 o = mk3(S.ox, S.oy, S.oz);
-        if (boxDist2(loc, o, S.h, S) > rr * rr) continue;
-        bool inside;
-        double cmax;
-        const double phi = triAt(P, S, 1.0, loc, o, 1. / S.h, inside, cmax);
-        if (inside && phi > S.lip * rs * (1.0 + 1e-6) + 1e-9 * S.h + 1e-12 * cmax) continue;
-        emit(PT_PW, w);
-      }
-    }
-  }
-  // periodic ghost images: any node inside the image's grid box is tested, so the reach is
-  // the image's grid-box radius.  Images are found through their sources in the particle grid:
-  // an image shifted by the set's offset lies near x_A - offset; images left at the source's own
-  // position (a source outside the domain) are searched around x_A only when such images exist.
-  if (P.periodicX || P.periodicY || P.periodicSector) {
-    const float4 g = P.sPRw[t];  // post-wrap centre (images are built from it)
-    const float mg = fmaxf(fmaxf(fabsf(g.x), fabsf(g.y)), fabsf(g.z));
-    const double reach = (double(g.w) + P.boxRMax + 2.0 * P.halfSkin) * (1.0 + 2e-6) + 1e-6 * double(mg) + 1e-12;
-    const GridGeom& G = P.gridP;
-    const double hs = P.halfSkin;
-    const float lx = float(G.mx.x - G.mn.x), ly = float(G.mx.y - G.mn.y);
-    const bool anyUnshifted = P.devInt[ghostCountIdx(P.curBuf)] > 0;
-    const bool sector = P.periodicSector != 0;
-    for (int s = 0; s < 3; ++s) {
-      const bool on = sector || (s == 0 && P.periodicX) || (s == 1 && P.periodicY) ||
-                      (s == 2 && P.periodicX && P.periodicY);
-      if (!on) continue;
-      const float offx = s != 1 ? lx : 0.f, offy = s != 0 ? ly : 0.f;
-      const int col = sector ? imageColumn<true>(s) : imageColumn<false>(s);
-      // the image of a source at b (shifted by the period, or turned about the corner's z axis)
-      auto image = [&](float4 b) {
-        if (!sector) return make_float4(b.x + offx, b.y + offy, b.z, 0.f);
-        const d3 r = G.mn + secTurn(P, s, mk3(b.x, b.y, b.z) - G.mn);
-        return make_float4(float(r.x), float(r.y), float(r.z), 0.f);
-      };
-      for (int pass = 0; pass < 2; ++pass) {
-        const bool shifted = pass == 0;
-        if (!shifted && !anyUnshifted) break;
-        // sources whose image lies near x_A lie near the inverse image of x_A (a turn the other way)
-        const int inv = 2 - s;
-        const d3 c = !shifted ? mk3(g.x, g.y, g.z)
-                     : (sector ? G.mn + secTurn(P, inv, mk3(g.x, g.y, g.z) - G.mn)
-                               : mk3(double(g.x) - double(offx), double(g.y) - double(offy), double(g.z)));
-        if (searchBoxDist2(P.sg, c) > reach * reach) continue;
-        visitNear(P.sg, P.cellStart, c, reach, [&](int k) {
-          const float4 b = P.sPRw[k];
-          const float rb = P.sBoxR[k] + skin;
-          const float4 im = shifted ? image(b) : b;
-          if (!spheresMayOverlap(g, im, rb)) return;
-          const int j = P.sorted[k];
-          const d3 pj = P.pos[j];
-          if (shifted) {
-            if (!potInColumn(G, pj, col, hs)) return;
-          } else {
-            if (!potOutOfDomain(P, pj, hs) || !potOutColumn(G, pj, col, hs)) return;
-            // one pair per (A, image): the shifted pass already took it
-            if (potInColumn(G, pj, col, hs) && spheresMayOverlap(g, image(b), rb)) return;
-          }
-          emit(PT_GX + s, j);
-        });
-      }
-    }
-  }
-  return cnt;
+// Rank of a candidate pair among its partner's reactions as counted so far (sorted later), where the partner
+// takes the reaction (particle-particle, ghosts with j != A); else -1.
+__device__ __forceinline__ int reactionRank(const Params& P, int A, uint32_t info) {
+  const uint32_t type = info >> 28;
+  const int partner = int(info & kPartnerMask);
+  return type == PT_PP || (type >= PT_GX && partner != A) ? atomicAdd(&P.rcCount[partner], 1) : -1;
 }
 
-// Broad phase, one thread per master in spatial order: count and keep the first candidates.
-__device__ void pairsFind(const Params& P, Span g) {
-  for (int t = g.tid; t < P.nP; t += g.nth) {
-    const int A = P.sorted[t];
-    P.pairCount[A] = pairsOf<false>(P, t, A, 0);
+// Candidate pairs of the master in sorted position t (A = sorted[t]) come in a fixed order, particle
+// partners, walls, then ghost images set by set, found by a group of 32 lanes.  DIRECT writes them to the
+// pair list from `out` on; otherwise the first kPairSlab go to the master's part of the slab and all are counted.
+constexpr int kPairSlab = kPairSlabHost;
+template <bool DIRECT>
+struct PairSink {
+  const Params& P;
+  int t, A;
+  long long out;
+  int cnt;
+  // (by the whole group: the lanes with a hit are numbered in lane order)
+  __device__ __forceinline__ void put(const FindGroup& G, bool hit, uint32_t type, int partner) {
+    const unsigned int m = G.ballot(hit);
+    if (hit) {
+      const uint32_t info = (type << 28) | uint32_t(partner);
+      const int k = cnt + __popc(m & G.below());
+      if (DIRECT) {
+        if (out + k < P.pairCap) {
+          P.pairA[out + k] = A;
+          P.pairInfo[out + k] = info;
+          P.rcRank[out + k] = reactionRank(P, A, info);
+        }
+      } else if (k < kPairSlab) {
+        P.pairSlab[(long long)t * kPairSlab + k] = info;
+      }
+    }
+    cnt += __popc(m);
+  }
+};
+
+// Particle partners (B > A, B inside the domain, bounding spheres within the skin), then walls (each wall's
+// key is checked each step when the pair is used).
+template <bool DIRECT>
+__device__ __forceinline__ void nearPairs(const Params& P, PairSink<DIRECT>& sink, const FindGroup& G) {
+  const int A = sink.A;
+  const float4 a = P.sPR[sink.t];
+  const unsigned long long walls = P.nW > 0 && P.nW <= kMaskWalls ? P.wallMask[sink.t] : 0ull;
+  const float skin = float(2.0 * P.halfSkin);
+  const float ma = fmaxf(fmaxf(fabsf(a.x), fabsf(a.y)), fabsf(a.z));
+  const double reach = (double(a.w) + P.rMax + 2.0 * P.halfSkin) * (1.0 + 2e-6) + 1e-6 * double(ma) + 1e-12;
+  struct Item {
+    float4 b;
+    int id;
+  };
+  visitNear<4>(P.sg, P.cellStart, mk3(a.x, a.y, a.z), reach, G, [&](int k) { return Item{P.sPR[k], P.sorted[k]}; },
+               [&](const Item& it, int, bool in) {
+                 sink.put(G, in && it.b.w >= 0.f && it.id > A && spheresMayOverlap(a, it.b, it.b.w + skin), PT_PP,
+                          it.id);
+               });
+  if (P.nW > kMaskWalls) {
+    const WallReach R(P, A);
+    for (int w0 = 0; w0 < P.nW; w0 += kFindLanes) {
+      const int w = w0 + G.l;
+      sink.put(G, w < P.nW && R.reaches(P, w), PT_PW, w);
+    }
+  } else if (P.nW > 0) {
+    for (int w0 = 0; w0 < P.nW; w0 += kFindLanes) sink.put(G, (walls >> (w0 + G.l)) & 1ull, PT_PW, w0 + G.l);
   }
 }
-__global__ void k_pairs_find(Params P) {
-  LSD_GATE(P.devInt + rebuildFlagIdx(P.curBuf));
-  pairsFind(P, gridSpan());
+
+// Periodic ghost images of a master: any node inside the image's grid box is tested, so the reach is
+// the image's grid-box radius.  Images are found through their sources in the particle grid:
+// an image shifted by the set's offset lies near x_A - offset; images left at the source's own
+// position (a source outside the domain) are searched around x_A only when such images exist.
+struct ImageSearch {
+  const Params& P;
+  float4 g;      // post-wrap centre (images are built from it)
+  double reach;
+  float lx, ly;
+  bool sector, anyUnshifted;
+  __device__ __forceinline__ ImageSearch(const Params& P_, int t) : P(P_) {
+    g = P.sPRw[t];
+    const float mg = fmaxf(fmaxf(fabsf(g.x), fabsf(g.y)), fabsf(g.z));
+    reach = (double(g.w) + P.boxRMax + 2.0 * P.halfSkin) * (1.0 + 2e-6) + 1e-6 * double(mg) + 1e-12;
+    lx = float(P.gridP.mx.x - P.gridP.mn.x);
+    ly = float(P.gridP.mx.y - P.gridP.mn.y);
+    sector = P.periodicSector != 0;
+    anyUnshifted = P.devInt[ghostCountIdx(P.curBuf)] > 0;
+  }
+  __device__ __forceinline__ bool on(int s) const {
+    return sector || (s == 0 && P.periodicX) || (s == 1 && P.periodicY) || (s == 2 && P.periodicX && P.periodicY);
+  }
+  // where the sources of set s's images near the master lie (a turn the other way for sector images);
+  // shifted = false: of its images at their source's own position
+  __device__ __forceinline__ d3 centre(int s, bool shifted) const {
+    const d3 x = mk3(g.x, g.y, g.z);
+    if (!shifted) return x;
+    if (sector) return P.gridP.mn + secTurn(P, 2 - s, x - P.gridP.mn);
+    return mk3(x.x - double(s != 1 ? lx : 0.f), x.y - double(s != 0 ? ly : 0.f), x.z);
+  }
+  // the image of a source at b (shifted by the period, or turned about the corner's z axis)
+  __device__ __forceinline__ float4 image(int s, float4 b) const {
+    if (!sector) return make_float4(b.x + (s != 1 ? lx : 0.f), b.y + (s != 0 ? ly : 0.f), b.z, 0.f);
+    const d3 r = P.gridP.mn + secTurn(P, s, mk3(b.x, b.y, b.z) - P.gridP.mn);
+    return make_float4(float(r.x), float(r.y), float(r.z), 0.f);
+  }
+  __device__ __forceinline__ bool reaches(int s, bool shifted) const {
+    return on(s) && !(searchBoxDist2(P.sg, centre(s, shifted)) > reach * reach);
+  }
+};
+// Whether a master has any images to search for (most lie too far from the periodic faces).
+__device__ __forceinline__ bool mayMeetImages(const Params& P, int t) {
+  const ImageSearch I(P, t);
+  bool any = false;
+  for (int s = 0; s < 3; ++s) any = any || I.reaches(s, true) || (I.anyUnshifted && I.reaches(s, false));
+  return any;
 }
-// Pair list in master order: copy the slab, or search again for masters with more candidates.
-__device__ void pairsEmit(const Params& P, Span g) {
-  for (int t = g.tid; t < P.nP; t += g.nth) {
-    const int A = P.sorted[t];
-    const int n = P.pairCount[A];
-    const long long out = P.pairStart[A];
-    if (n > kPairSlab) {
-      pairsOf<true>(P, t, A, out);
-      continue;
+template <bool DIRECT>
+__device__ __forceinline__ void imagePairs(const Params& P, PairSink<DIRECT>& sink, const FindGroup& G) {
+  const ImageSearch I(P, sink.t);
+  const GridGeom& grid = P.gridP;
+  const double hs = P.halfSkin;
+  const float skin = float(2.0 * P.halfSkin);
+  for (int s = 0; s < 3; ++s) {
+    const int col = I.sector ? imageColumn<true>(s) : imageColumn<false>(s);
+    for (int pass = 0; pass < 2; ++pass) {
+      const bool shifted = pass == 0;
+      if (!shifted && !I.anyUnshifted) break;
+      if (!I.reaches(s, shifted)) continue;
+      struct Item {
+        float4 b;
+        float box;
+      };
+      visitNear<1>(P.sg, P.cellStart, I.centre(s, shifted), I.reach, G,
+                   [&](int k) { return Item{P.sPRw[k], P.sBoxR[k]}; },
+                   [&](const Item& it, int k, bool in) {
+                     bool hit = false;
+                     int j = -1;
+                     const float rb = it.box + skin;
+                     if (in && spheresMayOverlap(I.g, shifted ? I.image(s, it.b) : it.b, rb)) {
+                       j = P.sorted[k];
+                       const d3 pj = P.pos[j];
+                       if (shifted) {
+                         hit = potInColumn(grid, pj, col, hs);
+                       } else {
+                         // (one pair per master and image: the shifted pass already took it)
+                         hit = potOutOfDomain(P, pj, hs) && potOutColumn(grid, pj, col, hs) &&
+                               !(potInColumn(grid, pj, col, hs) && spheresMayOverlap(I.g, I.image(s, it.b), rb));
+                       }
+                     }
+                     sink.put(G, hit, PT_GX + s, j);
+                   });
     }
-    for (int k = 0; k < n; ++k) {
-      if (out + k >= P.pairCap) break;
-      P.pairA[out + k] = A;
-      P.pairInfo[out + k] = P.pairSlab[(long long)k * P.nP + t];
+  }
+}
+
+// The masters of a block's turn: its share of the sorted order, 32 consecutive ones at a time from all over
+// it (consecutive ones meet the same cells; sizes may be sorted in space, so no block gets one end).
+struct MasterShare {
+  int chunk;  // masters of a full turn's part, 32 per block and turn
+  __device__ __forceinline__ explicit MasterShare(int nP) {
+    const int turns = (nP + int(gridDim.x) * 32 - 1) / (int(gridDim.x) * 32);
+    chunk = turns * 32;
+  }
+  __device__ __forceinline__ int at(int i) const {  // sorted position of the block's i-th master (may be >= nP)
+    return ((i >> 5) * int(gridDim.x) + int(blockIdx.x)) * 32 + (i & 31);
+  }
+};
+
+// Broad phase, 32 lanes per master: count its candidates and keep the first.  Bound by each master's chain of
+// round trips (its own data, the row lookups, four rounds of 32 items at a time) and by how unevenly masters
+// meet neighbours.  Images are searched in a turn of their own for the masters that may have any.  (One
+// thread per master, an item a round trip: 398 us of a rebuild's 522 for 4,000 bodies in a quarter sector, 340
+// of 507 for 20,000 of scattered sizes, 597 of 1,028 for 200,000; now 42 of 152, 126 of 276 and 325 of 700.
+// Tried and left out: a largest radius per search cell to shorten the runs, with cells of 1, 0.5 and 0.35
+// of this edge: 348 us of search at 200,000 for 440 then, 139 for 148 at 20,000, slower below; finer
+// cells slower everywhere.)
+// queues: kFindQueue ints of LDS per group of the block; many: an int per thread, and one.
+__device__ void pairsFind(const Params& P, int* queues, int* many) {
+  const FindGroup G = findGroup(queues);
+  const MasterShare share(P.nP);
+  const int group = int(threadIdx.x) / kFindLanes, groups = int(blockDim.x) / kFindLanes;
+  for (int i = group; i < share.chunk; i += groups) {
+    const int t = share.at(i);
+    if (t >= P.nP) continue;
+    PairSink<false> sink{P, t, P.sorted[t], 0, 0};
+    nearPairs(P, sink, G);
+    if (G.l == 0) P.pairCount[sink.A] = sink.cnt;
+  }
+  if (!(P.periodicX || P.periodicY || P.periodicSector)) return;
+  int* const nMany = many + blockDim.x;
+  for (int i0 = 0; i0 < share.chunk; i0 += int(blockDim.x)) {
+    __threadfence_block();
+    __syncthreads();
+    if (threadIdx.x == 0) *nMany = 0;
+    __syncthreads();
+    const int i = i0 + int(threadIdx.x), ti = share.at(i);
+    if (i < share.chunk && ti < P.nP && mayMeetImages(P, ti)) many[atomicAdd(nMany, 1)] = ti;
+    __syncthreads();
+    for (int m = group; m < *nMany; m += groups) {
+      const int t = many[m], A = P.sorted[t];
+      PairSink<false> sink{P, t, A, 0, P.pairCount[A]};
+      imagePairs(P, sink, G);
+      if (G.l == 0) P.pairCount[A] = sink.cnt;
     }
+  }
+}
+constexpr int kFindThreads = 256;  // block of the separate search launches
+__global__ __launch_bounds__(kFindThreads) void k_pairs_find(Params P) {
+  LSD_GATE(P.devInt + rebuildFlagIdx(P.curBuf));
+  __shared__ int queues[kFindThreads / kFindLanes * kFindQueue], many[kFindThreads + 1];
+  pairsFind(P, queues, many);
+}
+// Pair list in master order: eight lanes per master copy its part of the slab, eight candidates a turn (a thread
+// per master took as many turns as a master has candidates: 24 us of a rebuild for 4,000 bodies in a quarter
+// sector, now 7); the masters of the block's turn with more candidates than the slab holds are listed in
+// LDS and searched again, 32 lanes each.
+__device__ void pairsEmit(const Params& P, int* queues, int* many) {
+  constexpr int kLanes = 8;
+  const FindGroup G = findGroup(queues);
+  int* const nMany = many + blockDim.x;
+  const int l = int(threadIdx.x) & (kLanes - 1), perBlock = int(blockDim.x) / kLanes;
+  for (int t0 = int(blockIdx.x) * perBlock; t0 < P.nP; t0 += int(gridDim.x) * perBlock) {
+    const int t = t0 + int(threadIdx.x) / kLanes;
+    if (threadIdx.x == 0) *nMany = 0;
+    __syncthreads();
+    if (t < P.nP) {
+      const int A = P.sorted[t];
+      const int n = P.pairCount[A];
+      const long long out = P.pairStart[A];
+      if (n <= kPairSlab) {
+        for (int k = l; k < n; k += kLanes) {
+          const uint32_t info = P.pairSlab[(long long)t * kPairSlab + k];
+          const int rank = reactionRank(P, A, info);
+          if (out + k < P.pairCap) {
+            P.pairA[out + k] = A;
+            P.pairInfo[out + k] = info;
+            P.rcRank[out + k] = rank;
+          }
+        }
+      } else if (l == 0) {
+        many[atomicAdd(nMany, 1)] = t;
+      }
+    }
+    __syncthreads();
+    for (int m = int(threadIdx.x) / kFindLanes; m < *nMany; m += int(blockDim.x) / kFindLanes) {
+      const int A = P.sorted[many[m]];
+      PairSink<true> sink{P, many[m], A, P.pairStart[A], 0};
+      nearPairs(P, sink, G);
+      if (P.periodicX || P.periodicY || P.periodicSector) imagePairs(P, sink, G);
+    }
+    __syncthreads();
   }
 }
 // Keep the pair list being replaced (per-master starts, entries, certificates) for the
@@ -1071,28 +1240,17 @@ __device__ __forceinline__ bool pairOverflow(const Params& P) {
   }
   return true;
 }
-__global__ void k_pairs_emit(Params P) {
+__global__ __launch_bounds__(kFindThreads) void k_pairs_emit(Params P) {
   LSD_GATE(P.devInt + rebuildFlagIdx(P.curBuf));
   if (pairOverflow(P)) return;
-  pairsEmit(P, gridSpan());
+  __shared__ int queues[kFindThreads / kFindLanes * kFindQueue], many[kFindThreads + 1];
+  pairsEmit(P, queues, many);
 }
 __global__ void k_mark_build(Params P) {
   LSD_GATE(P.devInt + rebuildFlagIdx(P.curBuf));
   markBuild(P, gridSpan());
 }
 
-// Pairs whose partner particle receives the reaction (particle-particle, ghosts with j != A).
-__device__ void rcCountPairs(const Params& P, Span g) {
-  const int n = min(P.pairStart[P.nP], (int)P.pairCap);
-  for (int p = g.tid; p < n; p += g.nth) {
-    const uint32_t info = P.pairInfo[p];
-    const uint32_t type = info >> 28;
-    const int partner = int(info & kPartnerMask);
-    int r = -1;
-    if (type == PT_PP || (type >= PT_GX && partner != P.pairA[p])) r = atomicAdd(&P.rcCount[partner], 1);
-    P.rcRank[p] = r;
-  }
-}
 __device__ void rcScatterPairs(const Params& P, Span g) {
   const int n = min(P.pairStart[P.nP], (int)P.pairCap);
   for (int p = g.tid; p < n; p += g.nth) {
@@ -1102,10 +1260,6 @@ __device__ void rcScatterPairs(const Params& P, Span g) {
     const int d = P.rcStart[partner] + r;
     if (d < P.pairCap) P.rcTmp[d] = p;
   }
-}
-__global__ void k_rc_count(Params P) {
-  LSD_GATE(P.devInt + rebuildFlagIdx(P.curBuf));
-  rcCountPairs(P, gridSpan());
 }
 __global__ void k_rc_scatter(Params P) {
   LSD_GATE(P.devInt + rebuildFlagIdx(P.curBuf));
@@ -1440,7 +1594,7 @@ __device__ __forceinline__ EvalRecords evalRecords(const Params& P) {
   for (int g = 0; g < 8; ++g) {
     e.pre[g] = sum;
     e.base[g] = groupFirstTile(nTiles, g) * kCheckTile;
-    sum += P.evalCount[g * kBarrierLine];
+    sum += evalCount(P)[g * kBarrierLine];
   }
   e.n = sum;
   return e;
@@ -1588,7 +1742,7 @@ __global__ __launch_bounds__(256) void k_pair_check(Params P, int full) {
       }
     }
     __syncthreads();
-    if (threadIdx.x == 0) sBase = sCount ? region + atomicAdd(&P.evalCount[xcd * kBarrierLine], sCount) : 0;
+    if (threadIdx.x == 0) sBase = sCount ? region + atomicAdd(&evalCount(P)[xcd * kBarrierLine], sCount) : 0;
     __syncthreads();
     for (int k = threadIdx.x; k < sCount; k += 256) {
       const int p = sList[k], a = sBase + k;
@@ -2854,6 +3008,11 @@ __device__ void stepEnd(const Params& P) {
 // The whole broad phase in one launch (rebuild steps only; every block returns at once
 // otherwise).  Phases are separated by grid barriers; every block runs every phase, so all blocks
 // reach every barrier.  The host sizes the grid so that all its blocks are resident together.
+// A rebuild is a chain of short phases: a barrier costs 2.3 to 2.9 us, a phase at least its own few dependent
+// reads, so phases share barriers where neither reads what the other writes (14 barriers, once 19), and the sorts
+// of long buckets are passed over when there are none.  Whole rebuild, before -> now: 27 bodies 105 -> 84 us,
+// 1,000 163 -> 103, 4,000 in a quarter sector 522 -> 152, 20,000 of scattered sizes 507 -> 276, 27,000 packed
+// 223 -> 200, 200,000 of scattered sizes 1,028 -> 700.
 // ------------------------------------------------------------------------------------------
 // Blocks of the single-launch broad phase: large, so that few blocks meet at each barrier (the
 // cost of a barrier grows with the number of blocks) while many threads work between them.
@@ -2915,36 +3074,45 @@ __global__ __launch_bounds__(kBroadThreads) void k_broad_phase(Params P) {
   LSD_HALT(P);
   if (P.devInt[rebuildFlagIdx(P.curBuf)] == 0) return;  // written by the drift kernel before this launch: grid-uniform
   __shared__ int lds[kScanLds];
+  __shared__ int queues[kBroadThreads / kFindLanes * kFindQueue], many[kBroadThreads + 1];
   GridBarrier grid{P, int(gridDim.x), 0};
   const Span g = gridSpan();
   const int wave = g.tid >> 6, nWaves = g.nth >> 6;
   const int ncell = P.sg.ncell;
+  int* const bigCells = P.devInt + kBigCellsIdx;  // any cell (any reaction list) of more than kSmallBucket items:
+  int* const bigRc = P.devInt + kBigRcIdx;        // without one, the phase that sorts those is left out
   // counting sort of the particles by search cell
   for (int i = g.tid; i < ncell; i += g.nth) P.cellCount[i] = 0;
   for (int i = g.tid; i < P.nP; i += g.nth) {
     P.rcCount[i] = 0;
     P.scell[i] = searchCellOf(P, i);
   }
-  if (g.tid == 0) P.devInt[2] = 0;  // large-bucket list
+  if (g.tid == 0) {
+    P.devInt[2] = 0;  // large-bucket list
+    *bigCells = 0;
+    *bigRc = 0;
+  }
   if (grid.sync()) return;
   bucketCount(P.scell, P.nP, P.cellCount, P.rank, g);
   if (grid.sync()) return;
   scanReduceTiles(P.cellCount, ncell, P.scanTiles, lds);
   if (grid.sync()) return;
-  scanApplyTiles(P.cellCount, ncell, P.scanTiles, P.cellStart, lds);
+  scanApplyTiles(P.cellCount, ncell, P.scanTiles, P.cellStart, lds, bigCells);
   if (grid.sync()) return;
   bucketScatter(P.scell, P.nP, P.cellStart, P.rank, P.sortTmp, g);
   if (grid.sync()) return;
   bucketSortSmall(P.cellStart, ncell, P.sortTmp, P.sorted, nullptr, P.sortBig, P.devInt + 2, g, P.nP);
   if (grid.sync()) return;
-  bucketSortBig(P.cellStart, P.sortTmp, P.sorted, nullptr, P.sortBig, P.devInt + 2, wave, nWaves, ncell, P.nP);
-  if (grid.sync()) return;
+  if (*bigCells) {
+    bucketSortBig(P.cellStart, P.sortTmp, P.sorted, nullptr, P.sortBig, P.devInt + 2, wave, nWaves, ncell, P.nP);
+    if (grid.sync()) return;
+  }
   // particle data in sorted order; candidate pairs per master, prefix, pair list
   for (int k = g.tid; k < P.nP; k += g.nth) gatherParticle(P, k);
   backupPairs(P, g);
   if (g.tid == 0) P.devInt[2] = 0;  // large-bucket list of the reaction sort
   if (grid.sync()) return;
-  pairsFind(P, g);
+  pairsFind(P, queues, many);
   if (grid.sync()) return;
   scanReduceTiles(P.pairCount, P.nP, P.scanTiles, lds);
   if (grid.sync()) return;
@@ -2952,23 +3120,20 @@ __global__ __launch_bounds__(kBroadThreads) void k_broad_phase(Params P) {
   if (grid.sync()) return;
   // every block reads the same total after the barrier: all leave together when it does not fit
   if (pairOverflow(P)) return;
-  pairsEmit(P, g);
+  pairsEmit(P, queues, many);
   if (grid.sync()) return;
   inheritCerts(P, g);  // reads the motion records before they restart
-  if (grid.sync()) return;
-  markBuild(P, g);
-  if (grid.sync()) return;
-  // reaction CSR: pairs by partner, in pair order
-  rcCountPairs(P, g);
-  if (grid.sync()) return;
+  // reaction CSR: pairs by partner (counted as they were written), in pair order
   scanReduceTiles(P.rcCount, P.nP, P.scanTiles, lds);
   if (grid.sync()) return;
-  scanApplyTiles(P.rcCount, P.nP, P.scanTiles, P.rcStart, lds);
+  markBuild(P, g);
+  scanApplyTiles(P.rcCount, P.nP, P.scanTiles, P.rcStart, lds, bigRc);
   if (grid.sync()) return;
   rcScatterPairs(P, g);
   if (grid.sync()) return;
   const int nRc = min(P.rcStart[P.nP], int(P.pairCap));
   bucketSortSmall(P.rcStart, P.nP, P.rcTmp, P.rcPair, P.rcSlot, P.sortBig, P.devInt + 2, g, nRc);
+  if (!*bigRc) return;
   if (grid.sync()) return;
   bucketSortBig(P.rcStart, P.rcTmp, P.rcPair, P.rcSlot, P.sortBig, P.devInt + 2, wave, nWaves, P.nP, nRc);
 }

@@ -2289,11 +2289,11 @@ int lsdem_surrogate_train(lsdem_ctx* c, const lsdem_surrogate_params* prm) {
     SurTrainArgs T{surNet(c), SurSamples{S.sx.p, S.sslot.p, S.st.p, p.samples},
                    (long long)((unsigned long long)it * (unsigned long long)p.batch % (unsigned long long)p.samples),
                    stride, p.batch, S.partial.p};
-    hipLaunchKernelGGL(k_sur_train, dim3(unsigned(blocks)), dim3(256), 0, c->stream, T);
+    hipLaunchKernelGGL(k_sur_train, dim3(unsigned(blocks)), dim3(kSurTrainThreads), 0, c->stream, T);
     SurAdamArgs Ad{S.param.p, S.embF.p, S.m.p, S.v.p, S.partial.p, blocks, S.nShapes, float(lr), float(b1), float(b2),
                    1e-8f, float(1.0 / (1.0 - std::pow(b1, it + 1))), float(1.0 / (1.0 - std::pow(b2, it + 1))),
                    S.wF.p, S.wB.p, S.emb.p, S.loss1.p};
-    hipLaunchKernelGGL(k_sur_adam, dim3(unsigned((nAll + 255) / 256)), dim3(256), 0, c->stream, Ad);
+    hipLaunchKernelGGL(k_sur_adam, dim3(unsigned((nAll + 64) / 64)), dim3(64), 0, c->stream, Ad);
   }
   HIPCHK(hipGetLastError());
   HIPCHK(hipEventRecord(e1, c->stream));
@@ -2414,7 +2414,7 @@ int lsdem_surrogate_gradient(lsdem_ctx* c, int64_t n, const float* points, const
   HIPCHK(hipMemcpy(t.p, targets, size_t(n) * sizeof(float), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(sl.p, slot.data(), size_t(n) * sizeof(int), hipMemcpyHostToDevice));
   SurTrainArgs T{surNet(c), SurSamples{x.p, sl.p, t.p, n}, 0, 1, int(n), part.p};
-  hipLaunchKernelGGL(k_sur_train, dim3(unsigned(blocks)), dim3(256), 0, c->stream, T);
+  hipLaunchKernelGGL(k_sur_train, dim3(unsigned(blocks)), dim3(kSurTrainThreads), 0, c->stream, T);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(c->stream));
   std::vector<float> h(size_t(blocks) * (nAll + 1));
@@ -2528,7 +2528,7 @@ int lsdem_surrogate_gradient_noalloc(lsdem_ctx* c, int64_t n, const float* point
                      shape_ids, (long long)n, (const int*)S.slotOfShape.p, int(c->shapes.size()), slot, bad);
   SurTrainArgs T{surNet(c), SurSamples{const_cast<float*>(points), slot, const_cast<float*>(targets), n}, 0, 1,
                  int(n), part};
-  hipLaunchKernelGGL(k_sur_train, dim3(unsigned(blocks)), dim3(256), 0, s, T);
+  hipLaunchKernelGGL(k_sur_train, dim3(unsigned(blocks)), dim3(kSurTrainThreads), 0, s, T);
   hipLaunchKernelGGL(k_sum_partials, dim3(unsigned((nAll + 1 + 255) / 256)), dim3(256), 0, s, (const float*)part,
                      blocks, nAll, grad, loss);
   HIPCHK(hipGetLastError());

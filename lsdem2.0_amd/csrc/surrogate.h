@@ -105,78 +105,8 @@ __device__ __forceinline__ float surFeature(int k, float ux, float uy, float uz)
   return (k & 1) ? cospif(t) : sinpif(t);
 }
 
-// Input operand blocks of one pass: lane's sample (ux, uy, uz, shape) and its 4 features per block.
-__device__ __forceinline__ void surInput(const SurNet& N, float ux, float uy, float uz, int shape, int lane,
-                                         sur_v4s x[kSurKB1], float xf[kSurKB1][4]) {
-  const int q = lane >> 4;
-#pragma unroll
-  for (int kb = 0; kb < kSurKB1; ++kb) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int k = 16 * kb + 4 * q + i;
-      xf[kb][i] = kb < 6 ? surFeature(k, ux, uy, uz) : surF32(N.emb[shape * kSurEmb + (k - 96)]);
-    }
-    x[kb] = surPack(xf[kb][0], xf[kb][1], xf[kb][2], xf[kb][3]);
-  }
-}
-
-// One dense layer in transposed form: z^T = W^T h^T + b for the pass's 16 samples.
-template <int KB>
-__device__ __forceinline__ void surLayer(const SurNet& N, int layer, const sur_v4s* in, int lane, float z[4][4]) {
-  const int q = lane >> 4;
-  const float* b = N.param + kSurOffB[layer];
-#pragma unroll
-  for (int mb = 0; mb < 4; ++mb) {
-    const sur_v4f acc = surMfmaK<KB>([&](int kb) { return N.wF[(kSurTileBase[layer] + mb * KB + kb) * 64 + lane]; },
-                                     [&](int kb) { return in[kb]; }, sur_v4f{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-    for (int i = 0; i < 4; ++i) z[mb][i] = acc[i] + b[16 * mb + 4 * q + i];
-  }
-}
-
-// Output of the pass for the lane's sample (all 4 lanes of a sample get the same value).
-__device__ __forceinline__ float surOutput(const SurNet& N, const float h4[4][4], int lane) {
-  const int q = lane >> 4;
-  const float* w5 = N.param + kSurOffW5;
-  float s = 0.f;
-#pragma unroll
-  for (int mb = 0; mb < 4; ++mb)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) s += h4[mb][i] * w5[16 * mb + 4 * q + i];
-  s += __shfl_xor(s, 16, 64);
-  s += __shfl_xor(s, 32, 64);
-  return s + N.param[kSurOffB5];
-}
-
-// Forward of one pass.  Keeps z of every layer (for training) when Z != nullptr.
-__device__ __forceinline__ float surForward(const SurNet& N, float ux, float uy, float uz, int shape, int lane,
-                                            sur_v4s x[kSurKB1], float zs[4][4][4], sur_v4s hs[3][4],
-                                            float h4[4][4]) {
-  float xf[kSurKB1][4];
-  surInput(N, ux, uy, uz, shape, lane, x, xf);
-  float z[4][4];
-  surLayer<kSurKB1>(N, 0, x, lane, z);
-#pragma unroll
-  for (int layer = 0; layer < 4; ++layer) {
-    if (layer > 0) surLayer<4>(N, layer, hs[layer - 1], lane, z);
-#pragma unroll
-    for (int mb = 0; mb < 4; ++mb) {
-      float a[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        zs[layer][mb][i] = z[mb][i];
-        a[i] = surSilu(z[mb][i]);
-      }
-      if (layer < 3) hs[layer][mb] = surPack(a[0], a[1], a[2], a[3]);
-      else
-#pragma unroll
-        for (int i = 0; i < 4; ++i) h4[mb][i] = a[i];
-    }
-  }
-  return surOutput(N, h4, lane);
-}
-
-// Forward of one pass for inference only (no saved activations): same arithmetic as surForward.
+// Forward of one pass (16 samples): output of the lane's sample, the same in its 4 lanes (the arithmetic of the
+// training kernel's forward).
 __device__ __forceinline__ float surForwardInfer(const SurNet& N, float ux, float uy, float uz, int shape, int lane) {
   const int q = lane >> 4;
   sur_v4s h[4];

@@ -6,7 +6,8 @@
 
 namespace lsd {
 
-constexpr int kSurRows = 64;  // samples per training block (4 waves x 16)
+constexpr int kSurRows = 64;  // samples per training block
+constexpr int kSurTrainThreads = 1024;  // 16 waves: 4 x 16 samples, each by 4 waves of 16 outputs
 
 struct SurSamples {
   float* x;        // [n][3] unscaled local points

@@ -22,7 +22,7 @@ __global__ void k_scan_apply(const int* in, long long n, const int* blockSum, in
 template <bool SEC> __global__ void k_kick_drift(Params P, int forceRebuild);
 __global__ void k_search_cells(Params P);
 template <bool SEC> __global__ void k_reduce_drift(Params P, StepHead H);
-__global__ void k_reduce_drift_small(Params P, StepHead H);
+template <bool SEC> __global__ void k_reduce_drift_small(Params P, StepHead H);
 __global__ void k_broad_phase(Params P);
 __global__ void k_bucket_count(const int* bucket, int n, int* count, int* rank, const int* gate);
 __global__ void k_bucket_scatter(const int* bucket, int n, const int* start, const int* rank, int* out,
@@ -549,12 +549,10 @@ void launchKickDrift(lsdem_ctx* c, int force) {
 void launchReduceDrift(lsdem_ctx* c, const StepHead& H) {
   const Params& P = c->P;
   const int bs = c->cfg.block_size > 0 ? c->cfg.block_size : 256;
-  if (P.periodicSector)
-    hipLaunchKernelGGL(k_reduce_drift<true>, dim3(blocksFor(P.nP + P.nW, bs)), dim3(bs), 0, c->stream, P, H);
-  else if (P.nP <= kWaveEndBodies)
-    hipLaunchKernelGGL(k_reduce_drift_small, dim3(blocksFor(P.nP + P.nW, bs)), dim3(bs), 0, c->stream, P, H);
-  else
-    hipLaunchKernelGGL(k_reduce_drift<false>, dim3(blocksFor(P.nP + P.nW, bs)), dim3(bs), 0, c->stream, P, H);
+  const bool small = P.nP <= kWaveEndBodies;
+  const auto kernel = P.periodicSector ? (small ? k_reduce_drift_small<true> : k_reduce_drift<true>)
+                                       : (small ? k_reduce_drift_small<false> : k_reduce_drift<false>);
+  hipLaunchKernelGGL(kernel, dim3(blocksFor(P.nP + P.nW, bs)), dim3(bs), 0, c->stream, P, H);
 }
 template <bool SUR>
 void launchCandidatesKernel(lsdem_ctx* c) {

@@ -512,12 +512,13 @@ __device__ __forceinline__ void kickDrift(const Params& P, int i, const BodyIn& 
   }
   if (unshifted) atomicAdd(&P.devInt[ghostCountIdx(buf)], unshifted);
   // rebuild the candidate pairs when a body has moved half the skin since the last build (a
-  // periodic wrap always does)
+  // periodic wrap always does, and a turn across a sector's face is one wherever it ends).  Sector images
+  // are turned about the corner's axis, so they move as far as their sources and the skin covers them as it
+  // covers shifted ones.  (Rebuilt every step, as sector periodicity once did: 4,000 bodies 0.22 ms a step,
+  // 0.059 now.)
   const double hs2 = P.halfSkin * P.halfSkin;
   const d3 dd = pDet - in.xBuild, dw = p - in.xBuildW;
-  // (with sector periodicity the pairs are rebuilt every step: a turned body's images and
-  // detection pose change by a quarter turn)
-  const bool moved = sector || len2(dd) > hs2 || len2(dw) > hs2;
+  const bool moved = turned || len2(dd) > hs2 || len2(dw) > hs2;
   if (__ballot(moved) && (threadIdx.x & 63) == __builtin_ctzll(__ballot(moved))) atomicOr(&P.devInt[rebuildFlagIdx(buf)], 1);
   // motion since the build for the separation certificates (a step that wraps rebuilds, so posDet
   // and pos move alike on every step that reads this)
@@ -2801,18 +2802,19 @@ __global__ void k_reduce_drift(Params P, StepHead H) {
     P.forceSet[b] = any ? 1 : 0;
   }
 }
-// The same for a small simulation (up to kWaveEndBodies bodies, no sector periodicity), whose
+// The same for a small simulation (up to kWaveEndBodies bodies), whose
 // counters the first wavefront closes (stepEndWave): its body pass is short, and thread 0's rounds of
 // counter reads were its last wavefront's (256 drums of 19k bodies in all: 0.0472 -> 0.0433 ms per
 // step).  In the 200k-body pass thread 0's version is the faster, and the kernel above is left as it
 // compiles alone (any change to it shifts its code generation).
+template <bool SEC>
 __global__ void k_reduce_drift_small(Params P, StepHead H) {
   LSD_HALT(P);
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
   BodyIn in;
   bool set = false;
   if (b < P.nP) {
-    in = loadBody<false>(P, b);
+    in = loadBody<SEC>(P, b);
     set = P.forceSet[b] != 0;
   }
   if (blockIdx.x == 0 && threadIdx.x < 64) stepEndWave(P, int(threadIdx.x));
@@ -2823,7 +2825,7 @@ __global__ void k_reduce_drift_small(Params P, StepHead H) {
   }
   d3 F, T;
   const bool any = reduceBody(P, b, F, T);
-  kickDrift<false>(P, b, in, F, T, 2, H.buf);
+  kickDrift<SEC>(P, b, in, F, T, 2, H.buf);
   if (any || set) {
     P.force[b] = F;
     P.torque[b] = T;
@@ -3146,6 +3148,8 @@ template __global__ void k_kick_drift<false>(Params P, int forceRebuild);
 template __global__ void k_kick_drift<true>(Params P, int forceRebuild);
 template __global__ void k_reduce_drift<false>(Params P, StepHead H);
 template __global__ void k_reduce_drift<true>(Params P, StepHead H);
+template __global__ void k_reduce_drift_small<false>(Params P, StepHead H);
+template __global__ void k_reduce_drift_small<true>(Params P, StepHead H);
 template __global__ void k_pair_check<false>(Params P, int full);
 template __global__ void k_pair_check<true>(Params P, int full);
 

@@ -1559,13 +1559,18 @@ __device__ __forceinline__ void makeF32(const Params& P, const PairView& v, Pair
 // build stays below the slack recorded at its last evaluation (all its nodes were culled then
 // with that much room).  Skipped pairs have no contacts.  full != 0 (an audit step of the
 // surrogate) also evaluates every live pair whose certificate rests on the surrogate's slack.
-// A block compacts a tile of 1024 pairs in LDS, appends it with one atomic, then writes the FP32
+// A block compacts a tile of pairs in LDS, appends it with one atomic, then writes the FP32
 // map records of its evaluated pairs (FP64 poses in, one 160-byte record out, in evaluation
-// order).  A block group g (blockIdx mod 8) checks one contiguous eighth of the tiles and writes the
+// order).  A tile has 256 pairs, one per thread, as long as those tiles are resident together (two
+// blocks per CU), else 1024: a short list is bound by each thread's chain of reads, which a thread's four
+// pairs lengthen (those near contact read the state of their last evaluation one after another, and their
+// records take several rounds), a long one by the number of tiles.  (Four pairs per thread on every list, before
+// -> now: @@ us.)  A block group g (blockIdx mod 8) checks one contiguous eighth of the tiles and writes the
 // records of its evaluated pairs from the first pair of its first tile on, with its own counter
 // (evalCount[g]): 8 counters on 8 lines instead of one, since returning atomics on one address are
 // served one after another (~11 ns each) and every tile takes one.
-constexpr int kCheckTile = 1024;
+constexpr int kCheckTile = 1024, kCheckTileShort = 256, kShortPairs = 512 * kCheckTileShort;
+__device__ __forceinline__ int checkTileSize(int nPairs) { return nPairs <= kShortPairs ? kCheckTileShort : kCheckTile; }
 
 // The evaluated pairs' map records, numbered densely group after group (record a of the narrow
 // phase) and found at their place in the groups' regions of pairMap.
@@ -1582,51 +1587,50 @@ struct EvalRecords {
     return pos;
   }
 };
-__device__ __forceinline__ int checkTiles(const Params& P) {
-  const int nPairs = min(P.pairStart[P.nP], (int)P.pairCap);
-  return (nPairs + kCheckTile - 1) / kCheckTile;
-}
 __device__ __forceinline__ int groupFirstTile(int nTiles, int g) { return int((long long)nTiles * g / 8); }
 __device__ __forceinline__ EvalRecords evalRecords(const Params& P) {
   EvalRecords e;
-  const int nTiles = checkTiles(P);
+  const int nPairs = min(P.pairStart[P.nP], (int)P.pairCap), tile = checkTileSize(nPairs);
+  const int nTiles = (nPairs + tile - 1) / tile;
   int sum = 0;
 #pragma unroll
   for (int g = 0; g < 8; ++g) {
     e.pre[g] = sum;
-    e.base[g] = groupFirstTile(nTiles, g) * kCheckTile;
+    e.base[g] = groupFirstTile(nTiles, g) * tile;
     sum += evalCount(P)[g * kBarrierLine];
   }
   e.n = sum;
   return e;
 }
-template <bool SEC>
-__global__ __launch_bounds__(256) void k_pair_check(Params P, int full) {
-  __shared__ int sList[kCheckTile], sA[kCheckTile];
-  __shared__ uint32_t sInfo[kCheckTile];
+struct CheckLds {
+  int list[kCheckTile], A[kCheckTile];
+  uint32_t info[kCheckTile];
+  int count, base;
+};
+// R: pairs of a tile per thread (tiles of 256 R)
+template <bool SEC, int R>
+__device__ void checkPairs(const Params& P, int full, int nPairs, CheckLds& L) {
+  constexpr int kTile = 256 * R;
+  int *const sList = L.list, *const sA = L.A;
+  uint32_t* const sInfo = L.info;
+  int &sCount = L.count, &sBase = L.base;
   PairF32* out = reinterpret_cast<PairF32*>(P.pairMap);
-  __shared__ int sCount, sBase;
-  LSD_HALT(P);  // (a failed broad phase leaves no pair list to read)
-  // the broad phase of this step is over: its grid barrier's words start the next one at zero
-  if (blockIdx.x == 0 && threadIdx.x < 10) P.barrier[threadIdx.x * kBarrierLine] = 0;
-  const int nPairs = min(P.pairStart[P.nP], (int)P.pairCap);
   const bool rebuilt = P.devInt[rebuildFlagIdx(P.curBuf)] != 0;  // a new pair list this step
   const bool fresh = !P.useCert;  // (a new list holds the certificates it inherited)
   const int lane = threadIdx.x & 63;
   const unsigned long long ltMask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   // XCD-aware tiles: workgroups go to the 8 XCDs in turn (blockIdx mod 8), so each XCD takes one
   // contiguous eighth of the pair list and its partners' data stays in that XCD's L2
-  const int nTiles = (nPairs + kCheckTile - 1) / kCheckTile;
+  const int nTiles = (nPairs + kTile - 1) / kTile;
   const int xcd = int(blockIdx.x) & 7, perX = (int(gridDim.x) - xcd + 7) >> 3;  // blocks on this XCD
   const int tLo = groupFirstTile(nTiles, xcd), tHi = groupFirstTile(nTiles, xcd + 1);
-  const int region = tLo * kCheckTile;  // this group's records: at most its pairs, from its first pair on
+  const int region = tLo * kTile;  // this group's records: at most its pairs, from its first pair on
   unsigned int evNodes = 0;  // boundary nodes of the masters of this thread's evaluated pairs
   for (int t = tLo + (int(blockIdx.x) >> 3); t < tHi; t += perX) {
-    const int t0 = t * kCheckTile;
+    const int t0 = t * kTile;
     if (threadIdx.x == 0) sCount = 0;
     __syncthreads();
     // the tile's pairs of this thread, with the loads of one kind issued together
-    constexpr int R = kCheckTile / 256;
     // (vector types: an element picked by a runtime index stays in registers, where an array's
     // would be read from scratch)
     typedef int IntR __attribute__((ext_vector_type(R)));
@@ -1743,34 +1747,49 @@ __global__ __launch_bounds__(256) void k_pair_check(Params P, int full) {
       }
     }
     __syncthreads();
-    if (threadIdx.x == 0) sBase = sCount ? region + atomicAdd(&evalCount(P)[xcd * kBarrierLine], sCount) : 0;
-    __syncthreads();
-    for (int k = threadIdx.x; k < sCount; k += 256) {
-      const int p = sList[k], a = sBase + k;
-      const PairView v = loadPair<SEC>(P, p, sInfo[k], sA[k]);
-      // the motion state of this evaluation, for the pair's certificate against later motion
-      // (loaded before the stores below)
-      const BodyStep sa = P.step[v.A];
-      const float4 qA = P.qrel[v.A];
-      float4 mB, qB;
-      float flip = 0.f;
-      if (v.type == PT_PW) {
-        mB = P.wMotion[v.partner];
-        qB = P.wQrel[v.partner];
-      } else {
-        const BodyStep sb = P.step[v.partner];
-        mB = sb.motion;
-        qB = P.qrel[v.partner];
-        if (v.type >= PT_GX) flip = float((partnerKey(sb.key, v.type) >> kFlipBit) & 1);
-      }
+    // (a short list's reservation returns while the pairs' states are read: it is the last wavefront's, which
+    // has a pair to read only when three quarters of the round are full; on a long one the others' reads hide it
+    // and the records, kept over the barrier, cost 1 us of 37)
+    const int count = sCount;
+    if (threadIdx.x == (R == 1 ? 255 : 0) && count) sBase = region + atomicAdd(&evalCount(P)[xcd * kBarrierLine], count);
+    if (R > 1) __syncthreads();
+    for (int k0 = 0; k0 < count; k0 += 256) {
+      const int k = k0 + int(threadIdx.x);
+      const bool on = k < count;
       PairF32 f;
-      makeF32(P, v, f);
-      out[a] = f;
-      P.pairRec[p] = a;
-      evNodes += unsigned(v.nNodes);
-      P.certE[p] = make_float4(sa.motion.x - mB.x, sa.motion.y - mB.y, sa.motion.z - mB.z, flip);
-      P.certQA[p] = qA;
-      P.certQB[p] = qB;
+      float4 e0 = make_float4(0.f, 0.f, 0.f, 0.f), qA = e0, qB = e0;
+      int p = 0;
+      if (on) {
+        p = sList[k];
+        const PairView v = loadPair<SEC>(P, p, sInfo[k], sA[k]);
+        // the motion state of this evaluation, for the pair's certificate against later motion
+        // (loaded before the stores below)
+        const BodyStep sa = P.step[v.A];
+        qA = P.qrel[v.A];
+        float4 mB;
+        float flip = 0.f;
+        if (v.type == PT_PW) {
+          mB = P.wMotion[v.partner];
+          qB = P.wQrel[v.partner];
+        } else {
+          const BodyStep sb = P.step[v.partner];
+          mB = sb.motion;
+          qB = P.qrel[v.partner];
+          if (v.type >= PT_GX) flip = float((partnerKey(sb.key, v.type) >> kFlipBit) & 1);
+        }
+        makeF32(P, v, f);
+        e0 = make_float4(sa.motion.x - mB.x, sa.motion.y - mB.y, sa.motion.z - mB.z, flip);
+        evNodes += unsigned(v.nNodes);
+      }
+      if (R == 1) __syncthreads();  // sBase (one round)
+      if (on) {
+        const int a = sBase + k;
+        out[a] = f;
+        P.pairRec[p] = a;
+        P.certE[p] = e0;
+        P.certQA[p] = qA;
+        P.certQB[p] = qB;
+      }
     }
     __syncthreads();
   }
@@ -1779,6 +1798,16 @@ __global__ __launch_bounds__(256) void k_pair_check(Params P, int full) {
     const unsigned long long sum = (unsigned long long)wsum(double(evNodes));
     if (lane == 0) atomicAdd(statSlot(P, 4, blockIdx.x & (kStatSlots - 1)), sum);
   }
+}
+template <bool SEC>
+__global__ __launch_bounds__(256) void k_pair_check(Params P, int full) {
+  __shared__ CheckLds L;
+  LSD_HALT(P);  // (a failed broad phase leaves no pair list to read)
+  // the broad phase of this step is over: its grid barrier's words start the next one at zero
+  if (blockIdx.x == 0 && threadIdx.x < 10) P.barrier[threadIdx.x * kBarrierLine] = 0;
+  const int nPairs = min(P.pairStart[P.nP], (int)P.pairCap);
+  if (checkTileSize(nPairs) == kCheckTileShort) checkPairs<SEC, 1>(P, full, nPairs, L);
+  else checkPairs<SEC, 4>(P, full, nPairs, L);
 }
 
 // The FP32 prefilters may contract a * b + c into one rounding: their margins bound the rounding
@@ -2506,16 +2535,20 @@ __global__ __launch_bounds__(kNarrowBlock, 3) void k_candidates(Params P) {
     if (mine) P.pairCcnt[sF[lane].pair] = contacts;
     statCand += (lane == 0) ? unsigned(total) : 0u;
   }
-  const unsigned long long t = (unsigned long long)wsum(double(statCand));
-  const unsigned long long te = (unsigned long long)wsum(double(statEnt));
-  const unsigned long long tq = (unsigned long long)wsum(double(statQueries));
-  const unsigned long long tc = (unsigned long long)wsum(double(statContacts));
-  if (lane0 == 0 && (t | te)) {
+  // (lane 0 counted the batches' candidates and entries; without a candidate no lane tested one)
+  const unsigned int t = __builtin_amdgcn_readfirstlane(statCand), te = __builtin_amdgcn_readfirstlane(statEnt);
+  if (!(t | te)) return;
+  unsigned long long tq = 0, tc = 0;
+  if (t) {
+    tq = (unsigned long long)wsum(double(statQueries));
+    tc = (unsigned long long)wsum(double(statContacts));
+  }
+  if (lane0 == 0) {
     const int slot = (blockIdx.x + wl) & (kStatSlots - 1);
-    atomicAdd(statSlot(P, 0, slot), t);
+    atomicAdd(statSlot(P, 0, slot), (unsigned long long)t);
     atomicAdd(statSlot(P, 1, slot), tq);
     atomicAdd(statSlot(P, 2, slot), tc);
-    atomicAdd(statSlot(P, 3, slot), te);
+    atomicAdd(statSlot(P, 3, slot), (unsigned long long)te);
   }
 }
 

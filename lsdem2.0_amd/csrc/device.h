@@ -120,6 +120,7 @@ struct Params {
   const float4* nodes32;  // same nodes in FP32 (x, y, z, 0) for the conservative prefilter
   const float* sdf;
   int maxClusters;        // largest cluster count of any shape
+  int residentWaves;      // wavefronts of the candidate kernel that are on the GPU together
 
   // ---- particles ----
   // State vectors lie in one block of nBodies = nP + nW entries each, walls after the particles, in the

@@ -1565,7 +1565,7 @@ __device__ __forceinline__ void makeF32(const Params& P, const PairView& v, Pair
 // blocks per CU), else 1024: a short list is bound by each thread's chain of reads, which a thread's four
 // pairs lengthen (those near contact read the state of their last evaluation one after another, and their
 // records take several rounds), a long one by the number of tiles.  (Four pairs per thread on every list, before
-// -> now: @@ us.)  A block group g (blockIdx mod 8) checks one contiguous eighth of the tiles and writes the
+// -> now: 15.7 -> 7.1 us for 1,000 bodies in a box, 15.2 -> 8.6 for 20,000 falling, 13.1 -> 7.3 for 8,000 bonded.)  A block group g (blockIdx mod 8) checks one contiguous eighth of the tiles and writes the
 // records of its evaluated pairs from the first pair of its first tile on, with its own counter
 // (evalCount[g]): 8 counters on 8 lines instead of one, since returning atomics on one address are
 // served one after another (~11 ns each) and every tile takes one.
@@ -2210,6 +2210,7 @@ __global__ __launch_bounds__(kNarrowBlock, 3) void k_candidates(Params P) {
   unsigned int* sMask = reinterpret_cast<unsigned int*>(sSub + subCap);  // 16-bit node masks, then also first slot << 16
   static_assert(kBatch * 4096 <= 65536, "a batch's slot offsets fit 16 bits (shapes have at most 4096 nodes)");
   const float kInf = __builtin_huge_valf();
+  __shared__ int sTotal[kNarrowBlock / 64], sFirst;
   LSD_HALT(P);
   unsigned int statCand = 0, statEnt = 0, statQueries = 0, statContacts = 0;
   const EvalRecords rec = evalRecords(P);
@@ -2220,13 +2221,18 @@ __global__ __launch_bounds__(kNarrowBlock, 3) void k_candidates(Params P) {
   const int iters = (maxC + 7) >> 3;
   // batch bi takes the evaluated pairs bi, bi + NB, bi + 2 NB, ...: pairs near contact come in
   // spatial runs, and spreading them over the batches keeps the slowest wavefront short
-  // pairs per batch: when few pairs are evaluated, small batches spread the slowest pairs (those
-  // near contact, with many surviving clusters) over more wavefronts (one pair per wavefront when
-  // there are at least eight wavefronts per pair, as in small simulations)
+  // pairs per batch: the smallest number whose batches are all on the GPU together, which spreads the slowest
+  // pairs (those near contact, with many surviving clusters) over the most wavefronts; eight beyond that, since
+  // the lanes of a batch of eight are all used.  (One only from eight wavefronts per pair on, two from two: 11.2
+  // ms for 200 steps of 1,000 bodies in a box, now 10.3; 4.14 and 3.98 for 50 of 27; others within 2 %.)
+  const int fit = min(nWaves, P.residentWaves);
   const int nb = P.narrowBatch > 0 ? P.narrowBatch
-                                   : (nAct <= nWaves / 8 ? 1 : (nAct <= nWaves / 2 ? 2 : (nAct <= nWaves ? 4 : kBatch)));
+                                   : (nAct <= fit ? 1 : (nAct <= 2 * fit ? 2 : (nAct <= 4 * fit ? 4 : kBatch)));
   const int NB = (nAct + nb - 1) / nb;
-  for (int bi = wave; bi < NB; bi += nWaves) {
+  // (the block's wavefronts turn together: each turn reserves for all four; one past the last batch has no pairs)
+  for (int b0 = int(blockIdx.x * (kNarrowBlock / 64)); b0 < NB; b0 += nWaves) {
+    const int bi = b0 + wave % (kNarrowBlock / 64);
+    const int nAct = bi < NB ? rec.n : 0;
     // (what follows from the lane is worked out in each batch: kept in registers through the loop, the
     // addresses of every stage together take half of a wavefront's registers)
     const int lane = inLoop(lane0, bi);
@@ -2372,10 +2378,20 @@ __global__ __launch_bounds__(kNarrowBlock, 3) void k_candidates(Params P) {
       }
     }
     __builtin_amdgcn_wave_barrier();
-    // ---- one reservation per batch, exact size, and the reads of what the exact tests need: in flight
-    // together, used after the certificates and the list of slots are done ----
-    int first = 0;
-    if (total > 0 && lane == 0) first = atomicAdd(&P.devInt[1], total);
+    // ---- one reservation per turn of the block, exact size, and the reads of what the exact tests need: in
+    // flight together, used after the certificates and the list of slots are done.  (Returning atomics on one
+    // address are served 11 ns apart: one per batch was 8.7 us of the kernel's 32 for 794 batches that arrive
+    // together, now 25 in all; an ordered bed of 10,000 batches 157 -> 147.) ----
+    if (lane == 0) sTotal[wl] = total;
+    __syncthreads();
+    int ahead = 0, blockTotal = 0, blockFirst = 0;
+#pragma unroll
+    for (int w = 0; w < kNarrowBlock / 64; ++w) {
+      const int t = sTotal[w];
+      ahead += w < wl ? t : 0;
+      blockTotal += t;
+    }
+    if (blockTotal > 0 && threadIdx.x == 0) blockFirst = atomicAdd(&P.devInt[1], blockTotal);
     const bool mine = lane < nb && bi + lane * NB < nAct;
     const bool share = own && sCnt[j] > 0;
     PairShare part{};
@@ -2453,7 +2469,11 @@ __global__ __launch_bounds__(kNarrowBlock, 3) void k_candidates(Params P) {
         __builtin_amdgcn_wave_barrier();
         pairLaw(sF[j].info, k, sX[j]);
       }
-      first = __builtin_amdgcn_readfirstlane(first);
+    }
+    if (threadIdx.x == 0) sFirst = blockFirst;
+    __syncthreads();
+    const int first = __builtin_amdgcn_readfirstlane(sFirst + ahead);
+    if (total > 0) {
       if ((long long)first + total > P.contactCap) {
         // the call halts with a capacity error; slots reserved below the capacity stay empty
         if (lane == 0) {

@@ -552,7 +552,7 @@ void launchReduceDrift(lsdem_ctx* c, const StepHead& H) {
   const bool small = P.nP <= kWaveEndBodies;
   const auto kernel = P.periodicSector ? (small ? k_reduce_drift_small<true> : k_reduce_drift<true>)
                                        : (small ? k_reduce_drift_small<false> : k_reduce_drift<false>);
-  hipLaunchKernelGGL(kernel, dim3(blocksFor(P.nP + P.nW, bs)), dim3(bs), 0, c->stream, P, H);
+  hipLaunchKernelGGL(kernel, dim3(blocksFor(P.nP + P.nW, bs) + (small ? 1 : 0)), dim3(bs), 0, c->stream, P, H);
 }
 template <bool SUR>
 void launchCandidatesKernel(lsdem_ctx* c) {
@@ -598,13 +598,13 @@ void launchReduceKick(lsdem_ctx* c) {
   const int bs = c->cfg.block_size > 0 ? c->cfg.block_size : 256;
   hipStream_t s = c->stream;
   if (c->hookFn) {
-    hipLaunchKernelGGL(k_reduce_kick, dim3(blocksFor(P.nP, bs)), dim3(bs), 0, s, P, 0);
+    hipLaunchKernelGGL(k_reduce_kick, dim3(blocksFor(P.nP, bs) + 1), dim3(bs), 0, s, P, 0);
     lsdem_device_view v;
     deviceView(c, &v);
     c->hookFn(c->hookUser, c->time, &v);
     hipLaunchKernelGGL(k_kick, dim3(blocksFor(P.nP, bs)), dim3(bs), 0, s, P);
   } else {
-    hipLaunchKernelGGL(k_reduce_kick, dim3(blocksFor(P.nP, bs)), dim3(bs), 0, s, P, 1);
+    hipLaunchKernelGGL(k_reduce_kick, dim3(blocksFor(P.nP, bs) + 1), dim3(bs), 0, s, P, 1);
   }
 }
 

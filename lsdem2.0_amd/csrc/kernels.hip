@@ -2811,11 +2811,13 @@ __device__ __forceinline__ bool reduceBody(const Params& P, int b, d3& F, d3& T)
   return any;
 }
 
-// One thread per body.  Thread 0 also closes the step's bookkeeping.
+// One thread per body.  The last block, which has no bodies of its own, closes the step's bookkeeping with its
+// first wavefront (thread 0 before its body's sums: 9.2 us of 27 bodies' steps one by one, now 4.5; 9.8 and 4.6 for
+// 3,000 with a hook).
 __global__ void k_reduce_kick(Params P, int kick) {
   LSD_HALT(P);
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b == 0) stepEnd(P);
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x < 64) stepEndWave(P, int(threadIdx.x));
   if (b >= P.nP) return;
   d3 F, T;
   reduceBody(P, b, F, T);
@@ -2856,10 +2858,11 @@ __global__ void k_reduce_drift(Params P, StepHead H) {
   }
 }
 // The same for a small simulation (up to kWaveEndBodies bodies), whose
-// counters the first wavefront closes (stepEndWave): its body pass is short, and thread 0's rounds of
-// counter reads were its last wavefront's (256 drums of 19k bodies in all: 0.0472 -> 0.0433 ms per
-// step).  In the 200k-body pass thread 0's version is the faster, and the kernel above is left as it
-// compiles alone (any change to it shifts its code generation).
+// counters a wavefront of a block of its own closes (stepEndWave): its body pass is short, and thread 0's
+// rounds of counter reads were its last wavefront's (256 drums of 19k bodies in all: 0.0472 -> 0.0433 ms per
+// step; the wavefront beside the bodies instead of before them another 1 % for 1,000).  In the 200k-body pass
+// thread 0's version is the faster, and the kernel above is left as it compiles alone (any change to it shifts
+// its code generation).
 template <bool SEC>
 __global__ void k_reduce_drift_small(Params P, StepHead H) {
   LSD_HALT(P);
@@ -2870,8 +2873,10 @@ __global__ void k_reduce_drift_small(Params P, StepHead H) {
     in = loadBody<SEC>(P, b);
     set = P.forceSet[b] != 0;
   }
-  if (blockIdx.x == 0 && threadIdx.x < 64) stepEndWave(P, int(threadIdx.x));
-  stepHead(P, H, b, int(gridDim.x * blockDim.x));
+  // (the last block's thread 0 clears what its wavefront has just summed)
+  const int bs = int(blockDim.x), last = int(gridDim.x - 1) * bs;
+  if (b >= last && threadIdx.x < 64) stepEndWave(P, int(threadIdx.x));
+  stepHead(P, H, b >= last ? b - last : b + bs, last + bs);
   if (b >= P.nP) {
     if (b - P.nP < P.nW) wallDrift(P, b - P.nP, H.buf);
     return;

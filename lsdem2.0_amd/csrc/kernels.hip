@@ -2891,7 +2891,7 @@ __global__ void k_reduce_drift_small(Params P, StepHead H) {
   }
 }
 
-// Close of the pre-loop build: step bookkeeping, and the contact flags of the candidate kernel
+// Close of the pre-loop build: step bookkeeping, and the contact masks of the candidate kernel
 // cleared (no sums follow; the stored forces stay those of the last step).
 __global__ void k_prime_end(Params P) {
   LSD_HALT(P);

@@ -141,6 +141,20 @@ __device__ __forceinline__ int prefetchArgs(int v) {
 #undef LSD_LINE
   return v;
 }
+// v, as a value of turn `turn` of a loop (of item `item`): what is computed from it is worked out there, and not kept
+// in registers from before.  (No volatile asm, as for prefetchArgs.)
+__device__ __forceinline__ int inLoop(int v, int turn) {
+  asm("" : "+v"(v) : "s"(turn));
+  return v;
+}
+__device__ __forceinline__ int uniformInItem(int v, int item) {
+  asm("" : "+s"(v) : "v"(item));
+  return v;
+}
+__device__ __forceinline__ double inItem(double v, int item) {
+  asm("" : "+v"(v) : "v"(item));
+  return v;
+}
 // An error flag is up: this kernel has nothing to do.
 #define LSD_HALT(P) \
   if ((P).devInt[prefetchArgs(3)] != 0) return
@@ -194,7 +208,6 @@ struct Span {
 __device__ __forceinline__ Span gridSpan() {
   return Span{int(blockIdx.x * blockDim.x + threadIdx.x), int(gridDim.x * blockDim.x)};
 }
-
 // Phase 1 of the scan: the sum of each tile of blockDim.x x kScanItems inputs (blocks loop over
 // tiles).
 __device__ void scanReduceTiles(const int* in, long long n, int* tileSum, int* lds) {
@@ -320,6 +333,12 @@ __device__ __forceinline__ d3* imgVel(const Params& P, int s) { return pick3(s, 
 __device__ __forceinline__ d3 secTurn(const Params& P, int s, d3 v) {
   return rodrigues(v, pick3(s, P.secW[0], P.secW[1], P.secW[2]), pick3(s, P.secA[0], P.secA[1], P.secA[2]),
                    pick3(s, P.secB[0], P.secB[1], P.secB[2]));
+}
+// The same, with the set's constants read by their index from the argument block (Params is its first member): picked
+// from all three sets they take the registers of all three.  For kernels, not for functions that are called.
+__device__ __forceinline__ d3 secTurnByIndex(int s, d3 v) {
+  const auto* a = (const __attribute__((address_space(4))) Params*)__builtin_amdgcn_kernarg_segment_ptr();
+  return rodrigues(v, mk3(a->secW[s].x, a->secW[s].y, a->secW[s].z), a->secA[s], a->secB[s]);
 }
 __device__ __forceinline__ q4 secQuat(const Params& P, int s) { return pick3(s, P.secR[0], P.secR[1], P.secR[2]); }
 
@@ -667,10 +686,10 @@ __device__ void bucketSortSmall(const int* start, int nb, const int* tmp, int* i
   }
 }
 // One wavefront per listed bucket: each item's place is the number of smaller items (items are
-// distinct indices).  `wave` / `nWaves`: this wavefront's index and the number of wavefronts.
+// distinct indices).
 __device__ void bucketSortBig(const int* start, const int* tmp, int* items, int* inv, const int* bigList,
-                              const int* bigCount, int wave, int nWaves, int nb, int nItems) {
-  const int lane = threadIdx.x & 63;
+                              const int* bigCount, Span g, int nb, int nItems) {
+  const int lane = threadIdx.x & 63, wave = g.tid >> 6, nWaves = g.nth >> 6;
   const int nBig = min(*bigCount, nb);
   for (int q = wave; q < nBig; q += nWaves) {
     const int b = bigList[q];
@@ -708,8 +727,7 @@ __global__ void k_bucket_sort(const int* start, int nb, const int* tmp, int* ite
 __global__ void k_bucket_sort_big(const int* start, int nb, const int* tmp, int* items, int* inv, const int* bigList,
                                   const int* bigCount, const int* gate, int nItems) {
   LSD_GATE(gate);
-  const Span g = gridSpan();
-  bucketSortBig(start, tmp, items, inv, bigList, bigCount, g.tid >> 6, g.nth >> 6, nb, nItems);
+  bucketSortBig(start, tmp, items, inv, bigList, bigCount, gridSpan(), nb, nItems);
 }
 
 __device__ __forceinline__ double triAt(const Params& P, const ShapeDev& S, double sc, d3 loc, d3 go, double invSp,
@@ -759,7 +777,7 @@ struct WallReach {
   float fx, fy, fz, fr, mA;
   __device__ __forceinline__ WallReach(const Params& P, int A) {
     xA = P.posDet[A];
-    rs = P.radius[A] + 2.0 * P.halfSkin;  // the wall and the particle each move < half the skin
+    rs = P.radius[A] + 2.0 * inItem(P.halfSkin, A);  // the wall and the particle each move < half the skin
     rr = rs * (1.0 + 1e-9) + 1e-12;
     fx = float(xA.x); fy = float(xA.y); fz = float(xA.z);
     fr = float(rr);
@@ -936,39 +954,25 @@ __device__ __forceinline__ int reactionRank(const Params& P, int A, uint32_t inf
 }
 
 // Candidate pairs of the master in sorted position t (A = sorted[t]) come in a fixed order, particle
-// partners, walls, then ghost images set by set, found by a group of 32 lanes.  DIRECT writes them to the
-// pair list from `out` on; otherwise the first kPairSlab go to the master's part of the slab and all are counted.
+// partners, walls, then ghost images set by set, found by a group of 32 lanes.  The first `room` of them go to
+// `list` (the master's part of the slab, or its entries of the pair list) and all are counted.
 constexpr int kPairSlab = kPairSlabHost;
-template <bool DIRECT>
 struct PairSink {
-  const Params& P;
   int t, A;
-  long long out;
-  int cnt;
+  uint32_t* list;
+  int room, cnt;
   // (by the whole group: the lanes with a hit are numbered in lane order)
   __device__ __forceinline__ void put(const FindGroup& G, bool hit, uint32_t type, int partner) {
     const unsigned int m = G.ballot(hit);
-    if (hit) {
-      const uint32_t info = (type << 28) | uint32_t(partner);
-      const int k = cnt + __popc(m & G.below());
-      if (DIRECT) {
-        if (out + k < P.pairCap) {
-          P.pairA[out + k] = A;
-          P.pairInfo[out + k] = info;
-          P.rcRank[out + k] = reactionRank(P, A, info);
-        }
-      } else if (k < kPairSlab) {
-        P.pairSlab[(long long)t * kPairSlab + k] = info;
-      }
-    }
+    const int k = cnt + __popc(m & G.below());
+    if (hit && k < room) list[k] = (type << 28) | uint32_t(partner);
     cnt += __popc(m);
   }
 };
 
 // Particle partners (B > A, B inside the domain, bounding spheres within the skin), then walls (each wall's
 // key is checked each step when the pair is used).
-template <bool DIRECT>
-__device__ __forceinline__ void nearPairs(const Params& P, PairSink<DIRECT>& sink, const FindGroup& G) {
+__device__ __forceinline__ void nearPairs(const Params& P, PairSink& sink, const FindGroup& G) {
   const int A = sink.A;
   const float4 a = P.sPR[sink.t];
   const unsigned long long walls = P.nW > 0 && P.nW <= kMaskWalls ? P.wallMask[sink.t] : 0ull;
@@ -1022,13 +1026,13 @@ struct ImageSearch {
   __device__ __forceinline__ d3 centre(int s, bool shifted) const {
     const d3 x = mk3(g.x, g.y, g.z);
     if (!shifted) return x;
-    if (sector) return P.gridP.mn + secTurn(P, 2 - s, x - P.gridP.mn);
+    if (sector) return P.gridP.mn + secTurnByIndex(2 - s, x - P.gridP.mn);
     return mk3(x.x - double(s != 1 ? lx : 0.f), x.y - double(s != 0 ? ly : 0.f), x.z);
   }
   // the image of a source at b (shifted by the period, or turned about the corner's z axis)
   __device__ __forceinline__ float4 image(int s, float4 b) const {
     if (!sector) return make_float4(b.x + (s != 1 ? lx : 0.f), b.y + (s != 0 ? ly : 0.f), b.z, 0.f);
-    const d3 r = P.gridP.mn + secTurn(P, s, mk3(b.x, b.y, b.z) - P.gridP.mn);
+    const d3 r = P.gridP.mn + secTurnByIndex(s, mk3(b.x, b.y, b.z) - P.gridP.mn);
     return make_float4(float(r.x), float(r.y), float(r.z), 0.f);
   }
   __device__ __forceinline__ bool reaches(int s, bool shifted) const {
@@ -1039,14 +1043,13 @@ struct ImageSearch {
 __device__ __forceinline__ bool mayMeetImages(const Params& P, int t) {
   const ImageSearch I(P, t);
   bool any = false;
+#pragma unroll 1
   for (int s = 0; s < 3; ++s) any = any || I.reaches(s, true) || (I.anyUnshifted && I.reaches(s, false));
   return any;
 }
-template <bool DIRECT>
-__device__ __forceinline__ void imagePairs(const Params& P, PairSink<DIRECT>& sink, const FindGroup& G) {
+__device__ __forceinline__ void imagePairs(const Params& P, PairSink& sink, const FindGroup& G) {
   const ImageSearch I(P, sink.t);
   const GridGeom& grid = P.gridP;
-  const double hs = P.halfSkin;
   const float skin = float(2.0 * P.halfSkin);
   for (int s = 0; s < 3; ++s) {
     const int col = I.sector ? imageColumn<true>(s) : imageColumn<false>(s);
@@ -1063,16 +1066,20 @@ __device__ __forceinline__ void imagePairs(const Params& P, PairSink<DIRECT>& si
                    [&](const Item& it, int k, bool in) {
                      bool hit = false;
                      int j = -1;
+                     // (the set and half the skin as values of this item: what follows from them in FP64, a turn's
+                     // terms and the bounds of the tests below, would be kept in registers through the search)
+                     const int si = uniformInItem(s, k);
                      const float rb = it.box + skin;
-                     if (in && spheresMayOverlap(I.g, shifted ? I.image(s, it.b) : it.b, rb)) {
+                     if (in && spheresMayOverlap(I.g, shifted ? I.image(si, it.b) : it.b, rb)) {
                        j = P.sorted[k];
+                       const double hs = inItem(P.halfSkin, j);
                        const d3 pj = P.pos[j];
                        if (shifted) {
                          hit = potInColumn(grid, pj, col, hs);
                        } else {
                          // (one pair per master and image: the shifted pass already took it)
                          hit = potOutOfDomain(P, pj, hs) && potOutColumn(grid, pj, col, hs) &&
-                               !(potInColumn(grid, pj, col, hs) && spheresMayOverlap(I.g, I.image(s, it.b), rb));
+                               !(potInColumn(grid, pj, col, hs) && spheresMayOverlap(I.g, I.image(si, it.b), rb));
                        }
                      }
                      sink.put(G, hit, PT_GX + s, j);
@@ -1094,6 +1101,25 @@ struct MasterShare {
   }
 };
 
+// Lists the masters of a block's share that want(t), a turn of blockDim.x at a time (many: an int per thread, and
+// one), and takes them one per group of 32 lanes: use(t).
+template <class Want, class Use>
+__device__ __forceinline__ void listedMasters(const Params& P, const MasterShare& share, int* many, Want&& want,
+                                              Use&& use) {
+  int* const nMany = many + blockDim.x;
+  const int group = int(threadIdx.x) / kFindLanes, groups = int(blockDim.x) / kFindLanes;
+  for (int i0 = 0; i0 < share.chunk; i0 += int(blockDim.x)) {
+    __threadfence_block();
+    __syncthreads();
+    if (threadIdx.x == 0) *nMany = 0;
+    __syncthreads();
+    const int i = i0 + int(threadIdx.x), t = share.at(i);
+    if (i < share.chunk && t < P.nP && want(t)) many[atomicAdd(nMany, 1)] = t;
+    __syncthreads();
+    for (int m = group; m < *nMany; m += groups) use(many[m]);
+  }
+}
+
 // Broad phase, 32 lanes per master: count its candidates and keep the first.  Bound by each master's chain of
 // round trips (its own data, the row lookups, four rounds of 32 items at a time) and by how unevenly masters
 // meet neighbours.  Images are searched in a turn of their own for the masters that may have any.  (One
@@ -1110,27 +1136,18 @@ __device__ void pairsFind(const Params& P, int* queues, int* many) {
   for (int i = group; i < share.chunk; i += groups) {
     const int t = share.at(i);
     if (t >= P.nP) continue;
-    PairSink<false> sink{P, t, P.sorted[t], 0, 0};
+    PairSink sink{t, P.sorted[t], P.pairSlab + (long long)t * kPairSlab, kPairSlab, 0};
     nearPairs(P, sink, G);
     if (G.l == 0) P.pairCount[sink.A] = sink.cnt;
   }
   if (!(P.periodicX || P.periodicY || P.periodicSector)) return;
-  int* const nMany = many + blockDim.x;
-  for (int i0 = 0; i0 < share.chunk; i0 += int(blockDim.x)) {
-    __threadfence_block();
-    __syncthreads();
-    if (threadIdx.x == 0) *nMany = 0;
-    __syncthreads();
-    const int i = i0 + int(threadIdx.x), ti = share.at(i);
-    if (i < share.chunk && ti < P.nP && mayMeetImages(P, ti)) many[atomicAdd(nMany, 1)] = ti;
-    __syncthreads();
-    for (int m = group; m < *nMany; m += groups) {
-      const int t = many[m], A = P.sorted[t];
-      PairSink<false> sink{P, t, A, 0, P.pairCount[A]};
-      imagePairs(P, sink, G);
-      if (G.l == 0) P.pairCount[A] = sink.cnt;
-    }
-  }
+  listedMasters(P, share, many, [&](int t) { return mayMeetImages(P, t); },
+                [&](int t) {
+                  const int A = P.sorted[t];
+                  PairSink sink{t, A, P.pairSlab + (long long)t * kPairSlab, kPairSlab, P.pairCount[A]};
+                  imagePairs(P, sink, G);
+                  if (G.l == 0) P.pairCount[inLoop(A, 1)] = sink.cnt;
+                });
 }
 constexpr int kFindThreads = 256;  // block of the separate search launches
 __global__ __launch_bounds__(kFindThreads) void k_pairs_find(Params P) {
@@ -1138,46 +1155,59 @@ __global__ __launch_bounds__(kFindThreads) void k_pairs_find(Params P) {
   __shared__ int queues[kFindThreads / kFindLanes * kFindQueue], many[kFindThreads + 1];
   pairsFind(P, queues, many);
 }
+// Entry k of master A's part of the pair list (from `out` on), its rank among the partner's reactions with it.
+__device__ __forceinline__ void emitPair(const Params& P, int A, long long out, int k, uint32_t info) {
+  const int rank = reactionRank(P, A, info);
+  if (out + k < P.pairCap) {
+    P.pairA[out + k] = A;
+    P.pairInfo[out + k] = info;
+    P.rcRank[out + k] = rank;
+  }
+}
 // Pair list in master order: eight lanes per master copy its part of the slab, eight candidates a turn (a thread
 // per master took as many turns as a master has candidates: 24 us of a rebuild for 4,000 bodies in a quarter
-// sector, now 7); the masters of the block's turn with more candidates than the slab holds are listed in
-// LDS and searched again, 32 lanes each.
+// sector, now 7); masters with more candidates than the slab holds are searched again, into their part of the list.
+// queues, many: as pairsFind.
 __device__ void pairsEmit(const Params& P, int* queues, int* many) {
   constexpr int kLanes = 8;
   const FindGroup G = findGroup(queues);
-  int* const nMany = many + blockDim.x;
+  const MasterShare share(P.nP);
   const int l = int(threadIdx.x) & (kLanes - 1), perBlock = int(blockDim.x) / kLanes;
-  for (int t0 = int(blockIdx.x) * perBlock; t0 < P.nP; t0 += int(gridDim.x) * perBlock) {
-    const int t = t0 + int(threadIdx.x) / kLanes;
-    if (threadIdx.x == 0) *nMany = 0;
-    __syncthreads();
-    if (t < P.nP) {
-      const int A = P.sorted[t];
-      const int n = P.pairCount[A];
-      const long long out = P.pairStart[A];
-      if (n <= kPairSlab) {
-        for (int k = l; k < n; k += kLanes) {
-          const uint32_t info = P.pairSlab[(long long)t * kPairSlab + k];
-          const int rank = reactionRank(P, A, info);
-          if (out + k < P.pairCap) {
-            P.pairA[out + k] = A;
-            P.pairInfo[out + k] = info;
-            P.rcRank[out + k] = rank;
-          }
-        }
-      } else if (l == 0) {
-        many[atomicAdd(nMany, 1)] = t;
-      }
-    }
-    __syncthreads();
-    for (int m = int(threadIdx.x) / kFindLanes; m < *nMany; m += int(blockDim.x) / kFindLanes) {
-      const int A = P.sorted[many[m]];
-      PairSink<true> sink{P, many[m], A, P.pairStart[A], 0};
-      nearPairs(P, sink, G);
-      if (P.periodicX || P.periodicY || P.periodicSector) imagePairs(P, sink, G);
-    }
-    __syncthreads();
+  int* const anyLarge = many + blockDim.x;
+  if (threadIdx.x == 0) *anyLarge = 0;
+  __syncthreads();
+  for (int i = int(threadIdx.x) / kLanes; i < share.chunk; i += perBlock) {
+    const int t = share.at(i);
+    if (t >= P.nP) continue;
+    const int A = P.sorted[t];
+    const int n = P.pairCount[A];
+    const long long out = P.pairStart[A];
+    if (n > kPairSlab) *anyLarge = 1;
+    else
+      for (int k = l; k < n; k += kLanes) emitPair(P, A, out, k, P.pairSlab[(long long)t * kPairSlab + k]);
   }
+  __syncthreads();
+  if (!*anyLarge) return;
+  // (three passes over the block's large masters: with both searches in one loop, registers spill.  rank, free
+  // since the sort, keeps how many partners and walls the first found.)
+  const auto isLarge = [&](int t) { return P.pairCount[P.sorted[t]] > kPairSlab; };
+  listedMasters(P, share, many, isLarge, [&](int t) {
+    const int A = P.sorted[t];
+    PairSink sink{t, A, P.pairInfo + P.pairStart[A], P.pairCount[A], 0};
+    nearPairs(P, sink, G);
+    if (G.l == 0) P.rank[t] = sink.cnt;
+  });
+  if (P.periodicX || P.periodicY || P.periodicSector)
+    listedMasters(P, share, many, isLarge, [&](int t) {
+      const int A = P.sorted[t];
+      PairSink sink{t, A, P.pairInfo + P.pairStart[A], P.pairCount[A], P.rank[t]};
+      imagePairs(P, sink, G);
+    });
+  listedMasters(P, share, many, isLarge, [&](int t) {
+    const int A = P.sorted[t], n = P.pairCount[A];
+    const long long out = P.pairStart[A];
+    for (int k = G.l; k < n; k += kFindLanes) emitPair(P, A, out, k, P.pairInfo[out + k]);
+  });
 }
 // Keep the pair list being replaced (per-master starts, entries, certificates) for the
 // certificates the new list inherits; runs before the new starts and entries are written.
@@ -2066,13 +2096,6 @@ __device__ __forceinline__ bool exactSlot(const Params& P, int c, const PairF32&
   P.cEs[c] = 0.5 * len2(spring) * ks;
   out = SlotTerms{F, cross(armA, F), cross(armB, -F)};
   return true;
-}
-
-// v, as a value of turn `turn` of a loop: what is computed from it stays inside the loop.  (No volatile asm,
-// as for prefetchArgs.)
-__device__ __forceinline__ int inLoop(int v, int turn) {
-  asm("" : "+v"(v) : "s"(turn));
-  return v;
 }
 
 // One lane's share of a pair's PairExact record: 8 lanes fill a record, 4 per body.  Lane t of a body reads
@@ -3078,6 +3101,12 @@ __device__ void stepEnd(const Params& P) {
 // cost of a barrier grows with the number of blocks) while many threads work between them.
 constexpr int kBroadThreads = 1024;
 
+// Grid-stride loop bounds of phase `n` (a constant), worked out there: kept from the kernel's start, the indices
+// cost the phases between registers.
+__device__ __forceinline__ Span phaseSpan(int n) {
+  return Span{int(blockIdx.x) * kBroadThreads + inLoop(int(threadIdx.x), n), int(gridDim.x) * kBroadThreads};
+}
+
 // Grid barrier in two levels (its words are zeroed by the pair check, the launch that follows every
 // broad phase, and by the host after a failed call): a block arrives on
 // its group's counter (group = blockIdx mod 8, the XCD the block runs on when the dispatcher deals
@@ -3095,8 +3124,8 @@ struct GridBarrier {
   __device__ bool sync() {
     __shared__ int abandon;
     __syncthreads();
+    ++passed;  // (by every thread: a uniform value takes no vector register)
     if (threadIdx.x == 0) {
-      ++passed;
       const int g = int(blockIdx.x) & 7;
       const int nGroups = min(nBlocks, 8);
       const int inGroup = (nBlocks - g + 7) >> 3;  // blocks b < nBlocks with b mod 8 == g
@@ -3130,47 +3159,54 @@ struct GridBarrier {
   }
 };
 
+// No vector register of this kernel may spill (1024 threads have 128 each): the compiler has put a spill at the head
+// of a join block, before the lanes of the other side are back, so that only some lanes' values were kept, and the
+// search then ran on garbage indices.
 __global__ __launch_bounds__(kBroadThreads) void k_broad_phase(Params P) {
   LSD_HALT(P);
   if (P.devInt[rebuildFlagIdx(P.curBuf)] == 0) return;  // written by the drift kernel before this launch: grid-uniform
   __shared__ int lds[kScanLds];
   __shared__ int queues[kBroadThreads / kFindLanes * kFindQueue], many[kBroadThreads + 1];
   GridBarrier grid{P, int(gridDim.x), 0};
-  const Span g = gridSpan();
-  const int wave = g.tid >> 6, nWaves = g.nth >> 6;
   const int ncell = P.sg.ncell;
   int* const bigCells = P.devInt + kBigCellsIdx;  // any cell (any reaction list) of more than kSmallBucket items:
   int* const bigRc = P.devInt + kBigRcIdx;        // without one, the phase that sorts those is left out
   // counting sort of the particles by search cell
-  for (int i = g.tid; i < ncell; i += g.nth) P.cellCount[i] = 0;
-  for (int i = g.tid; i < P.nP; i += g.nth) {
-    P.rcCount[i] = 0;
-    P.scell[i] = searchCellOf(P, i);
+  {
+    const Span g = phaseSpan(0);
+    for (int i = g.tid; i < ncell; i += g.nth) P.cellCount[i] = 0;
+    for (int i = g.tid; i < P.nP; i += g.nth) {
+      P.rcCount[i] = 0;
+      P.scell[i] = searchCellOf(P, i);
+    }
   }
-  if (g.tid == 0) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
     P.devInt[2] = 0;  // large-bucket list
     *bigCells = 0;
     *bigRc = 0;
   }
   if (grid.sync()) return;
-  bucketCount(P.scell, P.nP, P.cellCount, P.rank, g);
+  bucketCount(P.scell, P.nP, P.cellCount, P.rank, phaseSpan(1));
   if (grid.sync()) return;
   scanReduceTiles(P.cellCount, ncell, P.scanTiles, lds);
   if (grid.sync()) return;
   scanApplyTiles(P.cellCount, ncell, P.scanTiles, P.cellStart, lds, bigCells);
   if (grid.sync()) return;
-  bucketScatter(P.scell, P.nP, P.cellStart, P.rank, P.sortTmp, g);
+  bucketScatter(P.scell, P.nP, P.cellStart, P.rank, P.sortTmp, phaseSpan(2));
   if (grid.sync()) return;
-  bucketSortSmall(P.cellStart, ncell, P.sortTmp, P.sorted, nullptr, P.sortBig, P.devInt + 2, g, P.nP);
+  bucketSortSmall(P.cellStart, ncell, P.sortTmp, P.sorted, nullptr, P.sortBig, P.devInt + 2, phaseSpan(3), P.nP);
   if (grid.sync()) return;
   if (*bigCells) {
-    bucketSortBig(P.cellStart, P.sortTmp, P.sorted, nullptr, P.sortBig, P.devInt + 2, wave, nWaves, ncell, P.nP);
+    bucketSortBig(P.cellStart, P.sortTmp, P.sorted, nullptr, P.sortBig, P.devInt + 2, phaseSpan(4), ncell, P.nP);
     if (grid.sync()) return;
   }
   // particle data in sorted order; candidate pairs per master, prefix, pair list
-  for (int k = g.tid; k < P.nP; k += g.nth) gatherParticle(P, k);
-  backupPairs(P, g);
-  if (g.tid == 0) P.devInt[2] = 0;  // large-bucket list of the reaction sort
+  {
+    const Span g = phaseSpan(5);
+    for (int k = g.tid; k < P.nP; k += g.nth) gatherParticle(P, k);
+    backupPairs(P, g);
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) P.devInt[2] = 0;  // large-bucket list of the reaction sort
   if (grid.sync()) return;
   pairsFind(P, queues, many);
   if (grid.sync()) return;
@@ -3182,20 +3218,20 @@ __global__ __launch_bounds__(kBroadThreads) void k_broad_phase(Params P) {
   if (pairOverflow(P)) return;
   pairsEmit(P, queues, many);
   if (grid.sync()) return;
-  inheritCerts(P, g);  // reads the motion records before they restart
+  inheritCerts(P, phaseSpan(6));  // reads the motion records before they restart
   // reaction CSR: pairs by partner (counted as they were written), in pair order
   scanReduceTiles(P.rcCount, P.nP, P.scanTiles, lds);
   if (grid.sync()) return;
-  markBuild(P, g);
+  markBuild(P, phaseSpan(7));
   scanApplyTiles(P.rcCount, P.nP, P.scanTiles, P.rcStart, lds, bigRc);
   if (grid.sync()) return;
-  rcScatterPairs(P, g);
+  rcScatterPairs(P, phaseSpan(8));
   if (grid.sync()) return;
   const int nRc = min(P.rcStart[P.nP], int(P.pairCap));
-  bucketSortSmall(P.rcStart, P.nP, P.rcTmp, P.rcPair, P.rcSlot, P.sortBig, P.devInt + 2, g, nRc);
+  bucketSortSmall(P.rcStart, P.nP, P.rcTmp, P.rcPair, P.rcSlot, P.sortBig, P.devInt + 2, phaseSpan(9), nRc);
   if (!*bigRc) return;
   if (grid.sync()) return;
-  bucketSortBig(P.rcStart, P.rcTmp, P.rcPair, P.rcSlot, P.sortBig, P.devInt + 2, wave, nWaves, P.nP, nRc);
+  bucketSortBig(P.rcStart, P.rcTmp, P.rcPair, P.rcSlot, P.sortBig, P.devInt + 2, phaseSpan(10), P.nP, nRc);
 }
 
 template __global__ void k_candidates<false, false>(Params P);

@@ -1451,6 +1451,16 @@ int readFlags(lsdem_ctx* c, int& flags, int& step) {
   return LSDEM_OK;
 }
 
+// Leaves the context able to step again, from whatever state a halted call left.
+int clearFlags(lsdem_ctx* c) {
+  HIPCHK(hipMemset(c->dDevInt.p + 3, 0, sizeof(int)));
+  HIPCHK(hipMemset(c->dDevInt.p + kHaltedIdx, 0, sizeof(int)));
+  HIPCHK(hipMemset(c->dDevInt.p + kErrStepIdx, 0xFF, sizeof(int)));
+  HIPCHK(hipMemset(c->dBarrier.p, 0, kBarrierInts * sizeof(int)));
+  c->forceRebuild = true;
+  return LSDEM_OK;
+}
+
 int reportFlags(lsdem_ctx* c, int flags, int step) {
   int di[8];
   HIPCHK(hipMemcpy(di, c->dDevInt.p, sizeof di, hipMemcpyDeviceToHost));
@@ -1509,11 +1519,7 @@ int runCall(lsdem_ctx* c, Work&& work) {
     if (!flags) return LSDEM_OK;
     if (!recover || attempt >= kMaxRecoveries) {
       const int err = reportFlags(c, flags, step);
-      // leave the context able to step again (from whatever state the halted call left)
-      HIPCHK(hipMemset(c->dDevInt.p + 3, 0, sizeof(int)));
-      HIPCHK(hipMemset(c->dDevInt.p + kErrStepIdx, 0xFF, sizeof(int)));
-      HIPCHK(hipMemset(c->dBarrier.p, 0, kBarrierInts * sizeof(int)));
-      c->forceRebuild = true;
+      if ((rc = clearFlags(c))) return rc;
       return err;
     }
     const long long hCap = c->snap.hCap;
@@ -1595,10 +1601,7 @@ int lsdem_step_graph(lsdem_ctx* c, int32_t n) {
   if (!flags) return LSDEM_OK;
   if (!recover) {
     const int err = reportFlags(c, flags, step);
-    HIPCHK(hipMemset(c->dDevInt.p + 3, 0, sizeof(int)));
-    HIPCHK(hipMemset(c->dDevInt.p + kErrStepIdx, 0xFF, sizeof(int)));
-    HIPCHK(hipMemset(c->dBarrier.p, 0, kBarrierInts * sizeof(int)));
-    c->forceRebuild = true;
+    if ((rc = clearFlags(c))) return rc;
     return err;
   }
   if ((rc = growFor(c, flags))) return rc;
@@ -1634,10 +1637,7 @@ int phaseDone(lsdem_ctx* c, int next) {
   }
   if (flags) {
     const int err = reportFlags(c, flags, step);
-    HIPCHK(hipMemset(c->dDevInt.p + 3, 0, sizeof(int)));
-    HIPCHK(hipMemset(c->dDevInt.p + kErrStepIdx, 0xFF, sizeof(int)));
-    HIPCHK(hipMemset(c->dBarrier.p, 0, kBarrierInts * sizeof(int)));
-    c->forceRebuild = true;
+    if ((rc = clearFlags(c))) return rc;
     c->phaseNext = 0;
     return err;
   }

@@ -260,7 +260,8 @@ struct Params {
   //         [9] (unused), [10 + b] contact slots of the
   //         last step that filled history table b, [12] grid-barrier arrivals of the broad phase,
   //         [20] callStep of the step that raised the first error flag (-1: none), [21], [22] a rebuild's
-  //         large buckets (kBigCellsIdx, kBigRcIdx)
+  //         large buckets (kBigCellsIdx, kBigRcIdx), [23] error flags that a launch found up when it
+  //         began (kHaltedIdx)
   int* devInt;
   int* barrier;          // grid barrier of the single-launch broad phase: kBarrierLine-int lines, one per
                          // block group (blockIdx mod 8), then the groups' counter, then the release word;
@@ -349,6 +350,7 @@ __host__ __device__ inline int ghostCountIdx(int buf) { return 18 + buf; }
 constexpr int kDevStats = 16;  // devStat entries
 constexpr int kPairSlabHost = 32;        // candidate pairs of a master kept by the search (kPairSlab in the kernels)
 constexpr int kBroadThreadsHost = 1024;  // block of the single-launch broad phase (kBroadThreads)
+constexpr int kHaltedIdx = 23;           // devInt: error flags that a launch found up, for the launch after it
 constexpr int kBigCellsIdx = 21, kBigRcIdx = 22;  // devInt: a rebuild has cells (reaction lists) of many items
 constexpr uint32_t kInvalidInfo = 0xFFFFFFFFu;  // unused contact slot
 

@@ -110,14 +110,21 @@ __device__ __forceinline__ int ghostKey(const Params& P, d3 p) {
 #define LSD_GATE(g) \
   if ((g) != nullptr && *(g) == 0) return
 
-// Raise error flag `bit` (kErr*): the call halts (every later kernel returns at entry).  The rebuild
-// gates of both step buffers are cleared so that gated broad-phase launches skip as well; the index
-// of the failing step is kept for the host.
-__device__ __forceinline__ void raiseError(const Params& P, int bit) {
+// Raise error flag `bit` (kErr*): the call halts (every later kernel returns at entry); the index of the
+// failing step is kept for the host.
+__device__ __forceinline__ void raiseFlag(const Params& P, int bit) {
   atomicOr(&P.devInt[3], bit);
   atomicMax(&P.devInt[kErrStepIdx], P.callStep);
+}
+// The rebuild gates of both step buffers are cleared with it so that gated broad-phase launches skip as well.
+// (Not by the single-launch broad phase, whose blocks read their gate while others may raise.)
+__device__ __forceinline__ void dropGates(const Params& P) {
   atomicExch(&P.devInt[rebuildFlagIdx(0)], 0);
   atomicExch(&P.devInt[rebuildFlagIdx(1)], 0);
+}
+__device__ __forceinline__ void raiseError(const Params& P, int bit) {
+  raiseFlag(P, bit);
+  dropGates(P);
 }
 // Touches every 64-byte line of the kernel's Params (its first argument) at once.  The block is 1.6 KB and
 // more than the scalar registers hold, so the compiler reads members where it needs them; each first touch
@@ -155,9 +162,23 @@ __device__ __forceinline__ double inItem(double v, int item) {
   asm("" : "+v"(v) : "v"(item));
   return v;
 }
-// An error flag is up: this kernel has nothing to do.
+// An error flag is up: this kernel has nothing to do.  Each wavefront reads the flag for itself, which is
+// enough for a kernel that raises none: the flag then stays as it was when the launch began.
 #define LSD_HALT(P) \
   if ((P).devInt[prefetchArgs(3)] != 0) return
+// The same in a kernel that is followed by one which raises flags while its blocks meet at barriers: that a flag was
+// up when this launch began is kept for that one ...
+#define LSD_HALT_LATCH(P)                                                              \
+  if (const int halted = (P).devInt[prefetchArgs(3)]) {                                \
+    if (blockIdx.x == 0 && threadIdx.x == 0) (P).devInt[kHaltedIdx] = halted;          \
+    return;                                                                            \
+  }
+// ... which reads it in the flag's place.  A flag that another block raises while this one starts must not send
+// some of its wavefronts home and the rest on to the barriers: what the missing ones were to leave in LDS, a
+// reservation's first slot among it, would be garbage.  (One wavefront's read of the flag for its block, behind a
+// barrier, costs 2.5 to 3 us a step: 1,000 bodies in a box 9.94 -> 10.50 ms for 200.)
+#define LSD_HALT_LATCHED(P) \
+  if ((P).devInt[prefetchArgs(kHaltedIdx)] != 0) return
 
 __global__ void k_fill_int(int* a, long long n, int v, const int* gate) {
   LSD_GATE(gate);
@@ -557,7 +578,7 @@ __device__ __forceinline__ void kickDrift(const Params& P, int i, const BodyIn& 
 // One thread per particle, then one per wall.
 template <bool SEC>
 __global__ void k_kick_drift(Params P, int forceRebuild) {
-  LSD_HALT(P);
+  LSD_HALT_LATCH(P)
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   BodyIn in;
   d3 F, T;
@@ -1267,13 +1288,16 @@ __device__ __forceinline__ bool pairOverflow(const Params& P) {
   if ((long long)np <= P.pairCap) return false;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     atomicMax(&P.devInt[4], np);
-    raiseError(P, kErrPairs);
+    raiseFlag(P, kErrPairs);
   }
   return true;
 }
 __global__ __launch_bounds__(kFindThreads) void k_pairs_emit(Params P) {
   LSD_GATE(P.devInt + rebuildFlagIdx(P.curBuf));
-  if (pairOverflow(P)) return;
+  if (pairOverflow(P)) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) dropGates(P);
+    return;
+  }
   __shared__ int queues[kFindThreads / kFindLanes * kFindQueue], many[kFindThreads + 1];
   pairsEmit(P, queues, many);
 }
@@ -1832,7 +1856,7 @@ __device__ void checkPairs(const Params& P, int full, int nPairs, CheckLds& L) {
 template <bool SEC>
 __global__ __launch_bounds__(256) void k_pair_check(Params P, int full) {
   __shared__ CheckLds L;
-  LSD_HALT(P);  // (a failed broad phase leaves no pair list to read)
+  LSD_HALT_LATCH(P)  // (a failed broad phase leaves no pair list to read)
   // the broad phase of this step is over: its grid barrier's words start the next one at zero
   if (blockIdx.x == 0 && threadIdx.x < 10) P.barrier[threadIdx.x * kBarrierLine] = 0;
   const int nPairs = min(P.pairStart[P.nP], (int)P.pairCap);
@@ -2234,7 +2258,7 @@ __global__ __launch_bounds__(kNarrowBlock, 3) void k_candidates(Params P) {
   static_assert(kBatch * 4096 <= 65536, "a batch's slot offsets fit 16 bits (shapes have at most 4096 nodes)");
   const float kInf = __builtin_huge_valf();
   __shared__ int sTotal[kNarrowBlock / 64], sFirst;
-  LSD_HALT(P);
+  LSD_HALT_LATCHED(P);
   unsigned int statCand = 0, statEnt = 0, statQueries = 0, statContacts = 0;
   const EvalRecords rec = evalRecords(P);
   const int nAct = rec.n;
@@ -2497,14 +2521,15 @@ __global__ __launch_bounds__(kNarrowBlock, 3) void k_candidates(Params P) {
     __syncthreads();
     const int first = __builtin_amdgcn_readfirstlane(sFirst + ahead);
     if (total > 0) {
-      if ((long long)first + total > P.contactCap) {
+      // (a negative first: more than 2^31 slots asked for this step)
+      if (first < 0 || (long long)first + total > P.contactCap) {
         // the call halts with a capacity error; slots reserved below the capacity stay empty
         if (lane == 0) {
-          atomicMax(&P.devInt[5], first + total);
+          atomicMax(&P.devInt[5], int(min((long long)first + total, 0x7fffffffll)));
           raiseError(P, kErrContacts);
         }
-        for (int c = first + lane; c < (int)P.contactCap; c += 64) {
-          if (c >= first + total) break;
+        for (int c = first + lane; first >= 0 && c < (int)P.contactCap; c += 64) {
+          if (c - first >= total) break;
           P.cInfo[c] = kInvalidInfo;
           P.hashSlot[c] = -1;
         }
@@ -2856,7 +2881,7 @@ __global__ void k_reduce_kick(Params P, int kick) {
 // and this step's flags and counters are closed by thread 0 before it clears the next step's.
 template <bool SEC>
 __global__ void k_reduce_drift(Params P, StepHead H) {
-  LSD_HALT(P);
+  LSD_HALT_LATCH(P)
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
   BodyIn in;
   bool set = false;
@@ -2888,7 +2913,7 @@ __global__ void k_reduce_drift(Params P, StepHead H) {
 // its code generation).
 template <bool SEC>
 __global__ void k_reduce_drift_small(Params P, StepHead H) {
-  LSD_HALT(P);
+  LSD_HALT_LATCH(P)
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
   BodyIn in;
   bool set = false;
@@ -2967,6 +2992,7 @@ __global__ void k_snap_restore(Params P, SnapDev S) {
     P.devInt[rebuildFlagIdx(0)] = 0; P.devInt[rebuildFlagIdx(1)] = 0;
     P.devInt[ghostCountIdx(0)] = 0; P.devInt[ghostCountIdx(1)] = 0;
     P.devInt[3] = 0;
+    P.devInt[kHaltedIdx] = 0;
     P.devInt[kErrStepIdx] = -1;
   }
   for (int k = g.tid; k < 5 * kStatSlots; k += g.nth) P.statSlots[k * kStatStride] = 0;
@@ -3146,7 +3172,7 @@ struct GridBarrier {
            __hip_atomic_load(release, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < passed; ++it) {
         if (__hip_atomic_load(P.devInt + 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) break;
         if (it >= unsigned(P.barrierSpin)) {
-          raiseError(P, kErrBarrier);
+          raiseFlag(P, kErrBarrier);
           break;
         }
         __builtin_amdgcn_s_sleep(10);  // ~640 cycles between polls of the release word
@@ -3163,7 +3189,7 @@ struct GridBarrier {
 // of a join block, before the lanes of the other side are back, so that only some lanes' values were kept, and the
 // search then ran on garbage indices.
 __global__ __launch_bounds__(kBroadThreads) void k_broad_phase(Params P) {
-  LSD_HALT(P);
+  LSD_HALT_LATCHED(P);
   if (P.devInt[rebuildFlagIdx(P.curBuf)] == 0) return;  // written by the drift kernel before this launch: grid-uniform
   __shared__ int lds[kScanLds];
   __shared__ int queues[kBroadThreads / kFindLanes * kFindQueue], many[kBroadThreads + 1];

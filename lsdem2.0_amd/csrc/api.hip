@@ -1238,7 +1238,6 @@ int lsdem_initialize(lsdem_ctx* c) {
     HIPCHK(put(sv + kSvAng * nB, c->pAng));
     HIPCHK(put(c->dQuats.p, c->pQuat));
     HIPCHK(put(sv + kSvPos * nB + nP, c->wPos));
-    HIPCHK(put(sv + kSvDet * nB + nP, c->wPos));
     HIPCHK(put(sv + kSvVel * nB + nP, c->wVel));
     HIPCHK(put(sv + kSvAng * nB + nP, c->wAng));
     HIPCHK(put(c->dQuats.p + nP, c->wQuat));

@@ -129,7 +129,8 @@ struct Params {
   // periodicity).  Vector s of body i is pos[s * nBodies + i].
   int nBodies;
   d3* pos;      // state position (after any periodic wrap)
-  d3* posDet;   // position used by the particle-particle and wall detection of this step
+  d3* posDet;   // position used by the particle-particle and wall detection of this step (particles only: a
+                // wall is detected where it is)
   q4* quat;
   d3* vel;
   d3* angvel;

@@ -604,7 +604,6 @@ __device__ void wallDrift(const Params& P, int w, int buf) {
     q = qintegrate(q, P.wangvel[w], P.dt);
     P.wquat[w] = q;
   }
-  P.posDet[P.nP + w] = p;
   P.wkey[w] = refKey(P.gridW, p);
   // displacement bound of any point of the wall's grid box since the last build: translation plus
   // 2 R sin(angle / 2) for the rotation
@@ -1434,7 +1433,8 @@ __device__ __forceinline__ PairView loadPair(const Params& P, int p, uint32_t in
     v.xB = imgPos<SEC>(P, int(v.type - PT_GX))[j];
     v.qB = SEC ? imgQuat(P, int(v.type - PT_GX))[j] : P.quat[j];
   } else {
-    v.xB = P.posDet[j];
+    // (a wall's one position, which a caller may set between two phases of a step, is its detection position too)
+    v.xB = P.pos[(long long)(v.type == PT_PW ? kSvPos : kSvDet) * P.nBodies + j];
     v.qB = SEC && v.type == PT_PP ? P.quatDet[j] : P.quat[j];
   }
   const BodyProp& pB = P.prop[j];
@@ -2138,6 +2138,7 @@ __device__ __forceinline__ PairShare readShare(const Params& P, uint32_t info, i
   const int g = int(type) - int(PT_GX);
   const int idx = !B ? A : wall ? P.nP + j : j;
   int vSlot = t, qSlot = 0;
+  if (B && wall && t == kSvDet) vSlot = kSvPos;  // (as loadPair)
   if (B && ghost && t < 2) vSlot = kSvImg + g;
   if (SEC) {
     if (B && ghost && t == kSvVel) vSlot = kSvImgVel + g;

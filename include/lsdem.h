@@ -67,9 +67,9 @@ typedef struct lsdem_config {
                               device instead of one launch with grid barriers; results do not
                               depend on it */
   int32_t broad_phase_blocks; /* grid of the single-launch broad phase, blocks of 1024 threads (0:
-                              one per 512 particles or per 16,384 search cells, at least 8; below
-                              32,768 particles one per 64, up to a quarter of the CUs); capped at
-                              the CU count */
+                              one per 512 particles or per 16,384 search cells, at least 8); capped
+                              at the CU count.  All blocks of all simulations stepped at once on a
+                              GPU, one per CU, must fit on it */
   int32_t narrow_batch;   /* candidate pairs per wavefront batch of the narrow phase: 1, 2, 4 or 8
                              (0: chosen each step from the number of pairs it evaluates) */
   int32_t no_fused_steps; /* 1: launch each step's kick/drift and its closing sums separately

@@ -11,6 +11,7 @@
 
 #include "../../include/lsdem.h"
 #include "device.h"
+#include "launch_rules.h"
 #include "surrogate_train.h"
 
 namespace lsd {
@@ -1322,14 +1323,7 @@ int lsdem_initialize(lsdem_ctx* c) {
     HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, reinterpret_cast<const void*>(k_broad_phase),
                                                         kBroadThreadsHost, 0));
     if (perCU < 1) return fail(LSDEM_ERR_HIP, "the single-launch broad phase does not fit a CU");
-    // blocks of 1024 threads: one per 512 particles or per 16,384 search cells (the cell loops of a sparse
-    // domain, such as an ensemble of drums far apart), at most one per CU; for fewer than 32,768 particles
-    // one per 64, up to a quarter of the GPU, so that four simulations of that size (the hardware queues a
-    // process has) stepped concurrently still have all their blocks resident together (a rebuild of 4,000
-    // bodies takes 304 us with 8 blocks and 152 with 63, one of 20,000 339 with 40 and 276 with 64)
-    const long long byCells = ((long long)P.sg.ncell + 16383) / 16384;
-    const long long forSearch = std::min<long long>(c->numCU / 4, (nP + 63) / 64);
-    c->coopBlocks = int(std::min<long long>(c->numCU, std::max<long long>({8, (nP + 511) / 512, byCells, forSearch})));
+    c->coopBlocks = broadPhaseBlocks(nP, P.sg.ncell, c->numCU);
     if (c->cfg.broad_phase_blocks > 0) c->coopBlocks = std::min(c->numCU, int(c->cfg.broad_phase_blocks));
     c->coopBlocks = std::min(c->coopBlocks, perCU * c->numCU);  // all resident together on an idle GPU
   }

@@ -1315,7 +1315,6 @@ int lsdem_initialize(lsdem_ctx* c) {
   // narrow-phase grid: enough waves for ~16 candidate pairs per particle, at most 8 per SIMD
   c->narrowBlocks = int(std::min<long long>(c->numCU * 8ll, std::max<long long>(1, (16ll * nP + 8 * 4 - 1) / (8 * 4))));
   if (c->cfg.narrow_blocks > 0) c->narrowBlocks = int(c->cfg.narrow_blocks);
-  P.residentWaves = c->numCU * 12;  // three per SIMD
   // single-launch broad phase: a grid whose blocks can all be resident together
   c->coopBlocks = 0;
   if (!c->cfg.broad_phase_launches) {
@@ -1346,6 +1345,13 @@ int lsdem_initialize(lsdem_ctx* c) {
                                        " bytes of LDS per narrow-phase block, more than the device's " +
                                        std::to_string(prop.sharedMemPerBlock));
     }
+    // its wavefronts that are on the GPU together: three blocks of four per CU by its registers, two by its
+    // LDS with a shape of more than 15 clusters of nodes, one with more than 30
+    int perCU = 0;
+    HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+        &perCU, P.periodicSector ? reinterpret_cast<const void*>(k_candidates<false, true>)
+                                 : reinterpret_cast<const void*>(k_candidates<false, false>), 256, lds));
+    P.residentWaves = c->numCU * std::max(perCU, 1) * 4;
   }
   // candidate nodes (slots of the exact test); reserved per batch at their exact count
   long long contactCap = c->cfg.contact_capacity > 0 ? c->cfg.contact_capacity : 64ll * nP + 16384;

@@ -504,13 +504,12 @@ int pairLaunches(lsdem_ctx* c, const int* gate, Phase& phase) {
   Params& P = c->P;
   hipStream_t s = c->stream;
   int rc;
-  const unsigned gsFind = blocksFor(P.nP, 256 / 32);  // 32 lanes per master
-  hipLaunchKernelGGL(k_pairs_find, dim3(gsFind), dim3(256), 0, s, P);
+  hipLaunchKernelGGL(k_pairs_find, dim3(unsigned(pairsFindBlocks(P.nP))), dim3(kFindThreads), 0, s, P);
   hipLaunchKernelGGL(k_backup_pairs, dim3(unsigned(c->numCU * 4)), dim3(256), 0, s, P);
   rc = scan(c, P.pairCount, P.nP, P.pairStart, gate);
   if (rc) return rc;
   hipLaunchKernelGGL(k_fill_int, dim3(blocksFor(P.nP, 256)), dim3(256), 0, s, P.rcCount, (long long)P.nP, 0, gate);
-  hipLaunchKernelGGL(k_pairs_emit, dim3(blocksFor(P.nP, 32)), dim3(256), 0, s, P);
+  hipLaunchKernelGGL(k_pairs_emit, dim3(blocksFor(P.nP, 32)), dim3(kFindThreads), 0, s, P);
   hipLaunchKernelGGL(k_inherit_certs, dim3(unsigned(c->numCU * 4)), dim3(256), 0, s, P);
   hipLaunchKernelGGL(k_mark_build, dim3(blocksFor(std::max(P.nP, P.nW), 256)), dim3(256), 0, s, P);
   phase();

@@ -15,6 +15,7 @@
 //   k_bonds           parallel bonds
 //   k_reduce_kick     per-body segmented sum of contact and bond contributions + second half-kick
 #include "device.h"
+#include "launch_rules.h"
 #include "surrogate.h"
 
 namespace lsd {
@@ -875,7 +876,7 @@ __device__ __forceinline__ int clampCellF(float v, int n) { return int(fminf(fma
 
 // 32 lanes that search one master's neighbourhood together: its lane l of the group, the group's first lane
 // in the wavefront, and kFindQueue ints of LDS of its own.
-constexpr int kFindLanes = 32, kFindQueue = 256;
+constexpr int kFindQueue = 256;
 struct FindGroup {
   int l, first;
   int* q;
@@ -1108,27 +1109,14 @@ __device__ __forceinline__ void imagePairs(const Params& P, PairSink& sink, cons
   }
 }
 
-// The masters of a block's turn: its share of the sorted order, 32 consecutive ones at a time from all over
-// it (consecutive ones meet the same cells; sizes may be sorted in space, so no block gets one end).
-struct MasterShare {
-  int chunk;  // masters of a full turn's part, 32 per block and turn
-  __device__ __forceinline__ explicit MasterShare(int nP) {
-    const int turns = (nP + int(gridDim.x) * 32 - 1) / (int(gridDim.x) * 32);
-    chunk = turns * 32;
-  }
-  __device__ __forceinline__ int at(int i) const {  // sorted position of the block's i-th master (may be >= nP)
-    return ((i >> 5) * int(gridDim.x) + int(blockIdx.x)) * 32 + (i & 31);
-  }
-};
-
-// Lists the masters of a block's share that want(t), a turn of blockDim.x at a time (many: an int per thread, and
-// one), and takes them one per group of 32 lanes: use(t).
-template <class Want, class Use>
-__device__ __forceinline__ void listedMasters(const Params& P, const MasterShare& share, int* many, Want&& want,
-                                              Use&& use) {
-  int* const nMany = many + blockDim.x;
-  const int group = int(threadIdx.x) / kFindLanes, groups = int(blockDim.x) / kFindLanes;
-  for (int i0 = 0; i0 < share.chunk; i0 += int(blockDim.x)) {
+// Lists the masters of the share of a block of THREADS threads that want(t), THREADS at a time (many: an int per
+// thread, and one), and takes them one per group of 32 lanes: use(t).
+template <int THREADS, class Want, class Use>
+__device__ __forceinline__ void listedMasters(const Params& P, const MasterShare<THREADS / kFindLanes>& share, int* many,
+                                              Want&& want, Use&& use) {
+  int* const nMany = many + THREADS;
+  const int group = int(threadIdx.x) / kFindLanes, groups = THREADS / kFindLanes;
+  for (int i0 = 0; i0 < share.chunk; i0 += THREADS) {
     __threadfence_block();
     __syncthreads();
     if (threadIdx.x == 0) *nMany = 0;
@@ -1149,10 +1137,12 @@ __device__ __forceinline__ void listedMasters(const Params& P, const MasterShare
 // of this edge: 348 us of search at 200,000 for 440 then, 139 for 148 at 20,000, slower below; finer
 // cells slower everywhere.)
 // queues: kFindQueue ints of LDS per group of the block; many: an int per thread, and one.
+template <int THREADS>
 __device__ void pairsFind(const Params& P, int* queues, int* many) {
   const FindGroup G = findGroup(queues);
-  const MasterShare share(P.nP);
-  const int group = int(threadIdx.x) / kFindLanes, groups = int(blockDim.x) / kFindLanes;
+  constexpr int groups = THREADS / kFindLanes;
+  const MasterShare<groups> share(P.nP, int(gridDim.x), int(blockIdx.x));
+  const int group = int(threadIdx.x) / kFindLanes;
   for (int i = group; i < share.chunk; i += groups) {
     const int t = share.at(i);
     if (t >= P.nP) continue;
@@ -1161,19 +1151,17 @@ __device__ void pairsFind(const Params& P, int* queues, int* many) {
     if (G.l == 0) P.pairCount[sink.A] = sink.cnt;
   }
   if (!(P.periodicX || P.periodicY || P.periodicSector)) return;
-  listedMasters(P, share, many, [&](int t) { return mayMeetImages(P, t); },
-                [&](int t) {
-                  const int A = P.sorted[t];
-                  PairSink sink{t, A, P.pairSlab + (long long)t * kPairSlab, kPairSlab, P.pairCount[A]};
-                  imagePairs(P, sink, G);
-                  if (G.l == 0) P.pairCount[inLoop(A, 1)] = sink.cnt;
-                });
+  listedMasters<THREADS>(P, share, many, [&](int t) { return mayMeetImages(P, t); }, [&](int t) {
+    const int A = P.sorted[t];
+    PairSink sink{t, A, P.pairSlab + (long long)t * kPairSlab, kPairSlab, P.pairCount[A]};
+    imagePairs(P, sink, G);
+    if (G.l == 0) P.pairCount[inLoop(A, 1)] = sink.cnt;
+  });
 }
-constexpr int kFindThreads = 256;  // block of the separate search launches
 __global__ __launch_bounds__(kFindThreads) void k_pairs_find(Params P) {
   LSD_GATE(P.devInt + rebuildFlagIdx(P.curBuf));
   __shared__ int queues[kFindThreads / kFindLanes * kFindQueue], many[kFindThreads + 1];
-  pairsFind(P, queues, many);
+  pairsFind<kFindThreads>(P, queues, many);
 }
 // Entry k of master A's part of the pair list (from `out` on), its rank among the partner's reactions with it.
 __device__ __forceinline__ void emitPair(const Params& P, int A, long long out, int k, uint32_t info) {
@@ -1188,15 +1176,16 @@ __device__ __forceinline__ void emitPair(const Params& P, int A, long long out, 
 // per master took as many turns as a master has candidates: 24 us of a rebuild for 4,000 bodies in a quarter
 // sector, now 7); masters with more candidates than the slab holds are searched again, into their part of the list.
 // queues, many: as pairsFind.
+template <int THREADS>
 __device__ void pairsEmit(const Params& P, int* queues, int* many) {
   constexpr int kLanes = 8;
   const FindGroup G = findGroup(queues);
-  const MasterShare share(P.nP);
-  const int l = int(threadIdx.x) & (kLanes - 1), perBlock = int(blockDim.x) / kLanes;
-  int* const anyLarge = many + blockDim.x;
+  const MasterShare<THREADS / kFindLanes> share(P.nP, int(gridDim.x), int(blockIdx.x));
+  const int l = int(threadIdx.x) & (kLanes - 1);
+  int* const anyLarge = many + THREADS;
   if (threadIdx.x == 0) *anyLarge = 0;
   __syncthreads();
-  for (int i = int(threadIdx.x) / kLanes; i < share.chunk; i += perBlock) {
+  for (int i = int(threadIdx.x) / kLanes; i < share.chunk; i += THREADS / kLanes) {
     const int t = share.at(i);
     if (t >= P.nP) continue;
     const int A = P.sorted[t];
@@ -1211,19 +1200,19 @@ __device__ void pairsEmit(const Params& P, int* queues, int* many) {
   // (three passes over the block's large masters: with both searches in one loop, registers spill.  rank, free
   // since the sort, keeps how many partners and walls the first found.)
   const auto isLarge = [&](int t) { return P.pairCount[P.sorted[t]] > kPairSlab; };
-  listedMasters(P, share, many, isLarge, [&](int t) {
+  listedMasters<THREADS>(P, share, many, isLarge, [&](int t) {
     const int A = P.sorted[t];
     PairSink sink{t, A, P.pairInfo + P.pairStart[A], P.pairCount[A], 0};
     nearPairs(P, sink, G);
     if (G.l == 0) P.rank[t] = sink.cnt;
   });
   if (P.periodicX || P.periodicY || P.periodicSector)
-    listedMasters(P, share, many, isLarge, [&](int t) {
+    listedMasters<THREADS>(P, share, many, isLarge, [&](int t) {
       const int A = P.sorted[t];
       PairSink sink{t, A, P.pairInfo + P.pairStart[A], P.pairCount[A], P.rank[t]};
       imagePairs(P, sink, G);
     });
-  listedMasters(P, share, many, isLarge, [&](int t) {
+  listedMasters<THREADS>(P, share, many, isLarge, [&](int t) {
     const int A = P.sorted[t], n = P.pairCount[A];
     const long long out = P.pairStart[A];
     for (int k = G.l; k < n; k += kFindLanes) emitPair(P, A, out, k, P.pairInfo[out + k]);
@@ -1298,7 +1287,7 @@ __global__ __launch_bounds__(kFindThreads) void k_pairs_emit(Params P) {
     return;
   }
   __shared__ int queues[kFindThreads / kFindLanes * kFindQueue], many[kFindThreads + 1];
-  pairsEmit(P, queues, many);
+  pairsEmit<kFindThreads>(P, queues, many);
 }
 __global__ void k_mark_build(Params P) {
   LSD_GATE(P.devInt + rebuildFlagIdx(P.curBuf));
@@ -3235,7 +3224,7 @@ __global__ __launch_bounds__(kBroadThreads) void k_broad_phase(Params P) {
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) P.devInt[2] = 0;  // large-bucket list of the reaction sort
   if (grid.sync()) return;
-  pairsFind(P, queues, many);
+  pairsFind<kBroadThreads>(P, queues, many);
   if (grid.sync()) return;
   scanReduceTiles(P.pairCount, P.nP, P.scanTiles, lds);
   if (grid.sync()) return;
@@ -3243,7 +3232,7 @@ __global__ __launch_bounds__(kBroadThreads) void k_broad_phase(Params P) {
   if (grid.sync()) return;
   // every block reads the same total after the barrier: all leave together when it does not fit
   if (pairOverflow(P)) return;
-  pairsEmit(P, queues, many);
+  pairsEmit<kBroadThreads>(P, queues, many);
   if (grid.sync()) return;
   inheritCerts(P, phaseSpan(6));  // reads the motion records before they restart
   // reaction CSR: pairs by partner (counted as they were written), in pair order

@@ -28,3 +28,45 @@ def test_sparse_domains_and_small_gpus(tmp_path):
 
 def test_the_library_uses_the_rule():
     assert "c->coopBlocks = broadPhaseBlocks(nP, P.sg.ncell, c->numCU);" in (CSRC / "api.hip").read_text()
+
+
+def test_masters_are_shared_once_and_evenly(tmp_path):
+    src = tmp_path / "share.cpp"
+    src.write_text(r'''
+#include "launch_rules.h"
+#include <cstdio>
+#include <vector>
+template <int GROUPS>
+void run(int n, int blocks) {
+  std::vector<int> seen(n, 0);
+  int busy = 0, most = 0;
+  for (int b = 0; b < blocks; ++b) {
+    const lsd::MasterShare<GROUPS> s(n, blocks, b);
+    std::vector<int> of(GROUPS, 0);
+    for (int i = 0; i < s.chunk; ++i)
+      if (s.at(i) < n) {
+        ++seen[s.at(i)];
+        ++of[i % GROUPS];
+      }
+    int top = 0, sum = 0;
+    for (int v : of) { top = v > top ? v : top; sum += v; }
+    busy += sum > 0;
+    most = top > most ? top : most;
+  }
+  bool once = true;
+  for (int v : seen) once = once && v == 1;
+  std::printf("%d %d %d\n", once ? 1 : 0, blocks - busy, most);
+}
+int main() {
+  for (int n : {1, 7, 8, 9, 31, 33, 1000, 4001}) {
+    run<lsd::kFindThreads / lsd::kFindLanes>(n, lsd::pairsFindBlocks(n));  // separate launches
+    run<32>(n, 8);                                                          // the single launch
+  }
+}
+''')
+    exe = tmp_path / "share"
+    subprocess.run(["g++", "-std=c++17", f"-I{CSRC}", str(src), "-o", str(exe)], check=True)
+    rows = [tuple(map(int, r.split())) for r in
+            subprocess.run([str(exe)], capture_output=True, text=True, check=True).stdout.splitlines()]
+    assert all(once == 1 for once, _, _ in rows)
+    assert all(idle == 0 and most == 1 for _, idle, most in rows[::2])  # every block busy, a master per group

@@ -555,8 +555,8 @@ __device__ __forceinline__ void kickDrift(const Params& P, int i, const BodyIn& 
   // rebuild the candidate pairs when a body has moved half the skin since the last build (a
   // periodic wrap always does, and a turn across a sector's face is one wherever it ends).  Sector images
   // are turned about the corner's axis, so they move as far as their sources and the skin covers them as it
-  // covers shifted ones.  (Rebuilt every step, as sector periodicity once did: 4,000 bodies 0.22 ms a step,
-  // 0.059 now.)
+  // covers shifted ones.  (Rebuilt every step, as sector periodicity once did: 4,000 bodies 0.22 ms a step
+  // with the 32-lane search, 0.05 now.)
   const double hs2 = P.halfSkin * P.halfSkin;
   const d3 dd = pDet - in.xBuild, dw = p - in.xBuildW;
   const bool moved = turned || len2(dd) > hs2 || len2(dw) > hs2;
@@ -1132,7 +1132,7 @@ __device__ __forceinline__ void listedMasters(const Params& P, const MasterShare
 // round trips (its own data, the row lookups, four rounds of 32 items at a time) and by how unevenly masters
 // meet neighbours.  Images are searched in a turn of their own for the masters that may have any.  (One
 // thread per master, an item a round trip: 398 us of a rebuild's 522 for 4,000 bodies in a quarter sector, 340
-// of 507 for 20,000 of scattered sizes, 597 of 1,028 for 200,000; now 42 of 152, 126 of 276 and 325 of 700.
+// of 507 for 20,000 of scattered sizes, 597 of 1,028 for 200,000; whole rebuilds on the same grids now: 301, 319, 683.
 // Tried and left out: a largest radius per search cell to shorten the runs, with cells of 1, 0.5 and 0.35
 // of this edge: 348 us of search at 200,000 for 440 then, 139 for 148 at 20,000, slower below; finer
 // cells slower everywhere.)
@@ -1358,7 +1358,7 @@ __device__ __forceinline__ d3 histLookup(const Params& P, unsigned long long key
 }
 
 // ------------------------------------------------------------------------------------------
-// Narrow phase: node-vs-SDF detection, one wavefront per batch of 8 candidate pairs
+// Narrow phase: node-vs-SDF detection, one wavefront per batch of evaluated pairs
 // ------------------------------------------------------------------------------------------
 constexpr int kNarrowBlock = 256;
 
@@ -2213,10 +2213,10 @@ __device__ __forceinline__ float groupMin(float v) {
 
 // Candidate nodes: one wavefront per batch of up to 8 evaluated pairs, three levels of conservative
 // FP32 culls, then the exact test of what is left.  Bound by each wavefront's chain of round trips (about 9
-// with the exact test) and by how many wavefronts share a SIMD: 146 registers, 3 wavefronts (256 and 2 when
-// every lane of the exact test loaded its pair's state itself; 101 -> 77 us for 200,000 falling bodies that
-// evaluate some 15,000 pairs a step, 184 -> 160 us for an ordered bed that evaluates 80,000, a falling
-// column of 20,000 at its 20 us either way).  A limit of 128 registers spills 24 and LDS has no room for a
+// with the exact test) and by how many wavefronts share a SIMD: 150 registers, 3 wavefronts (256 and 2 when
+// every lane of the exact test loaded its pair's state itself; 101 us then and 74 now for 200,000 falling bodies that
+// evaluate some 15,000 pairs a step, 184 and 146 us for an ordered bed that evaluates 80,000, the block-wide
+// reservations below included, 20 and 19 us for a falling column of 20,000).  A limit of 128 registers spills 24 and LDS has no room for a
 // fourth wavefront.
 //   1. lanes = (pair, cluster of <= 64 nodes): bounding spheres, grid box, SDF Lipschitz bound at
 //      the cluster centre (or the surrogate's decision); survivors become entries;
@@ -3024,7 +3024,7 @@ __global__ void k_kick(Params P) {
 // ------------------------------------------------------------------------------------------
 // Step bookkeeping
 // ------------------------------------------------------------------------------------------
-// stepEnd by the first wavefront of block 0 (lanes l < min(64, blockDim.x)): the lanes read the stat
+// stepEnd by one wavefront, the first of the launch's last block (lanes l < min(64, blockDim.x)): the lanes read the stat
 // slots (a line each) together and sum them across lanes (in FP64, exact for counts below 2^53), where
 // thread 0 alone takes 8 dependent rounds of scalar loads.  Totals, flags and counters as stepEnd.
 __device__ void stepEndWave(const Params& P, int l) {
@@ -3109,9 +3109,9 @@ __device__ void stepEnd(const Params& P) {
 // reach every barrier.  The host sizes the grid so that all its blocks are resident together.
 // A rebuild is a chain of short phases: a barrier costs 2.3 to 2.9 us, a phase at least its own few dependent
 // reads, so phases share barriers where neither reads what the other writes (14 barriers, once 19), and the sorts
-// of long buckets are passed over when there are none.  Whole rebuild, before -> now: 27 bodies 105 -> 84 us,
-// 1,000 163 -> 103, 4,000 in a quarter sector 522 -> 152, 20,000 of scattered sizes 507 -> 276, 27,000 packed
-// 223 -> 200, 200,000 of scattered sizes 1,028 -> 700.
+// of long buckets are passed over when there are none.  Whole rebuild (the longest launch of a pass), before -> now: 27
+// bodies 113 -> 80 us, 1,000 162 -> 109, 4,000 in a quarter sector 520 -> 301, 20,000 of scattered sizes 508 -> 319,
+// 27,000 packed 225 -> 206, 200,000 of scattered sizes 1,074 -> 683.
 // ------------------------------------------------------------------------------------------
 // Blocks of the single-launch broad phase: large, so that few blocks meet at each barrier (the
 // cost of a barrier grows with the number of blocks) while many threads work between them.

@@ -1138,7 +1138,7 @@ __device__ __forceinline__ void listedMasters(const Params& P, const MasterShare
 // cells slower everywhere.)
 // queues: kFindQueue ints of LDS per group of the block; many: an int per thread, and one.
 template <int THREADS>
-__device__ void pairsFind(const Params& P, int* queues, int* many) {
+__device__ __forceinline__ void pairsFind(const Params& P, int* queues, int* many) {
   const FindGroup G = findGroup(queues);
   constexpr int groups = THREADS / kFindLanes;
   const MasterShare<groups> share(P.nP, int(gridDim.x), int(blockIdx.x));
@@ -1177,7 +1177,7 @@ __device__ __forceinline__ void emitPair(const Params& P, int A, long long out, 
 // sector, now 7); masters with more candidates than the slab holds are searched again, into their part of the list.
 // queues, many: as pairsFind.
 template <int THREADS>
-__device__ void pairsEmit(const Params& P, int* queues, int* many) {
+__device__ __forceinline__ void pairsEmit(const Params& P, int* queues, int* many) {
   constexpr int kLanes = 8;
   const FindGroup G = findGroup(queues);
   const MasterShare<THREADS / kFindLanes> share(P.nP, int(gridDim.x), int(blockIdx.x));
